@@ -10,11 +10,10 @@
 //
 // Two kernels share that layout.  copy_aligned_kernel serves plans whose records all
 // start on aligned addresses (the host certifies this): one aligned load and one aligned
-// store per unit.  copy_kernel serves any plan: the destination is written with aligned
-// stores after an element-wise head, and the source is read with aligned loads of the
-// unit's width and shifted into place with v_alignbyte, so intervals at any element
-// offset stream at full width.  A load never touches an aligned block that holds no byte
-// of the source interval.
+// store per unit.  copy_kernel serves any plan: it cuts each record's chunks on 128-byte
+// lines of the destination, so that only a record's first and last chunk write part of a
+// line, and reads its units where they lie with unaligned vector loads.  A load never
+// touches a byte outside the source interval.
 #include "hbt_common.hpp"
 
 namespace hbt {
@@ -24,6 +23,8 @@ namespace {
 // 1 KB and retires, the shape that streamed fastest against 512 B or 2 KB per
 // workgroup and against 256-thread workgroups walking larger chunks.
 constexpr int kCopyBlock = 64;
+// A cache line: what a store must cover whole for the memory behind the L2 to see one write.
+constexpr uint32_t kLineBytes = 128;
 // Non-temporal loads and stores: every byte is moved once.
 constexpr bool kCopyNT = true;
 
@@ -59,50 +60,14 @@ __device__ __forceinline__ void stg(gbyte* p, typename Vec<NW>::type x) {
     }
 }
 
-// A unit's source bytes as loaded: one aligned block, plus the next one when the
-// source is misaligned by k = s mod 4*NW bytes (k is uniform across the wave).  The
-// second block holds source bytes s + 4*NW - 1 and earlier ones only up to the block
-// boundary, so it lies inside the source's page.
+// NW dwords from an address on an element boundary (2 or 4 bytes): one vector load, which
+// the memory pipeline splits where it crosses a line.
 template <int NW>
-struct Raw {
-    typename Vec<NW>::type x, y;
-};
-template <int NW>
-__device__ __forceinline__ void load_raw(const gbyte* s, uint32_t k, Raw<NW>& r) {
-    static_assert(NW == 2 || NW == 4, "units are 8 or 16 bytes");
-    const gbyte* a = s - k;
-    r.x = ldg<NW>(a);
-    if (k != 0) r.y = ldg<NW>(a + 4 * NW);
-}
-// Shifts a loaded unit into place with v_alignbyte.
-template <int NW>
-__device__ __forceinline__ void align_raw(const Raw<NW>& raw, uint32_t k, uint32_t (&out)[NW]) {
-    if (k == 0) {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) out[i] = raw.x[i];
-        return;
-    }
-    uint32_t w[2 * NW];
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        w[i] = raw.x[i];
-        w[NW + i] = raw.y[i];
-    }
-    const uint32_t r = k & 3u;
-    const uint32_t q = k >> 2;  // whole dwords to skip, < NW
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        // Select w[i + q] and w[i + q + 1] with q uniform; unrolled over q's range.
-        uint32_t lo = w[i], hi = w[i + 1];
-#pragma unroll
-        for (int j = 1; j < NW; ++j) {
-            if (q == static_cast<uint32_t>(j)) {
-                lo = w[i + j];
-                hi = w[i + j + 1];
-            }
-        }
-        out[i] = __builtin_amdgcn_alignbyte(hi, lo, r);
-    }
+__device__ __forceinline__ typename Vec<NW>::type ldg_any(const gbyte* p) {
+    typedef typename Vec<NW>::type V __attribute__((aligned(2)));
+    typedef __attribute__((address_space(1))) const V GV;
+    if constexpr (kCopyNT) return __builtin_nontemporal_load(reinterpret_cast<GV*>(p));
+    return *reinterpret_cast<GV*>(p);
 }
 
 // Element semantics.  SB/DB are source/destination element bytes; a 2-byte element is
@@ -195,6 +160,35 @@ __device__ __forceinline__ void pack_unit_store(gbyte* d, const uint32_t (&e)[U]
     stg<NW>(d, x);
 }
 
+// Converts one unit as loaded and stores it.
+template <int SB, int DB, int OP, bool H>
+__device__ __forceinline__ void store_unit(gbyte* d, const typename Vec<unit_elems<SB, DB>() * SB / 4>::type& x,
+                                           float divisor) {
+    constexpr int U = unit_elems<SB, DB>();
+    constexpr int kSrcWords = U * SB / 4;
+    uint32_t words[kSrcWords];
+#pragma unroll
+    for (int i = 0; i < kSrcWords; ++i) words[i] = x[i];
+    uint32_t e[U];
+    unpack_unit<SB, U>(words, e);
+    if constexpr (rounds_to_b16<SB, DB, OP>()) {
+        // Two values per packed conversion, each the bits f32_to_b16 gives.
+        float f[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) f[i] = convert_value<SB, OP, H>(e[i], divisor);
+        uint32_t w[U / 2];
+        pack_rounded<H ? HBT_DTYPE_F16 : HBT_DTYPE_BF16, U / 2>(f, w);
+        typename Vec<U / 2>::type o;
+#pragma unroll
+        for (int i = 0; i < U / 2; ++i) o[i] = w[i];
+        stg<U / 2>(d, o);
+    } else {
+#pragma unroll
+        for (int i = 0; i < U; ++i) e[i] = convert<SB, DB, OP, H>(e[i], divisor);
+        pack_unit_store<DB, U>(d, e);
+    }
+}
+
 // Index of the record that owns `chunk`: the last record whose first_chunk <= chunk
 // (the host drops records with no chunks, so first_chunk strictly increases).  The
 // search runs on the scalar unit: its loads hit the scalar cache and do not queue behind
@@ -225,6 +219,16 @@ __device__ __forceinline__ int64_t owning_record(const int64_t* __restrict__ tab
     return lo;
 }
 
+// Any plan.  A record's chunk c covers elements [line + c * kChunk, line + (c + 1) * kChunk)
+// of it, `line` being the elements before its destination's first 128-byte line (chunk 0
+// takes those too), cut at the record's end: the same number of chunks as the table counts,
+// the last of them possibly empty.  Every chunk but a record's first and last then writes
+// whole lines, where chunks counted from the record's start write two partial lines each,
+// shared between two XCDs' L2 caches.  Units are read by one unaligned vector load each, where two
+// aligned loads and a shift read every line twice.  1 GiB moved between misaligned
+// addresses, GB/s (read + written), chunks from the record's start with two loads, then
+// this: source 2 bytes off 5,160 and 6,240; destination 2 off 4,600 and 6,210; both
+// 4,590 and 6,250; destination 16 off 5,850 and 6,230.
 template <int SB, int DB, int OP, bool H>
 __global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restrict__ table,
                                                           int64_t count, float divisor, int64_t chunk_base,
@@ -235,23 +239,28 @@ __global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restr
     const gbyte* src = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec[0]));
     gbyte* dst = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec[1]));
     const int64_t n = rec[2];
+    const int64_t c = chunk - rec[3];
     constexpr int64_t kChunk = chunk_elems<SB, DB>();
-    const int64_t e0 = (chunk - rec[3]) * kChunk;
-    const int64_t len = (n - e0) < kChunk ? (n - e0) : kChunk;
-
-    gbyte* d = dst + e0 * DB;
-    const gbyte* s = src != nullptr ? src + e0 * SB : nullptr;
     constexpr int U = unit_elems<SB, DB>();
     constexpr int kSrcWords = U * SB / 4;
     constexpr int kPerLane = static_cast<int>(kChunk / U / kCopyBlock);
     static_assert(kChunk == int64_t(kPerLane) * kCopyBlock * U, "a chunk is whole units on every lane");
+    static_assert(kLineBytes / DB <= kCopyBlock, "one lane per element of a head");
 
-    // Head: elements until the destination is 16-byte aligned.
-    int64_t head = static_cast<int64_t>(((16u - (static_cast<uint32_t>(reinterpret_cast<uintptr_t>(d)) & 15u)) & 15u) / DB);
+    const int64_t line = ((kLineBytes - (static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst)) & (kLineBytes - 1u))) &
+                          (kLineBytes - 1u)) / DB;
+    const int64_t e0 = c == 0 ? 0 : line + c * kChunk;
+    const int64_t past = line + (c + 1) * kChunk;
+    const int64_t len = (past < n ? past : n) - e0;
+    if (len <= 0) return;
+    gbyte* d = dst + e0 * DB;
+    const gbyte* s = src != nullptr ? src + e0 * SB : nullptr;
+
+    // Elements before the first line (chunk 0) and after the last whole unit, one per lane.
+    int64_t head = c == 0 ? line : 0;
     if (head > len) head = len;
     const int64_t units = (len - head) / U;
     const int64_t tail_begin = head + units * U;
-
     if (threadIdx.x < head) {
         const int64_t e = threadIdx.x;
         const uint32_t bits = s != nullptr ? convert<SB, DB, OP, H>(load_elem<SB>(s + e * SB), divisor) : 0u;
@@ -263,7 +272,7 @@ __global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restr
         store_elem<DB>(d + e * DB, bits);
     }
 
-    // Units per lane: kPerLane (2 for bf16 -> fp32, else 1).  Every unit's loads are
+    // Units per lane: kPerLane (4 for bf16 -> fp32, else 1).  Every unit's loads are
     // issued before the first store, so a workgroup pays one memory round trip.
     gbyte* dbody = d + head * DB;
     if (s == nullptr) {
@@ -278,25 +287,16 @@ __global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restr
         return;
     }
     const gbyte* sbody = s + head * SB;
-    const uint32_t k = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(sbody)) & (4u * kSrcWords - 1u);
-    Raw<kSrcWords> raw[kPerLane];
+    typename Vec<kSrcWords>::type x[kPerLane];
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
         const int64_t u = threadIdx.x + j * kCopyBlock;
-        if (u < units) load_raw<kSrcWords>(sbody + u * U * SB, k, raw[j]);
+        if (u < units) x[j] = ldg_any<kSrcWords>(sbody + u * U * SB);
     }
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
         const int64_t u = threadIdx.x + j * kCopyBlock;
-        if (u < units) {
-            uint32_t words[kSrcWords];
-            align_raw<kSrcWords>(raw[j], k, words);
-            uint32_t e[U];
-            unpack_unit<SB, U>(words, e);
-#pragma unroll
-            for (int i = 0; i < U; ++i) e[i] = convert<SB, DB, OP, H>(e[i], divisor);
-            pack_unit_store<DB, U>(dbody + u * U * DB, e);
-        }
+        if (u < units) store_unit<SB, DB, OP, H>(dbody + u * U * DB, x[j], divisor);
     }
 }
 
@@ -344,29 +344,7 @@ __global__ __launch_bounds__(kCopyBlock) void copy_aligned_kernel(const int64_t*
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
         const int64_t u = threadIdx.x + j * kCopyBlock;
-        if (u < units) {
-            uint32_t words[kSrcWords];
-#pragma unroll
-            for (int i = 0; i < kSrcWords; ++i) words[i] = x[j][i];
-            uint32_t e[U];
-            unpack_unit<SB, U>(words, e);
-            if constexpr (rounds_to_b16<SB, DB, OP>()) {
-                // Two values per packed conversion, each the bits f32_to_b16 gives.
-                float f[U];
-#pragma unroll
-                for (int i = 0; i < U; ++i) f[i] = convert_value<SB, OP, H>(e[i], divisor);
-                uint32_t w[U / 2];
-                pack_rounded<H ? HBT_DTYPE_F16 : HBT_DTYPE_BF16, U / 2>(f, w);
-                typename Vec<U / 2>::type o;
-#pragma unroll
-                for (int i = 0; i < U / 2; ++i) o[i] = w[i];
-                stg<U / 2>(d + u * U * DB, o);
-            } else {
-#pragma unroll
-                for (int i = 0; i < U; ++i) e[i] = convert<SB, DB, OP, H>(e[i], divisor);
-                pack_unit_store<DB, U>(d + u * U * DB, e);
-            }
-        }
+        if (u < units) store_unit<SB, DB, OP, H>(d + u * U * DB, x[j], divisor);
     }
     if (threadIdx.x < len - units * U) {
         const int64_t e = units * U + threadIdx.x;

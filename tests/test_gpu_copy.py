@@ -364,3 +364,31 @@ def test_bf16_float16_conversions_are_tensor_to(device):
         assert torch.equal(got.view(torch.int16), expect.view(torch.int16)), (src, dst)
         untouched = torch.cat([b[:3], b[3 + expect.numel() :]]).cpu()
         assert torch.equal(untouched, torch.full((4,), 7.0, dtype=dst))
+
+
+@pytest.mark.parametrize(("sdt", "ddt", "op"), CASES)
+@pytest.mark.parametrize("around", ["line", "chunk"])
+def test_records_cut_on_destination_lines(device, sdt, ddt, op, around):
+    """Records that start at every element offset from a destination line, of the lengths
+    where the cut on lines can go wrong: around the first line, and around whole chunks
+    with and without the elements before it.  Guard elements between them stay untouched."""
+    size = {torch.float64: 8, torch.float32: 4}.get(ddt, 2)
+    line = 128 // size
+    chunk = _native._copy_chunk(_native.library(), _native.dtype_code(sdt), _native.dtype_code(ddt))
+    rows, cursor = [], 0
+    for off in range(line):
+        head = (line - off) % line
+        ends = (1, head, head + 1, line) if around == "line" else (chunk - 1, chunk, head + chunk, chunk + head + 1,
+                                                                  2 * chunk + head - 1)
+        for k, n in enumerate(sorted({n for n in ends if n > 0})):
+            rows.append(((7 * off + k) % 97, cursor + off, n))
+            cursor += -(-(off + n + 3) // line) * line
+    src = (torch.randn(97 + 3 * chunk, dtype=torch.float32, device=device) * 3).to(sdt)
+    dst = torch.randn(cursor, dtype=torch.float32, device=device).to(ddt)
+    src_bits, dst_bits = _bits(src), _bits(dst)
+    expected = _expected(src_bits, dst_bits, rows, _converter(sdt, ddt, op, 3.0))
+    plan = _native.CopyPlan(device)
+    for s0, d0, n in rows:
+        plan.add(src, s0, dst, d0, n)
+    plan.run(src_dtype=sdt, dst_dtype=ddt, op=op, divisor=3.0)
+    assert np.array_equal(_bits(dst), expected)
