@@ -524,3 +524,70 @@ def test_grad_accumulate_tiles(device, acc_dtype, grad_dtype, assign):
                                    _native.pointer_array([grads[0].data_ptr()]), _native.int64_array([1]), 1,
                                    0 if acc_dtype == torch.float64 else _native.dtype_code(acc_dtype), 3, 0,
                                    stream) == -1  # fp64 gradients need an fp64 accumulator
+
+
+@pytest.mark.parametrize("group", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("shard", [513, 514, 515, 4 * 256 + 1, 17 * 256 + 3])
+@pytest.mark.parametrize("dtypes", [(torch.bfloat16, torch.float32), (torch.float16, torch.float32),
+                                    (torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                    (torch.float16, torch.float16)],
+                         ids=lambda d: "-".join(str(x).split(".")[1] for x in d))
+def test_local_share_groups_off_the_vectors(device, group, shard, dtypes):
+    """Every group size with an instantiation of its own and one past them, at shard lengths
+    that start ranks 1 to 3 one, two and three elements off a four-element vector: bitwise
+    the oracle's share, on one-launch and two-launch shards, with a short padding tail."""
+    in_dtype, master = dtypes
+    lib = _native.library()
+    valid = shard - 2
+    gen = torch.Generator(device=device).manual_seed(group * 1000 + shard)
+    grads = [(torch.randn(group * shard, device=device, generator=gen) * 0.3).to(in_dtype) for _ in range(group)]
+    host = [g.float().cpu().numpy() for g in grads]
+    for rank in range(1, min(group, 4)):
+        out = torch.full((shard,), 7.0, dtype=master, device=device)
+        partials = torch.empty(2, dtype=torch.float64, device=device)
+        tile_sums = torch.empty(-(-shard // 256), dtype=torch.float64, device=device)
+        _native.check(lib.hbt_grad_local_share_sqnorm(
+            _native.pointer_array([g.data_ptr() for g in grads]), group, rank, shard, valid,
+            _native.dtype_code(in_dtype), _native.dtype_code(master), float(group), _native.dtype_code(master),
+            out.data_ptr(), partials.data_ptr(), tile_sums.data_ptr(), _native.stream_of(device)), "test.share")
+        expect = oracle.local_share(host, rank, shard, valid, float(group), reduce=_REDUCE[master])
+        assert np.array_equal(out.float().cpu().numpy().view(np.int32), expect.view(np.int32)), rank
+        ref = math.fsum(float(x) * float(x) for x in expect)
+        got = partials.cpu().numpy()
+        assert abs(got[0] - ref) <= 1e-12 * ref and got[1] == 0.0, rank
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 511, 1025, 32769])
+@pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                    (torch.bfloat16, torch.bfloat16), (torch.float64, torch.float64)],
+                         ids=lambda d: "-".join(str(x).split(".")[1] for x in d))
+@pytest.mark.parametrize("write_back", [False, True])
+def test_steps_off_the_vectors_are_the_aligned_steps(device, n, dtypes, write_back):
+    """AdamW and momentum SGD on operands that each start one to three elements into their
+    allocation give bitwise what the same values at aligned addresses give, and leave the
+    elements around them alone."""
+    from hybrid_training_amd.optim import _adamw_call, _sgd_call
+
+    pdtype, gdtype = dtypes
+    lib = _native.library()
+    gen = torch.Generator(device=device).manual_seed(n)
+    flags = _native.STEP_WRITE_GRAD if write_back else 0
+    wide = pdtype == torch.float64
+    mul = torch.tensor([0.3125], dtype=torch.float64 if wide else torch.float32, device=device)
+    values = [(torch.randn(n, device=device, generator=gen).abs() * s).to(d)
+              for s, d in ((0.02, pdtype), (1e-2, gdtype), (1e-3, pdtype), (1e-4, pdtype))]
+    results = []
+    for leads in ((0, 0, 0, 0), (1, 2, 3, 1)):
+        stores = [torch.full((n + 8,), 3.0, dtype=v.dtype, device=device) for v in values]
+        views = [s[lead : lead + n].copy_(v) for s, lead, v in zip(stores, leads, values)]
+        p, g, m, v = ([t.data_ptr()] for t in views)
+        stream = _native.stream_of(device)
+        _native.check(_adamw_call(lib, pdtype, gdtype, p, g, m, v, [n], 1.0, mul.data_ptr(),
+                                  (1.0 - 3e-5, 0.1, 0.95, 0.05, 0.5, 1e-8, -1e-3), flags, stream), "test.adamw")
+        _native.check(_sgd_call(lib, pdtype, gdtype, p, g, m, [n], 1.0, mul.data_ptr(), (0.1, 0.9, 1.0, -1e-3),
+                                flags | _native.SGD_MOMENTUM | _native.SGD_WEIGHT_DECAY, stream), "test.sgd")
+        for s, lead in zip(stores, leads):
+            assert bool((s[:lead] == 3.0).all()) and bool((s[lead + n :] == 3.0).all())
+        results.append([_bits(t) for t in views])
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
