@@ -1097,28 +1097,37 @@ __global__ __launch_bounds__(kShareBlock) void tile_sums_to_partials_kernel(
 
 constexpr int kFinalBlock = 1024;
 
-__global__ __launch_bounds__(kFinalBlock) void norm_finalize_kernel(
-    const double* __restrict__ partials, int64_t count, double max_norm, double* __restrict__ sum_out,
-    double* __restrict__ norm_out, float* __restrict__ grad_mul_out, double* __restrict__ grad_mul64_out,
-    int32_t* __restrict__ nonfinite_out) {
-    // Four independent accumulators per thread keep four loads in flight; they are
-    // combined in a fixed order, so the sum stays reproducible.
+// Where a finalize writes what it derives from the weighted squared sum (each may be null).
+struct NormOutputs {
+    double* sum;
+    double* norm;
+    float* grad_mul;
+    double* grad_mul64;
+    int32_t* nonfinite;
+};
+
+// The sum of `count` values in a fixed order by one kFinalBlock-lane workgroup; the total is
+// valid in thread 0.  Four independent accumulators per thread keep four loads in flight.
+template <typename Value>
+__device__ __forceinline__ double finalize_sum(int64_t count, Value&& value) {
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
     int64_t i = threadIdx.x;
     for (; i + 3 * kFinalBlock < count; i += 4 * kFinalBlock) {
-        a0 += partials[i];
-        a1 += partials[i + kFinalBlock];
-        a2 += partials[i + 2 * kFinalBlock];
-        a3 += partials[i + 3 * kFinalBlock];
+        a0 += value(i);
+        a1 += value(i + kFinalBlock);
+        a2 += value(i + 2 * kFinalBlock);
+        a3 += value(i + 3 * kFinalBlock);
     }
-    for (; i < count; i += kFinalBlock) a0 += partials[i];
-    const double total = block_sum<kFinalBlock>((a0 + a1) + (a2 + a3));
-    if (threadIdx.x != 0) return;
+    for (; i < count; i += kFinalBlock) a0 += value(i);
+    return block_sum<kFinalBlock>((a0 + a1) + (a2 + a3));
+}
+
+__device__ __forceinline__ void write_norm_outputs(double total, double max_norm, const NormOutputs& out) {
     // clamp_min(0) keeps NaN; sqrt of fp64 is correctly rounded.
     const double clamped = total < 0.0 ? 0.0 : total;
     const double norm = sqrt(clamped);
-    if (sum_out != nullptr) sum_out[0] = total;
-    if (norm_out != nullptr) norm_out[0] = norm;
+    if (out.sum != nullptr) out.sum[0] = total;
+    if (out.norm != nullptr) out.norm[0] = norm;
     // The reference multiplies by the Python-double coefficient only when it is below 1:
     // fp32, bf16 and fp16 gradients take it as torch passes it to their kernels, rounded
     // to fp32; float64 gradients take the double itself.
@@ -1127,9 +1136,54 @@ __global__ __launch_bounds__(kFinalBlock) void norm_finalize_kernel(
         const double coef = max_norm / (norm + 1e-6);
         if (coef < 1.0) mul = coef;
     }
-    if (grad_mul_out != nullptr) grad_mul_out[0] = static_cast<float>(mul);
-    if (grad_mul64_out != nullptr) grad_mul64_out[0] = mul;
-    if (nonfinite_out != nullptr) nonfinite_out[0] = isfinite(total) ? 0 : 1;
+    if (out.grad_mul != nullptr) out.grad_mul[0] = static_cast<float>(mul);
+    if (out.grad_mul64 != nullptr) out.grad_mul64[0] = mul;
+    if (out.nonfinite != nullptr) out.nonfinite[0] = isfinite(total) ? 0 : 1;
+}
+
+__global__ __launch_bounds__(kFinalBlock) void norm_finalize_kernel(const double* __restrict__ partials, int64_t count,
+                                                                    double max_norm, NormOutputs out) {
+    const double total = finalize_sum(count, [&](int64_t i) { return partials[i]; });
+    if (threadIdx.x == 0) write_norm_outputs(total, max_norm, out);
+}
+
+// The finalize over partials that lie in several arrays, read where their producers left
+// them and multiplied by their array's weight: bitwise norm_finalize_kernel over one array
+// that holds the weighted partials one after another.  A list of FSDP units reduces into as
+// many arrays of partials as it has units; gathering them first took a copy launch per
+// unit, each with a table of its own to upload (13 units of GPT-2 small: 26 of a step's 55
+// launches, and 350 us of its 800).  The table rides in the launch's arguments and is
+// searched in LDS.
+struct PartTable {
+    const double* p[HBT_MAX_NORM_PARTS];
+    double w[HBT_MAX_NORM_PARTS];
+    int64_t first[HBT_MAX_NORM_PARTS + 1];
+    int32_t parts;
+};
+__global__ __launch_bounds__(kFinalBlock) void norm_finalize_parts_kernel(PartTable tab, double max_norm,
+                                                                          NormOutputs out) {
+    static_assert(HBT_MAX_NORM_PARTS < kFinalBlock, "one lane per part fills the LDS table");
+    __shared__ const double* p[HBT_MAX_NORM_PARTS];
+    __shared__ double w[HBT_MAX_NORM_PARTS];
+    __shared__ int64_t first[HBT_MAX_NORM_PARTS + 1];
+    const int t = static_cast<int>(threadIdx.x);
+    if (t < tab.parts) {
+        p[t] = tab.p[t];
+        w[t] = tab.w[t];
+    }
+    if (t <= tab.parts) first[t] = tab.first[t];
+    __syncthreads();
+    const int parts = tab.parts;
+    const double total = finalize_sum(first[parts], [&](int64_t i) {
+        int lo = 0, hi = parts - 1;  // the last part that starts at or before i
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (first[mid] <= i) lo = mid;
+            else hi = mid - 1;
+        }
+        return p[lo][i - first[lo]] * w[lo];
+    });
+    if (t == 0) write_norm_outputs(total, max_norm, out);
 }
 
 // ---- in-place scaling ---------------------------------------------------------------
@@ -2190,9 +2244,36 @@ int32_t hbt_grad_norm_finalize(const double* partials, int64_t count, double max
         set_error("hbt_grad_norm_finalize: bad partials/count");
         return HBT_ERR_INVALID_ARGUMENT;
     }
-    norm_finalize_kernel<<<1, kFinalBlock, 0, as_stream(stream)>>>(partials, count, max_norm, sum_out, norm_out,
-                                                                   grad_mul_out, grad_mul64_out, nonfinite_out);
+    norm_finalize_kernel<<<1, kFinalBlock, 0, as_stream(stream)>>>(
+        partials, count, max_norm, NormOutputs{sum_out, norm_out, grad_mul_out, grad_mul64_out, nonfinite_out});
     return check_launch("hbt_grad_norm_finalize");
+}
+
+int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_t* counts, const double* weights,
+                                     int32_t parts, double max_norm, double* sum_out, double* norm_out,
+                                     float* grad_mul_out, double* grad_mul64_out, int32_t* nonfinite_out,
+                                     void* stream) {
+    clear_error();
+    if (parts < 0 || parts > HBT_MAX_NORM_PARTS ||
+        (parts > 0 && (partials == nullptr || counts == nullptr || weights == nullptr))) {
+        set_error("hbt_grad_norm_finalize_parts: bad table (parts=%d of at most %d)", parts, HBT_MAX_NORM_PARTS);
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    PartTable tab{};
+    for (int i = 0; i < parts; ++i) {
+        if (counts[i] < 0 || (counts[i] > 0 && partials[i] == nullptr)) {
+            set_error("hbt_grad_norm_finalize_parts: part %d has a bad pointer or count", i);
+            return HBT_ERR_INVALID_ARGUMENT;
+        }
+        if (counts[i] == 0) continue;  // the search wants strictly increasing starts
+        tab.p[tab.parts] = partials[i];
+        tab.w[tab.parts] = weights[i];
+        tab.first[tab.parts + 1] = tab.first[tab.parts] + counts[i];
+        ++tab.parts;
+    }
+    norm_finalize_parts_kernel<<<1, kFinalBlock, 0, as_stream(stream)>>>(
+        tab, max_norm, NormOutputs{sum_out, norm_out, grad_mul_out, grad_mul64_out, nonfinite_out});
+    return check_launch("hbt_grad_norm_finalize_parts");
 }
 
 int32_t hbt_grad_norm_noalloc(const void* const* grads, const int64_t* numels, const double* weights,
@@ -2226,8 +2307,8 @@ int32_t hbt_grad_norm_noalloc(const void* const* grads, const int64_t* numels, c
     // kernel reads it, so the array needs no clearing between calls.
     status = launch_sqnorm("hbt_grad_norm_noalloc", tab, chunks, grad_dtype, unscale, partials, st);
     if (status != HBT_OK) return status;
-    norm_finalize_kernel<<<1, kFinalBlock, 0, st>>>(partials, chunks, max_norm, sum_out, norm_out,
-                                                   grad_mul_out, nullptr, nonfinite_out);
+    norm_finalize_kernel<<<1, kFinalBlock, 0, st>>>(
+        partials, chunks, max_norm, NormOutputs{sum_out, norm_out, grad_mul_out, nullptr, nonfinite_out});
     return check_launch("hbt_grad_norm_noalloc");
 }
 

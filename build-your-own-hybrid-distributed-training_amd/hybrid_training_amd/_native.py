@@ -51,6 +51,7 @@ __all__ = [
     "EXPORTED_SYMBOLS",
     "GraphRecording",
     "MAX_LOCAL_RANKS",
+    "MAX_NORM_PARTS",
     "MAX_TENSORS_PER_LAUNCH",
     "PIECES_PER_NORM_CHUNK",
     "check",
@@ -64,9 +65,10 @@ __all__ = [
     "stream_of",
 ]
 
-ABI_VERSION = 18
+ABI_VERSION = 19
 MAX_TENSORS_PER_LAUNCH = 16
 MAX_LOCAL_RANKS = 64
+MAX_NORM_PARTS = 128
 #: Doubles of working storage hbt_scale_inplace_sqnorm takes per partial for 2-byte gradients.
 PIECES_PER_NORM_CHUNK = 128
 
@@ -141,6 +143,11 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
     "hbt_grad_norm_finalize": (
         _c_i32,
         (_c_void_p, _c_i64, _c_f64, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p),
+    ),
+    "hbt_grad_norm_finalize_parts": (
+        _c_i32,
+        (_ptr_array, _i64_array, _f64_array, _c_i32, _c_f64, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+         _c_void_p),
     ),
     "hbt_grad_norm_noalloc": (
         _c_i32,

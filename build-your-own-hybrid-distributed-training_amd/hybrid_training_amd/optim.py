@@ -389,67 +389,49 @@ def gradient_norm_pass(
             batches.setdefault((grad.dtype, _pending_unscale(grad)), []).append(
                 (grad, offset, length, weight)
             )
+    # Every segment's partials in summation order: the ones its producer left, where they
+    # lie, or a run of slots in a fresh array that this pass fills.
+    slots = 0
+    order: list[tuple[torch.Tensor | None, int, int, float]] = []  # (producer's partials or None, slot, count, weight)
     launches: list[tuple[torch.dtype, float, list[tuple[torch.Tensor, int, int, float]], int]] = []
-    total_partials = 0
+    fresh: list[tuple[torch.Tensor, int, int, int, int]] = []  # segments whose partials are tagged
     for (dtype, unscale), items in batches.items():
         chunk_elems = norm_chunk_elems(dtype)  # hbt_norm_partials_count's chunk
-        for start in range(0, len(items), _native.MAX_TENSORS_PER_LAUNCH):
-            chunk = items[start : start + _native.MAX_TENSORS_PER_LAUNCH]
-            launches.append((dtype, unscale, chunk, total_partials))
-            total_partials += sum(-(-n // chunk_elems) for _, _, n, _ in chunk)
+        batch: list[tuple[torch.Tensor, int, int, float]] = []
+        for item in items:
+            grad, offset, length, weight = item
+            count = -(-length // chunk_elems)
+            cached = _cached_partials(grad, offset, length, unscale)
+            if cached is not None and cached.numel() == count and cached.is_contiguous():
+                # Partials a producer wrote over exact zeros are the same +0.0 under any
+                # finite non-negative weight.
+                if 0.0 <= weight < float("inf") and _zero_segment(grad, offset, length):
+                    weight = 1.0
+                order.append((cached, 0, count, weight))
+                continue
+            if tag and weight == 1.0 and unscale == 1.0:
+                fresh.append((grad, offset, length, slots, count))
+            if is_host(grad):
+                launches.append((dtype, unscale, [item], slots))
+            else:
+                if not batch or len(batch) == _native.MAX_TENSORS_PER_LAUNCH or is_host(launches[-1][2][0][0]):
+                    batch = []
+                    launches.append((dtype, unscale, batch, slots))
+                batch.append(item)
+            order.append((None, slots, count, 1.0))  # written with its weight applied
+            slots += count
     # sum, norm and the double clip multiplier, then the fp32 multiplier and the flag in
     # the last 8 bytes: one allocation for the finalize's outputs.
     scalars = torch.empty(4, dtype=torch.float64, device=device)
-    out = scalars.data_ptr()
+    partials = torch.empty(slots, dtype=torch.float64, device=device) if slots else None
     stream = _native.stream_of(device)
-    whole = _contiguous_cached_partials(launches, total_partials)
-    if whole is not None:
-        # Every segment's partials were written by its producer, with weight 1, one after
-        # another in one tensor in slot order: the finalize reads them where they are.
-        with _native.device_guard(device):
-            _native.check(lib.hbt_grad_norm_finalize(whole, total_partials, float(max_norm), out, out + 8,
-                                                     out + 24, out + 16, out + 28, stream),
-                          "optim.hbt_grad_norm_finalize")
-        return NormResult(scalars)
-    partials = torch.empty(max(1, total_partials), dtype=torch.float64, device=device)
-    fresh: list[tuple[torch.Tensor, int, int, int, int]] = []  # segments whose partials are tagged
     with _native.device_guard(device):
         for dtype, unscale, items, first in launches:
-            # Items whose producer already wrote their partials take them from there
-            # (times the weight, as the kernel would multiply); the others are summed
-            # here, each run of consecutive uncached items in one launch.  Every item
-            # keeps its slot, and the finalize sums the slots in a fixed order.
-            slot = first
-            pending: list[tuple[torch.Tensor, int, int, float]] = []
-            pending_first = slot
-            for grad, offset, length, weight in items:
-                count = int(lib.hbt_norm_partials_count(_native.int64_array([length]), 1, _native.dtype_code(dtype)))
-                cached = _cached_partials(grad, offset, length, unscale)
-                if tag and cached is None and weight == 1.0 and unscale == 1.0:
-                    fresh.append((grad, offset, length, slot, count))
-                if cached is not None and cached.numel() == count:
-                    _launch_sqnorm(lib, pending, dtype, unscale, partials, pending_first, stream)
-                    pending = []
-                    target = partials[slot : slot + count]
-                    if weight == 1.0:
-                        plan = _native.CopyPlan(device)
-                        plan.add(cached, 0, target, 0, count)
-                        plan.run(src_dtype=torch.float64, dst_dtype=torch.float64)
-                    else:
-                        torch.mul(cached, weight, out=target)
-                    pending_first = slot + count
-                elif is_host(grad):
-                    _launch_sqnorm(lib, pending, dtype, unscale, partials, pending_first, stream)
-                    pending = []
-                    _stream_sqnorm(lib, grad, offset, length, weight, dtype, unscale, partials, slot, device)
-                    pending_first = slot + count
-                else:
-                    pending.append((grad, offset, length, weight))
-                slot += count
-            _launch_sqnorm(lib, pending, dtype, unscale, partials, pending_first, stream)
-        status = lib.hbt_grad_norm_finalize(partials.data_ptr(), total_partials, float(max_norm), out, out + 8,
-                                            out + 24, out + 16, out + 28, stream)
-        _native.check(status, "optim.hbt_grad_norm_finalize")
+            if is_host(items[0][0]):
+                _stream_sqnorm(lib, *items[0], dtype, unscale, partials, first, device)
+            else:
+                _launch_sqnorm(lib, items, dtype, unscale, partials, first, stream)
+        _finalize(lib, order, partials, scalars, max_norm, device, stream)
     records: dict[int, tuple[torch.Tensor, dict[tuple[int, int], torch.Tensor]]] = {}
     for grad, offset, length, slot, count in fresh:
         records.setdefault(id(grad), (grad, {}))[1][(offset, length)] = partials[slot : slot + count]
@@ -469,33 +451,40 @@ def _zero_segment(grad: torch.Tensor, offset: int, length: int) -> bool:
     return record is not None and record.lookup(grad, offset, length) is not None and (offset, length) in record.zero
 
 
-def _contiguous_cached_partials(launches, total_partials: int) -> int | None:
-    """The device address of the partials of every segment in ``launches``, when each
-    segment has a producer's partials (:class:`NormPartials`) and no pending unscale,
-    has weight 1 or was written as exact zeros (its +0.0 partials times any finite
-    non-negative weight are the same +0.0), and those partials lie one after another in
-    one tensor in slot order, so a finalize over that address sees what the weighted
-    copy into a fresh array would give it."""
-    address = None
-    expected = None
-    for dtype, unscale, items, _ in launches:
-        if unscale != 1.0:
-            return None
-        chunk_elems = norm_chunk_elems(dtype)
-        for grad, offset, length, weight in items:
-            if weight != 1.0 and not (0.0 <= weight < float("inf") and _zero_segment(grad, offset, length)):
-                return None
-            cached = _cached_partials(grad, offset, length, unscale)
-            if cached is None or cached.numel() != -(-length // chunk_elems) or not cached.is_contiguous():
-                return None
-            if address is None:
-                address = cached.data_ptr()
-            elif cached.data_ptr() != expected:
-                return None
-            expected = cached.data_ptr() + 8 * cached.numel()
-    if address is None or expected - address != 8 * total_partials:
-        return None
-    return address
+def _finalize(lib, order, partials, scalars, max_norm, device, stream) -> None:
+    """Sum the partials of ``order`` into ``scalars`` (:class:`NormResult`'s layout) in one
+    launch: over one array when they lie one after another with weight 1, else over the
+    list of arrays.  Lists past ``MAX_NORM_PARTS`` arrays are gathered into one first."""
+    parts: list[tuple[int, int, float]] = []  # (address, count, weight), adjacent ones merged
+    for cached, slot, count, weight in order:
+        address = partials.data_ptr() + 8 * slot if cached is None else cached.data_ptr()
+        if parts and parts[-1][2] == weight and parts[-1][0] + 8 * parts[-1][1] == address:
+            parts[-1] = (parts[-1][0], parts[-1][1] + count, weight)
+        else:
+            parts.append((address, count, weight))
+    if len(parts) > _native.MAX_NORM_PARTS:
+        whole = torch.empty(sum(count for _, _, count, _ in order), dtype=torch.float64, device=device)
+        plan, first = _native.CopyPlan(device), 0
+        for cached, slot, count, weight in order:
+            source = partials[slot : slot + count] if cached is None else cached
+            if weight == 1.0:
+                plan.add(source, 0, whole, first, count)
+            else:
+                torch.mul(source, weight, out=whole[first : first + count])
+            first += count
+        plan.run(src_dtype=torch.float64, dst_dtype=torch.float64)
+        parts = [(whole.data_ptr(), first, 1.0)]
+    out = scalars.data_ptr()
+    outputs = (out, out + 8, out + 24, out + 16, out + 28, stream)
+    if len(parts) <= 1 and all(weight == 1.0 for _, _, weight in parts):
+        address, count, _ = parts[0] if parts else (None, 0, 1.0)
+        status = lib.hbt_grad_norm_finalize(address, count, float(max_norm), *outputs)
+        _native.check(status, "optim.hbt_grad_norm_finalize")
+        return
+    status = lib.hbt_grad_norm_finalize_parts(
+        _native.pointer_array([p for p, _, _ in parts]), _native.int64_array([n for _, n, _ in parts]),
+        _native.double_array([w for _, _, w in parts]), len(parts), float(max_norm), *outputs)
+    _native.check(status, "optim.hbt_grad_norm_finalize_parts")
 
 
 def norm_chunk_elems(dtype: torch.dtype) -> int:

@@ -170,6 +170,26 @@ int32_t hbt_grad_norm_finalize(const double* partials, int64_t count, double max
                                double* grad_mul64_out, int32_t* nonfinite_out, void* stream);
 
 /* ------------------------------------------------------------------------------
+ * Stage 2 over partials in several arrays: what hbt_grad_norm_finalize writes for one
+ * array that holds weights[0] * partials[0][0 .. counts[0]), then weights[1] *
+ * partials[1][0 .. counts[1]), and so on, bitwise, in one launch that reads each array
+ * where it lies.
+ *
+ * Replaces: distributed_gradient_norm's sum over contributions, clamp and sqrt
+ *   (optim/sharded_optimizer.py:236-241) and the clip-coefficient arithmetic of
+ *   ShardedOptimizer.clip_grad_norm (optim/sharded_optimizer.py:331-337), for gradients
+ *   whose producers left their partials (one array per FSDP unit).
+ * At most HBT_MAX_NORM_PARTS arrays; the table travels in the launch's arguments, so a
+ * recorded launch reads the same arrays at every replay.  The outputs are as for
+ * hbt_grad_norm_finalize.
+ * ---------------------------------------------------------------------------- */
+#define HBT_MAX_NORM_PARTS 128
+int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_t* counts, const double* weights,
+                                     int32_t parts, double max_norm, double* sum_out, double* norm_out,
+                                     float* grad_mul_out, double* grad_mul64_out, int32_t* nonfinite_out,
+                                     void* stream);
+
+/* ------------------------------------------------------------------------------
  * Weighted squared norm and clip coefficient with no allocation and no workspace.
  *
  * This entry point has no counterpart in the reference.  It is for callers that

@@ -614,3 +614,44 @@ def test_learning_rate_schedule_without_weight_decay(device):
         rel = np.abs(got - ref.detach().numpy()) / np.maximum(np.abs(ref.detach().numpy()), lr)
         assert float(rel.max()) <= 1e-6
     assert opt.learning_rate == 2.5e-4
+
+
+@pytest.mark.parametrize("counts", [[1], [0, 3, 0], [1] * 128, [1023, 1, 1025, 4096, 7], [5000] * 3 + [1] * 20])
+def test_finalize_over_parts_is_the_finalize_over_one_array(device, counts):
+    """Partials summed where their producers left them, weighted per array: every output
+    bitwise that of one array holding the weighted partials one after another."""
+    lib = _native.library()
+    gen = torch.Generator(device=device).manual_seed(len(counts))
+    arrays = [torch.rand(n + 1, dtype=torch.float64, device=device, generator=gen)[1:] for n in counts]
+    weights = [(1.0, 0.125, 3.0)[i % 3] for i in range(len(counts))]
+    whole = torch.cat([a * w for a, w in zip(arrays, weights)])
+    outs = [torch.full((4,), 9.0, dtype=torch.float64, device=device) for _ in range(2)]
+    stream = _native.stream_of(device)
+
+    def args(o):
+        p = o.data_ptr()
+        return p, p + 8, p + 24, p + 16, p + 28, stream
+
+    _native.check(lib.hbt_grad_norm_finalize(whole.data_ptr() if whole.numel() else None, whole.numel(), 0.5,
+                                             *args(outs[0])), "test.finalize")
+    _native.check(lib.hbt_grad_norm_finalize_parts(
+        _native.pointer_array([a.data_ptr() for a in arrays]), _native.int64_array(counts),
+        _native.double_array(weights), len(counts), 0.5, *args(outs[1])), "test.finalize_parts")
+    assert torch.equal(outs[0].view(torch.int64), outs[1].view(torch.int64))
+
+
+@pytest.mark.parametrize("tensors", [3, 128, 131])
+def test_norm_from_partials_in_many_arrays(device, tensors):
+    """Gradients that each carry their own partials, some weighted, one of them summed here,
+    at array counts up to and past one launch's table: within 1e-12 of the plain sum, twice
+    the same bits."""
+    gen = torch.Generator(device=device).manual_seed(tensors)
+    grads = [torch.randn(40_000 if i % 50 == 0 else 100, device=device, generator=gen) for i in range(tensors)]
+    for g in grads[:-1]:
+        gradient_norm_pass([(g, 0, g.numel(), 1.0)], device, max_norm=0.0, tag=True)
+    segments = [(g, 0, g.numel(), 0.5 if i % 5 == 1 else 1.0) for i, g in enumerate(grads)]
+    first = gradient_norm_pass(segments, device, max_norm=1.0)
+    again = gradient_norm_pass(segments, device, max_norm=1.0)
+    assert torch.equal(first.scalars.view(torch.int64), again.scalars.view(torch.int64))
+    ref = float(sum(w * g.double().square().sum() for g, _, _, w in segments))
+    assert abs(float(first.sum) - ref) <= 1e-12 * ref
