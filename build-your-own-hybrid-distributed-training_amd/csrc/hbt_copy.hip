@@ -8,9 +8,9 @@
 // taking consecutive units, so every load and store instruction of a wave covers one
 // contiguous span.
 //
-// Two kernels share that layout.  copy_aligned_kernel serves plans whose records all
+// Two ways to move a chunk share that layout.  CopyAligned serves plans whose records all
 // start on aligned addresses (the host certifies this): one aligned load and one aligned
-// store per unit.  copy_kernel serves any plan: it cuts each record's chunks on 128-byte
+// store per unit.  CopyAny serves any plan: it cuts each record's chunks on 128-byte
 // lines of the destination, so that only a record's first and last chunk write part of a
 // line, and reads its units where they lie with unaligned vector loads.  A load never
 // touches a byte outside the source interval.
@@ -189,34 +189,70 @@ __device__ __forceinline__ void store_unit(gbyte* d, const typename Vec<unit_ele
     }
 }
 
-// Index of the record that owns `chunk`: the last record whose first_chunk <= chunk
-// (the host drops records with no chunks, so first_chunk strictly increases).  The
-// search runs on the scalar unit: its loads hit the scalar cache and do not queue behind
-// the vector traffic of the waves in flight (a wave-wide search over vector loads waits
-// behind that traffic and was slower).  With
-// hints (the table followed by hints[j] = the record owning chunk j * kHintStride) the
-// search starts at the hinted record and steps forward, at most as many records as
-// start inside one hint stride; without them it bisects the whole table, log2(count)
-// dependent loads before the workgroup's first data load.
+// The interval a chunk belongs to.
+struct Record {
+    int64_t src;  // 0: write zeros
+    int64_t dst;
+    int64_t n;
+    int64_t first;  // its first chunk
+};
+
+// The record that owns `chunk`: the last one whose first_chunk <= chunk (records with no
+// chunks are dropped by the host, so first_chunk strictly increases).  The search runs on
+// the scalar unit: its loads hit the scalar cache and do not queue behind the vector
+// traffic of the waves in flight (a wave-wide search over vector loads waits behind that
+// traffic and was slower).  With hints (the table followed by hints[j] = the record owning
+// chunk j * kHintStride) the search starts at the hinted record and steps forward, at most
+// as many records as start inside one hint stride; without them it bisects the whole
+// table, log2(count) dependent loads before the workgroup's first data load.
 constexpr int kHintShift = 8;  // one hint per 256 chunks
-__device__ __forceinline__ int64_t owning_record(const int64_t* __restrict__ table, int64_t count,
-                                                 int64_t chunk, const int64_t* __restrict__ hints) {
+__device__ __forceinline__ Record owning_record(const int64_t* __restrict__ table, int64_t count,
+                                                int64_t chunk, const int64_t* __restrict__ hints) {
+    int64_t lo = 0;
     if (hints != nullptr) {
-        int64_t r = hints[chunk >> kHintShift];
-        r = r < 0 ? 0 : (r < count ? r : count - 1);  // a wrong hint stays inside the table
-        while (r + 1 < count && table[4 * (r + 1) + 3] <= chunk) ++r;
-        return r;
-    }
-    int64_t lo = 0, hi = count - 1;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi + 1) >> 1;
-        if (table[4 * mid + 3] <= chunk) {
-            lo = mid;
-        } else {
-            hi = mid - 1;
+        lo = hints[chunk >> kHintShift];
+        lo = lo < 0 ? 0 : (lo < count ? lo : count - 1);  // a wrong hint stays inside the table
+        while (lo + 1 < count && table[4 * (lo + 1) + 3] <= chunk) ++lo;
+    } else {
+        int64_t hi = count - 1;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (table[4 * mid + 3] <= chunk) {
+                lo = mid;
+            } else {
+                hi = mid - 1;
+            }
         }
     }
-    return lo;
+    const int64_t* rec = table + 4 * lo;
+    return Record{rec[0], rec[1], rec[2], rec[3]};
+}
+
+// A plan of up to HBT_COPY_MAX_ROWS records in the launch's own arguments, with a hint for
+// every 2^shift chunks (kRowHints of them cover the plan), four to a word: the record that
+// owns the first of them.  A plan built for
+// one use, such as an unpack into fresh tensors, then needs no table built in pinned memory
+// and uploaded ahead of the launch: 52 GPT-2 tensors rebuilt from 5 ragged shards (542 MB, 101 us of
+// kernel) took 406 us a call with the table and took 115 us without, the rows counted by
+// arithmetic; a Llama-3-8B layer gathered from 8 shards 199 and 197 us.  3.9 KB, inside the 4 KB a launch's arguments may take.
+constexpr int kRowHints = 256;
+constexpr uint32_t kHintSplit = 128;  // set when another record starts among the hint's chunks
+struct RowTable {
+    Record rec[HBT_COPY_MAX_ROWS];
+    uint32_t hint[kRowHints / 4];
+    int32_t count;
+    int32_t shift;
+};
+static_assert(HBT_COPY_MAX_ROWS <= kHintSplit, "a hint is one byte: a record and the split bit");
+static_assert(sizeof(RowTable) + 32 <= 4096, "the arguments of a launch");
+__device__ __forceinline__ Record owning_record(const RowTable& rows, int64_t chunk) {
+    const uint32_t j = static_cast<uint32_t>(chunk >> rows.shift);
+    const uint32_t hint = (rows.hint[j >> 2] >> (8 * (j & 3u))) & 0xFFu;
+    int r = static_cast<int>(hint & (kHintSplit - 1u));
+    if ((hint & kHintSplit) != 0) {
+        while (r + 1 < rows.count && rows.rec[r + 1].first <= chunk) ++r;
+    }
+    return rows.rec[r];  // one indexed read: a Record copied on two paths moves the table to scratch
 }
 
 // Any plan.  A record's chunk c covers elements [line + c * kChunk, line + (c + 1) * kChunk)
@@ -230,16 +266,16 @@ __device__ __forceinline__ int64_t owning_record(const int64_t* __restrict__ tab
 // this: source 2 bytes off 5,160 and 6,240; destination 2 off 4,600 and 6,210; both
 // 4,590 and 6,250; destination 16 off 5,850 and 6,230.
 template <int SB, int DB, int OP, bool H>
-__global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restrict__ table,
-                                                          int64_t count, float divisor, int64_t chunk_base,
-                                                          const int64_t* __restrict__ hints) {
+struct CopyAny {
+    typedef float Divisor;
+    static __device__ __forceinline__ void run(const Record& rec, int64_t c, float divisor);
+};
+template <int SB, int DB, int OP, bool H>
+__device__ __forceinline__ void CopyAny<SB, DB, OP, H>::run(const Record& rec, int64_t c, float divisor) {
     static_assert(kCopyBlock == 64, "a workgroup is one wave; its chunk is whole wave-wide spans of 16-byte source loads");
-    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
-    const int64_t* rec = table + 4 * owning_record(table, count, chunk, hints);
-    const gbyte* src = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec[0]));
-    gbyte* dst = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec[1]));
-    const int64_t n = rec[2];
-    const int64_t c = chunk - rec[3];
+    const gbyte* src = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec.src));
+    gbyte* dst = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec.dst));
+    const int64_t n = rec.n;
     constexpr int64_t kChunk = chunk_elems<SB, DB>();
     constexpr int U = unit_elems<SB, DB>();
     constexpr int kSrcWords = U * SB / 4;
@@ -306,22 +342,23 @@ __global__ __launch_bounds__(kCopyBlock) void copy_kernel(const int64_t* __restr
 // the record's end are masked off; a record whose length is not a whole number of units
 // finishes with an element loop in its last chunk.
 template <int SB, int DB, int OP, bool H>
-__global__ __launch_bounds__(kCopyBlock) void copy_aligned_kernel(const int64_t* __restrict__ table,
-                                                                  int64_t count, float divisor, int64_t chunk_base,
-                                                                  const int64_t* __restrict__ hints) {
+struct CopyAligned {
+    typedef float Divisor;
+    static __device__ __forceinline__ void run(const Record& rec, int64_t c, float divisor);
+};
+template <int SB, int DB, int OP, bool H>
+__device__ __forceinline__ void CopyAligned<SB, DB, OP, H>::run(const Record& rec, int64_t c, float divisor) {
     constexpr int U = unit_elems<SB, DB>();
     constexpr int kSrcWords = U * SB / 4;
     constexpr int64_t kChunk = chunk_elems<SB, DB>();
     constexpr int kPerLane = static_cast<int>(kChunk / U / kCopyBlock);
     static_assert(kChunk == int64_t(kPerLane) * kCopyBlock * U, "a chunk is whole units on every lane");
-    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
-    const int64_t* rec = table + 4 * owning_record(table, count, chunk, hints);
-    const int64_t e0 = (chunk - rec[3]) * kChunk;
-    const int64_t n = rec[2];
+    const int64_t e0 = c * kChunk;
+    const int64_t n = rec.n;
     const int64_t len = (n - e0) < kChunk ? (n - e0) : kChunk;
     const int64_t units = len / U;
-    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec[0]));
-    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec[1])) + e0 * DB;
+    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec.src));
+    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec.dst)) + e0 * DB;
     if (s == nullptr) {
         uint32_t zero[U];
 #pragma unroll
@@ -456,19 +493,20 @@ __device__ __forceinline__ void f64_to_words(const double (&x)[U], uint32_t (&w)
 // Any plan: lane l converts elements l, l + 64, ... of its chunk, so every load and store
 // instruction of the wave covers one contiguous span.
 template <int SD, int DD, int OP>
-__global__ __launch_bounds__(kCopyBlock) void convert_kernel(const int64_t* __restrict__ table, int64_t count,
-                                                             double divisor, int64_t chunk_base,
-                                                             const int64_t* __restrict__ hints) {
+struct ConvertAny {
+    typedef double Divisor;
+    static __device__ __forceinline__ void run(const Record& rec, int64_t c, double divisor);
+};
+template <int SD, int DD, int OP>
+__device__ __forceinline__ void ConvertAny<SD, DD, OP>::run(const Record& rec, int64_t c, double divisor) {
     constexpr int64_t SB = elem_bytes<SD>();
     constexpr int64_t DB = elem_bytes<DD>();
     constexpr int64_t kChunk = chunk_elems<SB, DB>();
-    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
-    const int64_t* rec = table + 4 * owning_record(table, count, chunk, hints);
-    const int64_t e0 = (chunk - rec[3]) * kChunk;
-    const int64_t n = rec[2];
+    const int64_t e0 = c * kChunk;
+    const int64_t n = rec.n;
     const int64_t len = (n - e0) < kChunk ? (n - e0) : kChunk;
-    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec[0]));
-    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec[1])) + e0 * DB;
+    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec.src));
+    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec.dst)) + e0 * DB;
     if (s != nullptr) s += e0 * SB;
     for (int64_t i = threadIdx.x; i < len; i += kCopyBlock) {
         narrow_store<DD>(d + i * DB, s != nullptr ? apply_op<OP>(widen_elem<SD>(s + i * SB), divisor) : 0.0);
@@ -481,12 +519,14 @@ __global__ __launch_bounds__(kCopyBlock) void convert_kernel(const int64_t* __re
 // lanes on consecutive units; a 1 KB-of-source chunk is kPerLane units per lane (1 for a
 // float64 source; a widening chunk is 2 KB of source, 4 or 8 units per lane), all loaded
 // before the first store.
-// The bits are convert_kernel's.
+// The bits are ConvertAny's.
 template <int SD, int DD, int OP>
-__global__ __launch_bounds__(kCopyBlock) void convert_aligned_kernel(const int64_t* __restrict__ table,
-                                                                     int64_t count, double divisor,
-                                                                     int64_t chunk_base,
-                                                                     const int64_t* __restrict__ hints) {
+struct ConvertAligned {
+    typedef double Divisor;
+    static __device__ __forceinline__ void run(const Record& rec, int64_t c, double divisor);
+};
+template <int SD, int DD, int OP>
+__device__ __forceinline__ void ConvertAligned<SD, DD, OP>::run(const Record& rec, int64_t c, double divisor) {
     constexpr int SB = elem_bytes<SD>();
     constexpr int DB = elem_bytes<DD>();
     constexpr int U = 16 / (SB > DB ? SB : DB);
@@ -495,14 +535,12 @@ __global__ __launch_bounds__(kCopyBlock) void convert_aligned_kernel(const int64
     constexpr int64_t kChunk = chunk_elems<SB, DB>();
     constexpr int kPerLane = static_cast<int>(kChunk / (int64_t(kCopyBlock) * U));
     static_assert(kChunk == int64_t(kPerLane) * kCopyBlock * U, "a chunk is whole units on every lane");
-    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
-    const int64_t* rec = table + 4 * owning_record(table, count, chunk, hints);
-    const int64_t e0 = (chunk - rec[3]) * kChunk;
-    const int64_t n = rec[2];
+    const int64_t e0 = c * kChunk;
+    const int64_t n = rec.n;
     const int64_t len = (n - e0) < kChunk ? (n - e0) : kChunk;
     const int64_t units = len / U;
-    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec[0]));
-    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec[1])) + e0 * DB;
+    const gbyte* s = reinterpret_cast<const gbyte*>(static_cast<uintptr_t>(rec.src));
+    gbyte* d = reinterpret_cast<gbyte*>(static_cast<uintptr_t>(rec.dst)) + e0 * DB;
     if (s == nullptr) {
         uint32_t zero[DW];
 #pragma unroll
@@ -541,69 +579,127 @@ __global__ __launch_bounds__(kCopyBlock) void convert_aligned_kernel(const int64
     }
 }
 
-template <int OP>
-int32_t launch_convert(int32_t src_dtype, int32_t dst_dtype, const int64_t* table, int64_t count, int64_t chunks,
-                       double divisor, bool aligned, const int64_t* hints, hipStream_t st) {
-    return launch_sliced("hbt_copy_intervals", chunks, kCopyBlock, [&](int64_t first, dim3 grid) {
-#define HBT_CVT(SD, DD)                                                                                        \
-    do {                                                                                                       \
-        if (aligned) convert_aligned_kernel<SD, DD, OP><<<grid, kCopyBlock, 0, st>>>(table, count, divisor, first, hints); \
-        else convert_kernel<SD, DD, OP><<<grid, kCopyBlock, 0, st>>>(table, count, divisor, first, hints);    \
-    } while (0)
-        if constexpr (OP != HBT_COPY_OP_COPY) {
-            HBT_CVT(HBT_DTYPE_F64, HBT_DTYPE_F64);  // the only division through double
+// ---- launches ------------------------------------------------------------------------
+template <typename Mover>
+__global__ __launch_bounds__(kCopyBlock) void copy_table_kernel(const int64_t* __restrict__ table, int64_t count,
+                                                                typename Mover::Divisor divisor, int64_t chunk_base,
+                                                                const int64_t* __restrict__ hints) {
+    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
+    const Record rec = owning_record(table, count, chunk, hints);
+    Mover::run(rec, chunk - rec.first, divisor);
+}
+template <typename Mover>
+__global__ __launch_bounds__(kCopyBlock) void copy_rows_kernel(RowTable rows, typename Mover::Divisor divisor,
+                                                               int64_t chunk_base) {
+    const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
+    const Record rec = owning_record(rows, chunk);
+    Mover::run(rec, chunk - rec.first, divisor);
+}
+
+// Where a launch finds its records: a device table, or the arguments (rows non-null).
+struct Plan {
+    const char* who;
+    const int64_t* table;
+    int64_t count;
+    const int64_t* hints;
+    const RowTable* rows;
+    int64_t chunks;
+    bool aligned;
+    hipStream_t stream;
+};
+template <typename Mover>
+int32_t launch_mover(const Plan& p, typename Mover::Divisor divisor) {
+    return launch_sliced(p.who, p.chunks, kCopyBlock, [&](int64_t first, dim3 grid) {
+        if (p.rows != nullptr) {
+            copy_rows_kernel<Mover><<<grid, kCopyBlock, 0, p.stream>>>(*p.rows, divisor, first);
         } else {
-#define HBT_CVT_TO(SD)                                                                                   \
-    do {                                                                                                 \
-        if (dst_dtype == HBT_DTYPE_F64) HBT_CVT(SD, HBT_DTYPE_F64);                                      \
-        else if (dst_dtype == HBT_DTYPE_F32) HBT_CVT(SD, HBT_DTYPE_F32);                                 \
-        else if (dst_dtype == HBT_DTYPE_BF16) HBT_CVT(SD, HBT_DTYPE_BF16);                               \
-        else HBT_CVT(SD, HBT_DTYPE_F16);                                                                 \
-    } while (0)
-            if (src_dtype == HBT_DTYPE_F64) HBT_CVT_TO(HBT_DTYPE_F64);
-            else if (src_dtype == HBT_DTYPE_F32) HBT_CVT_TO(HBT_DTYPE_F32);
-            else if (src_dtype == HBT_DTYPE_BF16) HBT_CVT_TO(HBT_DTYPE_BF16);
-            else HBT_CVT_TO(HBT_DTYPE_F16);
-#undef HBT_CVT_TO
+            copy_table_kernel<Mover><<<grid, kCopyBlock, 0, p.stream>>>(p.table, p.count, divisor, first, p.hints);
         }
-#undef HBT_CVT
     });
+}
+template <int SD, int DD, int OP>
+int32_t launch_convert_pair(const Plan& p, double divisor) {
+    return p.aligned ? launch_mover<ConvertAligned<SD, DD, OP>>(p, divisor) : launch_mover<ConvertAny<SD, DD, OP>>(p, divisor);
+}
+template <int SD>
+int32_t launch_convert_from(const Plan& p, int32_t dst_dtype) {
+    if (dst_dtype == HBT_DTYPE_F64) return launch_convert_pair<SD, HBT_DTYPE_F64, HBT_COPY_OP_COPY>(p, 1.0);
+    if (dst_dtype == HBT_DTYPE_F32) return launch_convert_pair<SD, HBT_DTYPE_F32, HBT_COPY_OP_COPY>(p, 1.0);
+    if (dst_dtype == HBT_DTYPE_BF16) return launch_convert_pair<SD, HBT_DTYPE_BF16, HBT_COPY_OP_COPY>(p, 1.0);
+    return launch_convert_pair<SD, HBT_DTYPE_F16, HBT_COPY_OP_COPY>(p, 1.0);
+}
+int32_t launch_convert(const Plan& p, int32_t src_dtype, int32_t dst_dtype) {
+    if (src_dtype == HBT_DTYPE_F64) return launch_convert_from<HBT_DTYPE_F64>(p, dst_dtype);
+    if (src_dtype == HBT_DTYPE_F32) return launch_convert_from<HBT_DTYPE_F32>(p, dst_dtype);
+    if (src_dtype == HBT_DTYPE_BF16) return launch_convert_from<HBT_DTYPE_BF16>(p, dst_dtype);
+    return launch_convert_from<HBT_DTYPE_F16>(p, dst_dtype);
 }
 
 template <int SB, int DB, int OP, bool H = false>
-int32_t launch_copy(const int64_t* table, int64_t count, int64_t chunks, float divisor, bool aligned,
-                    const int64_t* hints, hipStream_t s) {
-    return launch_sliced("hbt_copy_intervals", chunks, kCopyBlock, [&](int64_t first, dim3 grid) {
-        if (aligned) {
-            copy_aligned_kernel<SB, DB, OP, H><<<grid, kCopyBlock, 0, s>>>(table, count, divisor, first, hints);
-        } else {
-            copy_kernel<SB, DB, OP, H><<<grid, kCopyBlock, 0, s>>>(table, count, divisor, first, hints);
-        }
-    });
+int32_t launch_copy(const Plan& p, float divisor) {
+    return p.aligned ? launch_mover<CopyAligned<SB, DB, OP, H>>(p, divisor) : launch_mover<CopyAny<SB, DB, OP, H>>(p, divisor);
 }
 
 // Conversions and division for 4- and 2-byte elements; H: the 2-byte side is fp16.
 // Division by a power of two (the AVG pre-divide at a power-of-two world size) runs as a
 // multiply by the exact reciprocal: the same bits, without the division sequence.
+template <int OP, bool H>
+int32_t launch_arith_op(const Plan& p, int ssz, int dsz, float divisor) {
+    if (ssz == 4 && dsz == 4) return launch_copy<4, 4, OP>(p, divisor);
+    if (ssz == 2 && dsz == 2) return launch_copy<2, 2, OP, H>(p, divisor);
+    if (ssz == 4) return launch_copy<4, 2, OP, H>(p, divisor);
+    return launch_copy<2, 4, OP, H>(p, divisor);
+}
 template <bool H>
-int32_t launch_arith(int ssz, int dsz, int32_t op, float divisor, const int64_t* table, int64_t count,
-                     int64_t chunks, bool aligned, const int64_t* hints, hipStream_t s) {
-    const float recip = op == HBT_COPY_OP_DIVIDE ? exact_reciprocal(divisor) : 0.0f;
-    if (op == HBT_COPY_OP_DIVIDE && recip != 0.0f) {
-        if (ssz == 4 && dsz == 4) return launch_copy<4, 4, kOpScale>(table, count, chunks, recip, aligned, hints, s);
-        if (ssz == 2 && dsz == 2) return launch_copy<2, 2, kOpScale, H>(table, count, chunks, recip, aligned, hints, s);
-        if (ssz == 4) return launch_copy<4, 2, kOpScale, H>(table, count, chunks, recip, aligned, hints, s);
-        return launch_copy<2, 4, kOpScale, H>(table, count, chunks, recip, aligned, hints, s);
-    }
+int32_t launch_arith(const Plan& p, int ssz, int dsz, int32_t op, float divisor) {
     if (op == HBT_COPY_OP_DIVIDE) {
-        if (ssz == 4 && dsz == 4) return launch_copy<4, 4, HBT_COPY_OP_DIVIDE>(table, count, chunks, divisor, aligned, hints, s);
-        if (ssz == 2 && dsz == 2) return launch_copy<2, 2, HBT_COPY_OP_DIVIDE, H>(table, count, chunks, divisor, aligned, hints, s);
-        if (ssz == 4) return launch_copy<4, 2, HBT_COPY_OP_DIVIDE, H>(table, count, chunks, divisor, aligned, hints, s);
-        return launch_copy<2, 4, HBT_COPY_OP_DIVIDE, H>(table, count, chunks, divisor, aligned, hints, s);
+        const float recip = exact_reciprocal(divisor);
+        if (recip != 0.0f) return launch_arith_op<kOpScale, H>(p, ssz, dsz, recip);
+        return launch_arith_op<HBT_COPY_OP_DIVIDE, H>(p, ssz, dsz, divisor);
     }
     // conversions (same-dtype copies are bit copies)
-    if (ssz == 4) return launch_copy<4, 2, HBT_COPY_OP_COPY, H>(table, count, chunks, divisor, aligned, hints, s);
-    return launch_copy<2, 4, HBT_COPY_OP_COPY, H>(table, count, chunks, divisor, aligned, hints, s);
+    if (ssz == 4) return launch_copy<4, 2, HBT_COPY_OP_COPY, H>(p, divisor);
+    return launch_copy<2, 4, HBT_COPY_OP_COPY, H>(p, divisor);
+}
+
+// Launches a validated plan (a known dtype pair and op, at least one chunk).
+int32_t launch_plan(const Plan& p, int32_t src_dtype, int32_t dst_dtype, int32_t op, float divisor) {
+    const int ssz = dtype_size(src_dtype);
+    const int dsz = dtype_size(dst_dtype);
+    if (op == HBT_COPY_OP_DIVIDE && src_dtype == HBT_DTYPE_F64 && dst_dtype == HBT_DTYPE_F64) {
+        const float recip = exact_reciprocal(divisor);
+        if (recip != 0.0f) return launch_convert_pair<HBT_DTYPE_F64, HBT_DTYPE_F64, kOpScale>(p, recip);
+        return launch_convert_pair<HBT_DTYPE_F64, HBT_DTYPE_F64, HBT_COPY_OP_DIVIDE>(p, divisor);
+    }
+    if (op == HBT_COPY_OP_COPY && src_dtype == dst_dtype) {
+        // Bit copy; fp64 moves as pairs of dwords (the host doubles its numels).
+        if (ssz == 2) return launch_copy<2, 2, HBT_COPY_OP_COPY>(p, divisor);
+        if (ssz == 4) return launch_copy<4, 4, HBT_COPY_OP_COPY>(p, divisor);
+        set_error("%s: 8-byte elements must be passed as dword pairs (F32)", p.who);
+        return HBT_ERR_UNSUPPORTED;
+    }
+    const bool wide = ssz == 8 || dsz == 8;
+    const bool mixed_16 = (src_dtype == HBT_DTYPE_BF16 && dst_dtype == HBT_DTYPE_F16) ||
+                          (src_dtype == HBT_DTYPE_F16 && dst_dtype == HBT_DTYPE_BF16);
+    if (wide || mixed_16) {
+        if (op != HBT_COPY_OP_COPY) {
+            set_error("%s: division moves data within one dtype (F64, F32, BF16 or F16) or "
+                      "between F32 and a 2-byte dtype (got %d -> %d)", p.who, src_dtype, dst_dtype);
+            return HBT_ERR_UNSUPPORTED;
+        }
+        return launch_convert(p, src_dtype, dst_dtype);
+    }
+    if (src_dtype == HBT_DTYPE_F16 || dst_dtype == HBT_DTYPE_F16) return launch_arith<true>(p, ssz, dsz, op, divisor);
+    return launch_arith<false>(p, ssz, dsz, op, divisor);
+}
+
+bool copy_op_ok(const char* who, int32_t src_dtype, int32_t dst_dtype, int32_t op) {
+    if (dtype_size(src_dtype) == 0 || dtype_size(dst_dtype) == 0 ||
+        (op != HBT_COPY_OP_COPY && op != HBT_COPY_OP_DIVIDE)) {
+        set_error("%s: bad dtype pair (%d, %d) or op %d", who, src_dtype, dst_dtype, op);
+        return false;
+    }
+    return true;
 }
 
 }  // namespace
@@ -637,45 +733,53 @@ int32_t hbt_copy_intervals(const int64_t* table, int64_t count, int64_t total_ch
     }
     const bool aligned = (flags & HBT_COPY_ALIGNED) != 0;
     if (count == 0 || total_chunks == 0) return HBT_OK;
+    if (!copy_op_ok("hbt_copy_intervals", src_dtype, dst_dtype, op)) return HBT_ERR_INVALID_ARGUMENT;
     // The hints follow the count records of 4 int64 each.
     const int64_t* hints = (flags & HBT_COPY_HINTS) != 0 ? table + 4 * count : nullptr;
-    const int ssz = dtype_size(src_dtype);
-    const int dsz = dtype_size(dst_dtype);
-    if (ssz == 0 || dsz == 0 || (op != HBT_COPY_OP_COPY && op != HBT_COPY_OP_DIVIDE)) {
-        set_error("hbt_copy_intervals: bad dtype pair (%d, %d) or op %d", src_dtype, dst_dtype, op);
+    return launch_plan(Plan{"hbt_copy_intervals", table, count, hints, nullptr, total_chunks, aligned, as_stream(stream)},
+                       src_dtype, dst_dtype, op, divisor);
+}
+
+int32_t hbt_copy_rows(const int64_t* rows, int32_t count, int32_t src_dtype, int32_t dst_dtype, int32_t op,
+                      float divisor, void* stream) {
+    clear_error();
+    if (count < 0 || count > HBT_COPY_MAX_ROWS || (count > 0 && rows == nullptr)) {
+        set_error("hbt_copy_rows: bad rows/count (%d of at most %d)", count, HBT_COPY_MAX_ROWS);
         return HBT_ERR_INVALID_ARGUMENT;
     }
-    hipStream_t s = as_stream(stream);
-    if (op == HBT_COPY_OP_DIVIDE && src_dtype == HBT_DTYPE_F64 && dst_dtype == HBT_DTYPE_F64) {
-        const float recip = exact_reciprocal(divisor);
-        if (recip != 0.0f)
-            return launch_convert<kOpScale>(src_dtype, dst_dtype, table, count, total_chunks, recip, aligned, hints, s);
-        return launch_convert<HBT_COPY_OP_DIVIDE>(src_dtype, dst_dtype, table, count, total_chunks, divisor, aligned,
-                                                  hints, s);
+    if (!copy_op_ok("hbt_copy_rows", src_dtype, dst_dtype, op)) return HBT_ERR_INVALID_ARGUMENT;
+    int64_t scale = 1;
+    if (src_dtype == HBT_DTYPE_F64 && dst_dtype == HBT_DTYPE_F64 && op == HBT_COPY_OP_COPY) {
+        src_dtype = dst_dtype = HBT_DTYPE_F32;  // an 8-byte element moves as two dwords
+        scale = 2;
     }
-    if (op == HBT_COPY_OP_COPY && src_dtype == dst_dtype) {
-        // Bit copy; fp64 moves as pairs of dwords (the host doubles its numels).
-        if (ssz == 2) return launch_copy<2, 2, HBT_COPY_OP_COPY>(table, count, total_chunks, divisor, aligned, hints, s);
-        if (ssz == 4) return launch_copy<4, 4, HBT_COPY_OP_COPY>(table, count, total_chunks, divisor, aligned, hints, s);
-        set_error("hbt_copy_intervals: 8-byte elements must be passed as dword pairs (F32)");
-        return HBT_ERR_UNSUPPORTED;
-    }
-    const bool wide = ssz == 8 || dsz == 8;
-    const bool mixed_16 = (src_dtype == HBT_DTYPE_BF16 && dst_dtype == HBT_DTYPE_F16) ||
-                          (src_dtype == HBT_DTYPE_F16 && dst_dtype == HBT_DTYPE_BF16);
-    if (wide || mixed_16) {
-        if (op != HBT_COPY_OP_COPY) {
-            set_error("hbt_copy_intervals: division moves data within one dtype (F64, F32, BF16 or F16) or "
-                      "between F32 and a 2-byte dtype (got %d -> %d)", src_dtype, dst_dtype);
-            return HBT_ERR_UNSUPPORTED;
+    const int64_t chunk = hbt_copy_chunk_elems(src_dtype, dst_dtype);
+    const uint64_t ssz = static_cast<uint64_t>(dtype_size(src_dtype)), dsz = static_cast<uint64_t>(dtype_size(dst_dtype));
+    const uint64_t src_align = 16 * ssz / (ssz > dsz ? ssz : dsz);
+    RowTable tab{};
+    int64_t chunks = 0;
+    bool aligned = true;
+    for (int32_t i = 0; i < count; ++i) {
+        const int64_t src = rows[3 * i], dst = rows[3 * i + 1], n = rows[3 * i + 2];
+        if (n < 0 || (n > 0 && dst == 0)) {
+            set_error("hbt_copy_rows: row %d has a null destination or a negative count", i);
+            return HBT_ERR_INVALID_ARGUMENT;
         }
-        return launch_convert<HBT_COPY_OP_COPY>(src_dtype, dst_dtype, table, count, total_chunks, 1.0, aligned,
-                                                hints, s);
+        if (n == 0) continue;  // the search wants strictly increasing first chunks
+        aligned = aligned && static_cast<uint64_t>(dst) % 16 == 0 && static_cast<uint64_t>(src) % src_align == 0;
+        tab.rec[tab.count++] = Record{src, dst, n * scale, chunks};
+        chunks += (n * scale + chunk - 1) / chunk;
     }
-    if (src_dtype == HBT_DTYPE_F16 || dst_dtype == HBT_DTYPE_F16) {
-        return launch_arith<true>(ssz, dsz, op, divisor, table, count, total_chunks, aligned, hints, s);
+    if (chunks == 0) return HBT_OK;
+    while (((chunks - 1) >> tab.shift) >= kRowHints) ++tab.shift;
+    int r = 0;
+    for (int64_t j = 0; j <= (chunks - 1) >> tab.shift; ++j) {
+        while (r + 1 < tab.count && tab.rec[r + 1].first <= (j << tab.shift)) ++r;
+        const bool split = r + 1 < tab.count && tab.rec[r + 1].first < ((j + 1) << tab.shift);
+        tab.hint[j >> 2] |= (static_cast<uint32_t>(r) | (split ? kHintSplit : 0u)) << (8 * (j & 3));
     }
-    return launch_arith<false>(ssz, dsz, op, divisor, table, count, total_chunks, aligned, hints, s);
+    return launch_plan(Plan{"hbt_copy_rows", nullptr, tab.count, nullptr, &tab, chunks, aligned, as_stream(stream)},
+                       src_dtype, dst_dtype, op, divisor);
 }
 
 }  // extern "C"

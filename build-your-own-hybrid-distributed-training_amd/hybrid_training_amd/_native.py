@@ -21,6 +21,7 @@ import threading
 from collections import OrderedDict
 from collections.abc import Iterable, Sequence
 from contextvars import ContextVar
+from itertools import chain
 from typing import Any
 
 import torch
@@ -83,6 +84,8 @@ COPY_ALIGNED = 1
 COPY_HINTS = 2
 #: Chunks per entry of a copy plan's hint table (HBT_COPY_HINTS).
 COPY_HINT_STRIDE = 256
+#: Rows of a plan whose table travels in the launch's arguments (hbt_copy_rows).
+COPY_MAX_ROWS = 112
 ACCUMULATE_ASSIGN = 1
 _CODE_BYTES = {DTYPE_F32: 4, DTYPE_BF16: 2, DTYPE_F16: 2, DTYPE_F64: 8}
 
@@ -159,6 +162,7 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
         _c_i32,
         (_c_void_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p),
     ),
+    "hbt_copy_rows": (_c_i32, (_i64_array, _c_i32, _c_i32, _c_i32, _c_i32, _c_f32, _c_void_p)),
     "hbt_grad_local_share": (
         _c_i32,
         (_ptr_array, _c_i32, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p, _c_void_p),
@@ -270,7 +274,7 @@ _LIB: ctypes.CDLL | None = None
 # function of its rows (addresses, lengths, chunk prefix), so an entry stays valid
 # even after the tensors it was built for are freed; reuse skips the host-to-device
 # upload, which for a few hundred rows costs more than moving a GB on the device.
-_TABLE_CACHE: "OrderedDict[tuple, tuple[torch.Tensor, int, bool, bool]]" = OrderedDict()
+_TABLE_CACHE: "OrderedDict[tuple, tuple[torch.Tensor, int, bool]]" = OrderedDict()
 _TABLE_CACHE_SIZE = 256
 
 
@@ -612,9 +616,10 @@ def plan_is_aligned(rows: Sequence[tuple[int, int, int]], src_code: int, dst_cod
 
 def _prepared_plan(
     device: torch.device, rows: tuple[tuple[int, int, int], ...], src_code: int, dst_code: int, scale: int
-) -> tuple[torch.Tensor, int, bool, bool]:
-    """(device table, total chunks, aligned, hinted) for a plan, built once per distinct plan
-    and stream.  The table is uploaded on that stream, so later launches on it see it."""
+) -> tuple[torch.Tensor, int, bool]:
+    """(device table with its hints, total chunks, aligned) for a plan longer than one launch's
+    arguments hold, built once per distinct plan and stream.  The table is uploaded on that
+    stream, so later launches on it see it."""
     recording = graph_recording()
     stream = stream_of(device)
     key = (device, stream, src_code, dst_code, scale, rows)
@@ -627,10 +632,7 @@ def _prepared_plan(
     chunk = _copy_chunk(library(), src_code, dst_code)
     flat, first = plan_table(rows, chunk, scale)
     aligned = plan_is_aligned(rows, src_code, dst_code)
-    # Plans of several records carry the hint table after their records.
-    hinted = len(rows) > 1
-    if hinted:
-        flat = flat + plan_hints(flat[3::4], first)
+    flat = flat + plan_hints(flat[3::4], first)  # HBT_COPY_HINTS
     if recording is not None:
         # Inside a graph recording the table is written by launches that carry it in
         # their arguments, so every replay rewrites it from the recorded words; the
@@ -641,11 +643,11 @@ def _prepared_plan(
             words.extend((value & 0xFFFFFFFF, (value >> 32) & 0xFFFFFFFF))
         write_words(device, table, words)
         recording.tables.append(table)
-        return table, first, aligned, hinted
+        return table, first, aligned
     host = torch.tensor(flat, dtype=torch.int64).pin_memory()
     with torch.cuda.device(device):
         table = host.to(device, non_blocking=True)
-    entry = (table, first, aligned, hinted)
+    entry = (table, first, aligned)
     with _TABLE_LOCK:
         _TABLE_CACHE[key] = entry
         if len(_TABLE_CACHE) > _TABLE_CACHE_SIZE:
@@ -755,13 +757,23 @@ class CopyPlan:
             return
         src_code = dtype_code(src_dtype)
         dst_code = dtype_code(dst_dtype)
+        lib = library()
+        if len(self._rows) <= COPY_MAX_ROWS:
+            # The table rides in the launch: nothing to build on the device or to keep.
+            graph_recording()  # a capture that a replay could not repeat correctly is refused
+            flat = (ctypes.c_int64 * (3 * len(self._rows)))(*chain.from_iterable(self._rows))
+            with device_guard(self.device):
+                status = lib.hbt_copy_rows(flat, len(self._rows), src_code, dst_code, op, float(divisor),
+                                           stream_of(self.device))
+            check(status, "native.hbt_copy_rows")
+            bump_versions(self._dests.values())
+            return
         scale = 1
         if src_dtype == dst_dtype and op == COPY_OP_COPY and src_code == DTYPE_F64:
             # An 8-byte element moves as two dwords.
             src_code = dst_code = DTYPE_F32
             scale = 2
-        lib = library()
-        table, first, aligned, hinted = _prepared_plan(self.device, tuple(self._rows), src_code, dst_code, scale)
+        table, first, aligned = _prepared_plan(self.device, tuple(self._rows), src_code, dst_code, scale)
         with device_guard(self.device):
             status = lib.hbt_copy_intervals(
                 table.data_ptr(),
@@ -771,7 +783,7 @@ class CopyPlan:
                 dst_code,
                 op,
                 float(divisor),
-                (COPY_ALIGNED if aligned else 0) | (COPY_HINTS if hinted else 0),
+                (COPY_ALIGNED if aligned else 0) | COPY_HINTS,
                 stream_of(self.device),
             )
         check(status, "native.hbt_copy_intervals")

@@ -496,21 +496,25 @@ class FlatParamHandle:
 
     def full_tensors(self, peer_shards: Sequence[torch.Tensor] | None = None) -> dict[str, torch.Tensor]:
         """Every managed parameter, reconstructed by copy (``fsdp.py:912-925``)."""
-        shards = [self._on_device(s) for s in self._all_shards(peer_shards, "fsdp.full_tensors")]
-        dtype = shards[0].dtype
+        shards = [_native.contiguous_source(self._on_device(s))
+                  for s in self._all_shards(peer_shards, "fsdp.full_tensors")]
+        dtype, length = shards[0].dtype, self._shard_numel
+        for shard in shards:
+            _native.require_device_tensor(shard, "fsdp.full_tensors")
         out = {e.name: torch.empty(e.shape, dtype=dtype, device=self._device) for e in self._entries}
-        plan = _native.CopyPlan(self._device)
+        size = dtype.itemsize
+        bases = [shard.data_ptr() for shard in shards]
+        rows = []  # (source address, destination address, n): the shards each parameter crosses
         for entry in self._entries:
-            dest = out[entry.name].view(-1)
-            for rank, shard in enumerate(shards):
-                piece = intersect_ranges(
-                    ShardRange(rank * self._shard_numel, self._shard_numel),
-                    ShardRange(entry.offset, entry.numel),
-                )
-                if piece is not None:
-                    plan.add(_native.contiguous_source(shard.detach()), piece.start - rank * self._shard_numel,
-                             dest, piece.start - entry.offset, piece.length)
-        plan.run(src_dtype=dtype, dst_dtype=dtype)
+            dest, start, end = out[entry.name].data_ptr(), entry.offset, entry.offset + entry.numel
+            cursor = start
+            while cursor < end:
+                rank = cursor // length
+                stop = min(end, (rank + 1) * length)
+                rows.append((bases[rank] + (cursor - rank * length) * size, dest + (cursor - start) * size, stop - cursor))
+                cursor = stop
+        _native.CopyPlan.from_rows(self._device, rows).run(src_dtype=dtype, dst_dtype=dtype)
+        _native.bump_versions(out.values())
         return out
 
     # -- gradient ---------------------------------------------------------------------

@@ -286,6 +286,23 @@ int32_t hbt_copy_intervals(const int64_t* table, int64_t count, int64_t total_ch
                            int32_t flags, void* stream);
 
 /* ------------------------------------------------------------------------------
+ * The interval gather-copy of a short plan, given as host rows.
+ *
+ * Replaces: what hbt_copy_intervals replaces, for plans of at most HBT_COPY_MAX_ROWS
+ *   intervals, such as FlatParamHandle.full_tensors (parallel/fsdp.py:912-925) and
+ *   read_tensor_range (checkpoint/reshard.py:200-305).
+ * `rows` is a HOST array of `count` rows of 3 int64 each:
+ *   { src_address (0 => write zeros), dst_address, numel }
+ * numel in elements of src_dtype (also for a same-dtype F64 COPY); rows of no elements are
+ * skipped.  The table is built here and travels in the launch's arguments, so no device
+ * table is read and a recorded launch repeats the same copy.  Element semantics, bits and
+ * limits are hbt_copy_intervals'.
+ * ---------------------------------------------------------------------------- */
+#define HBT_COPY_MAX_ROWS 112
+int32_t hbt_copy_rows(const int64_t* rows, int32_t count, int32_t src_dtype, int32_t dst_dtype, int32_t op,
+                      float divisor, void* stream);
+
+/* ------------------------------------------------------------------------------
  * FSDP gradient local share on one device.
  *
  * Replaces: FlatParamHandle.reduce_scatter_gradient (parallel/fsdp.py:704-769) with

@@ -392,3 +392,53 @@ def test_records_cut_on_destination_lines(device, sdt, ddt, op, around):
         plan.add(src, s0, dst, d0, n)
     plan.run(src_dtype=sdt, dst_dtype=ddt, op=op, divisor=3.0)
     assert np.array_equal(_bits(dst), expected)
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 111, 112, 113])
+@pytest.mark.parametrize("spread", [1, 400, 60_000])
+@pytest.mark.parametrize(("sdt", "ddt"), [(torch.float32, torch.float32), (torch.bfloat16, torch.float32),
+                                          (torch.float64, torch.float64), (torch.float16, torch.bfloat16)])
+def test_plans_around_one_launchs_rows(device, count, spread, sdt, ddt):
+    """Plans up to and past the rows a launch's arguments hold, from fewer chunks than hints
+    to hundreds of chunks per hint, rows of no elements, one element and several chunks
+    next to each other, zero fills among them: bitwise the intervals copied one by one."""
+    rng = np.random.default_rng(count * 31 + spread)
+    sizes = [int(n) for n in rng.integers(1, spread + 1, size=count)]
+    sizes[count // 2] = max(1, 20 * spread)
+    sizes[-1] = 1
+    n_src = max(sizes) + 13
+    src = (torch.randn(n_src, dtype=torch.float32, device=device) * 3).to(sdt)
+    gaps = [int(g) for g in rng.integers(0, 5, size=count)]
+    dst = torch.randn(sum(sizes) + sum(gaps) + 5, dtype=torch.float32, device=device).to(ddt)
+    expected = dst.cpu()
+    source = src.cpu().to(ddt)
+    plan, cursor = _native.CopyPlan(device), 0
+    for k, (n, gap) in enumerate(zip(sizes, gaps)):
+        cursor += gap
+        s0 = int(rng.integers(0, n_src - n + 1))
+        if sdt == ddt and k % 17 == 5:
+            plan.add_zero(dst, cursor, n)
+            expected[cursor : cursor + n] = 0
+        else:
+            plan.add(src, s0, dst, cursor, n)
+            expected[cursor : cursor + n] = source[s0 : s0 + n]
+        cursor += n
+    plan.run(src_dtype=sdt, dst_dtype=ddt)
+    assert np.array_equal(_bits(dst), _bits(expected))
+
+
+def test_copy_rows_refuses_what_it_cannot_move(device):
+    lib = _native.library()
+    buf = torch.zeros(8, device=device)
+    stream = _native.stream_of(device)
+    ok = (buf.data_ptr(), buf.data_ptr() + 16, 4)
+
+    def status(rows, count=None, src=0, dst=0, op=0):
+        return lib.hbt_copy_rows(_native.int64_array([v for r in rows for v in r]), len(rows) if count is None else count,
+                                 src, dst, op, 2.0, stream)
+
+    assert status([ok]) == 0 and status([(0, 0, 0)] * 3) == 0 and status([], 0) == 0
+    assert status([ok], count=_native.COPY_MAX_ROWS + 1) == -1
+    assert status([(buf.data_ptr(), 0, 4)]) == -1 and status([(ok[0], ok[1], -1)]) == -1
+    assert status([ok], src=9) == -1 and status([ok], op=7) == -1
+    assert status([ok], src=3, dst=0, op=1) == -2
