@@ -117,6 +117,38 @@ __device__ __forceinline__ void store_one(void* base, int64_t e, float x) {
     }
 }
 
+// The K elements from element e that lie below n, the others 0, and their store: a lane whose
+// vector is whole takes one vector access, and only the lane that holds the ragged end steps
+// by elements, so the tile a tensor ends in costs about one memory round trip; element by
+// element it takes one for every 32 or 64 of its elements, each waited for, at the very end
+// of the launch.  The update kernels keep the element loop there: four updates inlined for
+// the last tile cost more instruction fetch than the round trips they saved (a 929-element
+// AdamW step 4.6 us with the loop, 6.3 us so).
+template <int D, int K>
+__device__ __forceinline__ void load_upto(const void* base, int64_t e, int64_t n, float (&x)[K]) {
+#pragma unroll
+    for (int c = 0; c < K; ++c) x[c] = 0.0f;
+    if (e + K <= n) {
+        load_vec<D, K>(base, e, x);
+    } else {
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            if (e + c < n) x[c] = load_one<D>(base, e + c);
+        }
+    }
+}
+template <int D, int K>
+__device__ __forceinline__ void store_upto(void* base, int64_t e, int64_t n, const float (&x)[K]) {
+    if (e + K <= n) {
+        store_vec<D, K>(base, e, x);
+    } else {
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            if (e + c < n) store_one<D>(base, e + c, x[c]);
+        }
+    }
+}
+
 // K consecutive doubles from element e (K even, e a multiple of 2, base 16-byte aligned):
 // K / 2 non-temporal 16-byte loads.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
@@ -499,11 +531,12 @@ __device__ __forceinline__ double add_sq(double acc, float x) {
 
 
 // A lane's eight elements of a piece from element e0 (its first), squared after the
-// unscale: vector loads when the whole lane vector lies inside and is aligned.
+// unscale: one vector load when the whole piece lies inside (`whole`, the same for every
+// lane of the wave).
 template <int GD, bool kUnscale>
-__device__ __forceinline__ double lane_sq_b16(const void* G, int64_t e0, int64_t n, bool vec, float unscale) {
+__device__ __forceinline__ double lane_sq_b16(const void* G, int64_t e0, int64_t n, bool whole, float unscale) {
     double acc = 0.0;
-    if (vec) {
+    if (whole) {
         float x[8];
         load_vec<GD, 8>(G, e0, x);
 #pragma unroll
@@ -564,9 +597,10 @@ __device__ __forceinline__ void sqnorm_b16_chunk(const NormTable& tab, float uns
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-            a[k] = lane_sq_b16<GD, kUnscale>(G, start + int64_t(k * 16 + w) * kPieceB16 + int64_t(lane) * 8, n, false,
-                                             unscale);
+        for (int k = 0; k < 8; ++k) {
+            const int64_t piece = start + int64_t(k * 16 + w) * kPieceB16;
+            a[k] = lane_sq_b16<GD, kUnscale>(G, piece + int64_t(lane) * 8, n, piece + kPieceB16 <= n, unscale);
+        }
     }
     const double d = piece_sums8(a, lane);
     if ((lane & 7) == 0) piece_sums[(lane >> 3) * 16 + w] = d;
@@ -644,13 +678,17 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
                 }
                 if constexpr (kStore) store_vec<GD, K>(const_cast<void*>(G), base + int64_t(threadIdx.x) * K, x);
             } else {
-                const int64_t end = base + kTile < n ? base + kTile : n;
-                for (int64_t e = base + threadIdx.x; e < end; e += kNormBlock) {
-                    float y = load_one<GD>(G, e);
+                const int64_t e = base + int64_t(threadIdx.x) * K;
+                float x[K];
+                load_upto<GD, K>(G, e, n, x);
+    #pragma unroll
+                for (int c = 0; c < K; ++c) {
+                    float y = x[c];
                     if constexpr (kUnscale) y = round_to<GD>(y * unscale);
-                    if constexpr (kStore) store_one<GD>(const_cast<void*>(G), e, y);
-                    acc += sq(y);
+                    if constexpr (kStore) x[c] = y;
+                    if (e + c < n) acc += sq(y);
                 }
+                if constexpr (kStore) store_upto<GD, K>(const_cast<void*>(G), e, n, x);
             }
         }
         const double block_total = block_sum<kNormBlock>(acc);
@@ -707,6 +745,11 @@ __device__ __forceinline__ float share_cast(float x) {
 // is issued, which beat all eight in flight at once, waiting after each load, and
 // waiting after four.  tile_sums may be null (the local share alone).
 constexpr int kShareIssue = 2;
+// A launch whose waves all fit the chip at once (256 CUs x 32 waves, one tile each) issues
+// every rank's loads together: it is bound by one wave's round trips, not by the stream.
+// 8 bf16 ranks with the partials, pairs and all together: 781 tiles 9.0 and 8.0 us, 7,812
+// tiles 11.4 and 10.8; past that the stream decides (106,500 tiles 88.9 and 89.6).
+constexpr int64_t kShareBurstTiles = 8192;
 // With the accumulator rows (kAcc) each rank is two loads, its gradient and its row;
 // waiting after every rank's pair streamed fastest (against every two, four or eight
 // ranks, or all gradients before the rows).
@@ -813,13 +856,20 @@ __device__ __forceinline__ float share_input(float g, float a) {
 template <int ID, int kG, bool kRecip, int RD, int OD, bool kAcc>
 __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const ShareAcc& accs, int32_t group_size,
                                              int64_t offset, int64_t shard_numel, int64_t valid_numel, float divisor,
-                                             float recip, void* __restrict__ out, int64_t tile,
+                                             float recip, int32_t burst, void* __restrict__ out, int64_t tile,
                                              int lane) {
     constexpr int64_t IB = bytes_of<ID>();
     const int64_t base = tile * kShareTile;
     double acc = 0.0;
-    if (base + kShareTile <= valid_numel) {
-        const int64_t e = base + int64_t(lane) * 4;
+    if (base < valid_numel && valid_numel >= kShareTile) {
+        // The tile the real elements end in reads and sums the whole tile that ends there and
+        // keeps what lies past the tile before it.  Stepped element by element it took a memory round trip per
+        // rank for every 64 elements, at the very end of the launch: 8 ranks into a shard of
+        // 885,984 bf16 elements (3460 tiles and 224 elements) in 11.0 us so and in 5.3 us
+        // so.
+        const bool whole = base + kShareTile <= valid_numel;
+        const int counted = whole ? 0 : static_cast<int>(base + kShareTile - valid_numel);
+        const int64_t e = (whole ? base : valid_numel - kShareTile) + int64_t(lane) * 4;
         float sum[4];
         if constexpr (kG > 0) {
             float x[kG][4];
@@ -828,7 +878,7 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
             for (int q = 0; q < kG; ++q) {
                 load_vec<ID, 4>(ranks.g[q] + offset * IB, e, x[q]);
                 if constexpr (kAcc) load_vec<RD, 4>(accs.a[q], e, a[q]);
-                if ((q + 1) % (kAcc ? kShareAccIssue : kShareIssue) == 0 && q + 1 < kG) wait_vmem();
+                if ((q + 1) % (kAcc ? kShareAccIssue : kShareIssue) == 0 && q + 1 < kG && !burst) wait_vmem();
             }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -871,13 +921,25 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) sum[c] = round_to<OD>(sum[c]);
-        store_vec<OD, 4>(out, e, sum);
+        if (whole) {
+            store_vec<OD, 4>(out, e, sum);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc += sq(sum[c]);
+            for (int c = 0; c < 4; ++c) acc += sq(sum[c]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (lane * 4 + c < counted) continue;
+                store_one<OD>(out, e + c, sum[c]);
+                acc += sq(sum[c]);
+            }
+            const int64_t end = base + kShareTile < shard_numel ? base + kShareTile : shard_numel;
+            for (int64_t z = valid_numel + lane; z < end; z += kShareBlock) store_one<OD>(out, z, 0.0f);
+        }
     } else if (base >= valid_numel && base + kShareTile <= shard_numel) {
         const float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         store_vec<OD, 4>(out, base + int64_t(lane) * 4, zero);
     } else {
+        // A shard shorter than a tile, or a tile of padding that the shard ends in.
         const int64_t end = base + kShareTile < shard_numel ? base + kShareTile : shard_numel;
         for (int64_t e = base + lane; e < end; e += kShareBlock) {
             float v = 0.0f;
@@ -902,11 +964,11 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
 template <int ID, int kG, bool kRecip, int RD, int OD, bool kAcc = false>
 __global__ __launch_bounds__(kShareBlock) void local_share_tiles_kernel(
     ShareRanks ranks, ShareAcc accs, int32_t group_size, int64_t offset, int64_t shard_numel, int64_t valid_numel,
-    float divisor, float recip, void* __restrict__ out, double* __restrict__ tile_sums,
+    float divisor, float recip, int32_t burst, void* __restrict__ out, double* __restrict__ tile_sums,
     int64_t block_base) {
     const int64_t tile = block_base + blockIdx.x;
     double acc = share_tile<ID, kG, kRecip, RD, OD, kAcc>(ranks, accs, group_size, offset, shard_numel, valid_numel,
-                                                          divisor, recip, out, tile,
+                                                          divisor, recip, burst, out, tile,
                                                           static_cast<int>(threadIdx.x));
     if (tile_sums == nullptr) return;
     acc = wave_sum(acc);
@@ -933,7 +995,7 @@ __global__ __launch_bounds__(kSmallShareTiles * kShareBlock) void local_share_sm
     const int lane = static_cast<int>(threadIdx.x) % kShareBlock;
     const ShareAcc none{};
     const double s = wave_sum(share_tile<ID, kG, kRecip, RD, OD, false>(
-        ranks, none, group_size, offset, shard_numel, valid_numel, divisor, recip, out, wave, lane));
+        ranks, none, group_size, offset, shard_numel, valid_numel, divisor, recip, 1, out, wave, lane));
     if (lane == 0) sums[wave] = s;
     __syncthreads();
     if (wave != 0) return;
@@ -1261,8 +1323,16 @@ __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale
         }
         return;
     }
-    const int64_t end = base + kTile < n ? base + kTile : n;
-    for (int64_t i = base + threadIdx.x; i < end; i += kScaleBlock) store_one<D>(X, i, scale_one<D>(load_one<D>(X, i), unscale, mul));
+    float v[scale_unroll<D>()][K];
+#pragma unroll
+    for (int u = 0; u < scale_unroll<D>(); ++u)
+        load_upto<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
+#pragma unroll
+    for (int u = 0; u < scale_unroll<D>(); ++u) {
+#pragma unroll
+        for (int c = 0; c < K; ++c) v[u][c] = scale_one<D>(v[u][c], unscale, mul);
+        store_upto<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
+    }
 }
 
 // ---- float64 parameters ---------------------------------------------------------------
@@ -1594,10 +1664,21 @@ __global__ __launch_bounds__(kAccumBlock) void accumulate_kernel(AccumTable tab,
         }
         return;
     }
-    const int64_t end = base + kAccumTile < n ? base + kAccumTile : n;
-    for (int64_t i = base + threadIdx.x; i < end; i += kAccumBlock) {
-        const float g = share_cast<GD, AD>(load_one<GD>(grad, i));
-        store_one<AD>(acc, i, kAssign ? g : round_to<AD>(load_one<AD>(acc, i) + g));
+    float a[2][4], g[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int64_t e = base + (int64_t(u) * kAccumBlock + threadIdx.x) * 4;
+        load_upto<GD, 4>(grad, e, n, g[u]);
+        if constexpr (!kAssign) load_upto<AD, 4>(acc, e, n, a[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            g[u][c] = share_cast<GD, AD>(g[u][c]);
+            if constexpr (!kAssign) g[u][c] = round_to<AD>(a[u][c] + g[u][c]);
+        }
+        store_upto<AD, 4>(acc, base + (int64_t(u) * kAccumBlock + threadIdx.x) * 4, n, g[u]);
     }
 }
 
@@ -1965,6 +2046,7 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
     const bool recip_exact = recip != 0.0f;
     // A small shard's share and partials take one launch (local_share_small_kernel).
     const bool small = partials != nullptr && !with_acc && !f64 && tiles <= kSmallShareTiles;
+    const int32_t burst = tiles <= kShareBurstTiles;
     const unsigned small_threads = static_cast<unsigned>(tiles) * kShareBlock;
     int32_t status = launch_sliced(who, tiles, kShareBlock, [&](int64_t first, dim3 grid) {
 #define HBT_TILES(ID, G, R, RD, OD)                                                                             \
@@ -1974,11 +2056,11 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
                 ranks, group_size, offset, shard_numel, valid_numel, divisor, recip, out, partials);    \
         else if (with_acc)                                                                                     \
             local_share_tiles_kernel<ID, G, R, RD, OD, true><<<grid, kShareBlock, 0, st>>>(                      \
-                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, out,          \
+                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
                 tile_scratch, first);                                                                          \
         else                                                                                                   \
             local_share_tiles_kernel<ID, G, R, RD, OD, false><<<grid, kShareBlock, 0, st>>>(                     \
-                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, out,          \
+                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
                 tile_scratch, first);                                                                          \
     } while (0)
 // Groups of 1 to 8 ranks have their own instantiations, every rank's load issued before

@@ -591,3 +591,33 @@ def test_steps_off_the_vectors_are_the_aligned_steps(device, n, dtypes, write_ba
         results.append([_bits(t) for t in views])
     for a, b in zip(*results):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("valid", [256, 257, 300, 511, 512, 767, 4097, 33_000])
+@pytest.mark.parametrize("pad", [0, 1, 200, 600])
+@pytest.mark.parametrize("group", [2, 8, 9])
+def test_local_share_tile_the_real_elements_end_in(device, valid, pad, group):
+    """The tile that the shard's real elements end in reads the whole tile ending there: the
+    elements it shares with the tile before it count once in the norm partials, and the
+    padding behind them is +0.0, up to tiles of padding alone."""
+    lib = _native.library()
+    shard = valid + pad
+    gen = torch.Generator(device=device).manual_seed(valid + pad + group)
+    grads = [torch.randn(group * shard, device=device, generator=gen).to(torch.bfloat16) for _ in range(group)]
+    host = [g.float().cpu().numpy() for g in grads]
+    rank = 1
+    out = torch.full((shard + 4,), 7.0, device=device)
+    count = -(-valid // 32768) + -(-pad // 32768)
+    partials = torch.full((count,), 5.0, dtype=torch.float64, device=device)
+    tile_sums = torch.empty(-(-shard // 256), dtype=torch.float64, device=device)
+    _native.check(lib.hbt_grad_local_share_sqnorm(
+        _native.pointer_array([g.data_ptr() for g in grads]), group, rank, shard, valid, 1, 0, float(group), 0,
+        out.data_ptr(), partials.data_ptr(), tile_sums.data_ptr(), _native.stream_of(device)), "test.share")
+    expect = oracle.local_share(host, rank, shard, valid, float(group))
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:shard].view(np.int32), expect.view(np.int32)) and np.all(got[shard:] == 7.0)
+    sums = partials.cpu().numpy()
+    for c in range(-(-valid // 32768)):
+        ref = math.fsum(float(x) * float(x) for x in expect[c * 32768 : min((c + 1) * 32768, valid)])
+        assert abs(sums[c] - ref) <= 1e-12 * ref, c
+    assert np.all(sums[-(-valid // 32768) :] == 0.0)
