@@ -55,31 +55,36 @@ __device__ __forceinline__ u32x4 pack8_rounded(const float (&y)[8]) {
 }
 
 // ---- vector memory helpers ----------------------------------------------------------
-// Every operand is touched exactly once per step, so loads and stores are marked
-// non-temporal: the lines are not kept in L2/MALL for reuse that never comes.
+// An operand that is touched once per step is loaded and stored non-temporally: its lines
+// are not kept in the L2 and the 256 MB memory-side cache (MALL) for reuse that never comes.
+// kKeep marks the accesses of a gradient that the step's next pass reads again (the norm,
+// then the clip, then the update) and that fits there: they are ordinary ones.
 //
 // K consecutive elements of dtype D starting at element e of `base`, widened exactly to
 // fp32, with one vector load of K * bytes(D) bytes (16 for 4 fp32 or 8 bf16/fp16, 8 for
 // 4 bf16/fp16).
-template <int D, int K>
+template <int D, int K, bool kKeep = false>
 __device__ __forceinline__ void load_vec(const void* base, int64_t e, float (&x)[K]) {
     static_assert(D == F32 || D == BF16 || D == F16, "vector loads move fp32, bf16 and fp16");
     if constexpr (D == F32) {
         static_assert(K == 4, "fp32 vectors are four elements");
-        const f32x4 w = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(static_cast<const float*>(base) + e));
+        const f32x4_any* p = reinterpret_cast<const f32x4_any*>(static_cast<const float*>(base) + e);
+        const f32x4 w = kKeep ? *p : __builtin_nontemporal_load(p);
         x[0] = w.x;
         x[1] = w.y;
         x[2] = w.z;
         x[3] = w.w;
     } else if constexpr (K == 4) {
-        const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2_any*>(static_cast<const uint16_t*>(base) + e));
+        const u32x2_any* p = reinterpret_cast<const u32x2_any*>(static_cast<const uint16_t*>(base) + e);
+        const u32x2 w = kKeep ? *p : __builtin_nontemporal_load(p);
         x[0] = b16_to_f32<D == F16>(w.x & 0xFFFFu);
         x[1] = b16_to_f32<D == F16>(w.x >> 16);
         x[2] = b16_to_f32<D == F16>(w.y & 0xFFFFu);
         x[3] = b16_to_f32<D == F16>(w.y >> 16);
     } else {
         static_assert(K == 8, "2-byte vectors are four or eight elements");
-        const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(static_cast<const uint16_t*>(base) + e));
+        const u32x4_any* p = reinterpret_cast<const u32x4_any*>(static_cast<const uint16_t*>(base) + e);
+        const u32x4 w = kKeep ? *p : __builtin_nontemporal_load(p);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             x[2 * i] = b16_to_f32<D == F16>(w[i] & 0xFFFFu);
@@ -88,19 +93,25 @@ __device__ __forceinline__ void load_vec(const void* base, int64_t e, float (&x)
     }
 }
 // Stores K values, each already representable in D (so the narrowing is exact).
-template <int D, int K>
+template <int D, int K, bool kKeep = false>
 __device__ __forceinline__ void store_vec(void* base, int64_t e, const float (&x)[K]) {
     static_assert(D == F32 || D == BF16 || D == F16, "vector stores move fp32, bf16 and fp16");
     if constexpr (D == F32) {
         static_assert(K == 4, "fp32 vectors are four elements");
-        __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<f32x4_any*>(static_cast<float*>(base) + e));
+        f32x4_any* p = reinterpret_cast<f32x4_any*>(static_cast<float*>(base) + e);
+        if constexpr (kKeep) *p = f32x4{x[0], x[1], x[2], x[3]};
+        else __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, p);
     } else if constexpr (K == 4) {
         uint32_t w[2];
         pack_rounded<D, 2>(x, w);
-        __builtin_nontemporal_store(u32x2{w[0], w[1]}, reinterpret_cast<u32x2_any*>(static_cast<uint16_t*>(base) + e));
+        u32x2_any* p = reinterpret_cast<u32x2_any*>(static_cast<uint16_t*>(base) + e);
+        if constexpr (kKeep) *p = u32x2{w[0], w[1]};
+        else __builtin_nontemporal_store(u32x2{w[0], w[1]}, p);
     } else {
         static_assert(K == 8, "2-byte vectors are four or eight elements");
-        __builtin_nontemporal_store(pack8_rounded<D>(x), reinterpret_cast<u32x4_any*>(static_cast<uint16_t*>(base) + e));
+        u32x4_any* p = reinterpret_cast<u32x4_any*>(static_cast<uint16_t*>(base) + e);
+        if constexpr (kKeep) *p = pack8_rounded<D>(x);
+        else __builtin_nontemporal_store(pack8_rounded<D>(x), p);
     }
 }
 template <int D>
@@ -124,12 +135,12 @@ __device__ __forceinline__ void store_one(void* base, int64_t e, float x) {
 // of the launch.  The update kernels keep the element loop there: four updates inlined for
 // the last tile cost more instruction fetch than the round trips they saved (a 929-element
 // AdamW step 4.6 us with the loop, 6.3 us so).
-template <int D, int K>
+template <int D, int K, bool kKeep = false>
 __device__ __forceinline__ void load_upto(const void* base, int64_t e, int64_t n, float (&x)[K]) {
 #pragma unroll
     for (int c = 0; c < K; ++c) x[c] = 0.0f;
     if (e + K <= n) {
-        load_vec<D, K>(base, e, x);
+        load_vec<D, K, kKeep>(base, e, x);
     } else {
 #pragma unroll
         for (int c = 0; c < K; ++c) {
@@ -137,10 +148,10 @@ __device__ __forceinline__ void load_upto(const void* base, int64_t e, int64_t n
         }
     }
 }
-template <int D, int K>
+template <int D, int K, bool kKeep = false>
 __device__ __forceinline__ void store_upto(void* base, int64_t e, int64_t n, const float (&x)[K]) {
     if (e + K <= n) {
-        store_vec<D, K>(base, e, x);
+        store_vec<D, K, kKeep>(base, e, x);
     } else {
 #pragma unroll
         for (int c = 0; c < K; ++c) {
@@ -533,12 +544,12 @@ __device__ __forceinline__ double add_sq(double acc, float x) {
 // A lane's eight elements of a piece from element e0 (its first), squared after the
 // unscale: one vector load when the whole piece lies inside (`whole`, the same for every
 // lane of the wave).
-template <int GD, bool kUnscale>
+template <int GD, bool kUnscale, bool kKeep>
 __device__ __forceinline__ double lane_sq_b16(const void* G, int64_t e0, int64_t n, bool whole, float unscale) {
     double acc = 0.0;
     if (whole) {
         float x[8];
-        load_vec<GD, 8>(G, e0, x);
+        load_vec<GD, 8, kKeep>(G, e0, x);
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc = add_sq(acc, kUnscale ? round_to<GD>(x[c] * unscale) : x[c]);
     } else {
@@ -570,7 +581,7 @@ __device__ __forceinline__ double piece_sums8(const double (&a)[8], int lane) {
 }
 
 // The plain pass for 2-byte gradients: chunk c's partial in the two-level order.
-template <int GD, bool kUnscale>
+template <int GD, bool kUnscale, bool kKeep>
 __device__ __forceinline__ void sqnorm_b16_chunk(const NormTable& tab, float unscale, double* __restrict__ partials,
                                                  int64_t chunk) {
     __shared__ double piece_sums[kPiecesPerChunk];
@@ -587,7 +598,7 @@ __device__ __forceinline__ void sqnorm_b16_chunk(const NormTable& tab, float uns
             float x[4][8];
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                load_vec<GD, 8>(G, start + int64_t((k0 + k) * 16 + w) * kPieceB16 + int64_t(lane) * 8, x[k]);
+                load_vec<GD, 8, kKeep>(G, start + int64_t((k0 + k) * 16 + w) * kPieceB16 + int64_t(lane) * 8, x[k]);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 a[k0 + k] = 0.0;
@@ -599,7 +610,7 @@ __device__ __forceinline__ void sqnorm_b16_chunk(const NormTable& tab, float uns
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int64_t piece = start + int64_t(k * 16 + w) * kPieceB16;
-            a[k] = lane_sq_b16<GD, kUnscale>(G, piece + int64_t(lane) * 8, n, piece + kPieceB16 <= n, unscale);
+            a[k] = lane_sq_b16<GD, kUnscale, kKeep>(G, piece + int64_t(lane) * 8, n, piece + kPieceB16 <= n, unscale);
         }
     }
     const double d = piece_sums8(a, lane);
@@ -619,13 +630,13 @@ __device__ __forceinline__ void sqnorm_b16_chunk(const NormTable& tab, float uns
 // kStore writes each unscaled value back in place as it is squared: the in-place unscale
 // and the norm of its result in one pass, with the partials of the norm pass over the
 // unscaled tensor (the same loads, the same order).
-template <int GD, bool kUnscale, bool kStore = false>
+template <int GD, bool kUnscale, bool kStore, bool kKeep>
 __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float unscale,
                                                             double* __restrict__ partials, int64_t block_base) {
     static_assert(!kStore || kUnscale, "a store without an unscale rewrites the same values");
     static_assert(!kStore || GD == F32, "2-byte gradients unscale in place through unscale_pieces_kernel");
     if constexpr (GD != F32) {
-        sqnorm_b16_chunk<GD, kUnscale>(tab, unscale, partials, block_base + blockIdx.x);
+        sqnorm_b16_chunk<GD, kUnscale, kKeep>(tab, unscale, partials, block_base + blockIdx.x);
     } else {
         constexpr int K = norm_vec<GD>();
         constexpr int64_t kTile = norm_tile<GD>();
@@ -644,7 +655,7 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
                 float x[kNormBatch][K];
     #pragma unroll
                 for (int k = 0; k < kNormBatch; ++k)
-                    load_vec<GD, K>(G, start + int64_t(k0 + k) * kTile + int64_t(threadIdx.x) * K, x[k]);
+                    load_vec<GD, K, kKeep>(G, start + int64_t(k0 + k) * kTile + int64_t(threadIdx.x) * K, x[k]);
     #pragma unroll
                 for (int k = 0; k < kNormBatch; ++k) {
     #pragma unroll
@@ -655,7 +666,7 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
                         acc += sq(y);
                     }
                     if constexpr (kStore)
-                        store_vec<GD, K>(const_cast<void*>(G), start + int64_t(k0 + k) * kTile + int64_t(threadIdx.x) * K,
+                        store_vec<GD, K, kKeep>(const_cast<void*>(G), start + int64_t(k0 + k) * kTile + int64_t(threadIdx.x) * K,
                                          x[k]);
                 }
             }
@@ -668,7 +679,7 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
             if (base >= n) break;
             if (base + kTile <= n) {
                 float x[K];
-                load_vec<GD, K>(G, base + int64_t(threadIdx.x) * K, x);
+                load_vec<GD, K, kKeep>(G, base + int64_t(threadIdx.x) * K, x);
     #pragma unroll
                 for (int c = 0; c < K; ++c) {
                     float y = x[c];
@@ -676,11 +687,11 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
                     if constexpr (kStore) x[c] = y;
                     acc += sq(y);
                 }
-                if constexpr (kStore) store_vec<GD, K>(const_cast<void*>(G), base + int64_t(threadIdx.x) * K, x);
+                if constexpr (kStore) store_vec<GD, K, kKeep>(const_cast<void*>(G), base + int64_t(threadIdx.x) * K, x);
             } else {
                 const int64_t e = base + int64_t(threadIdx.x) * K;
                 float x[K];
-                load_upto<GD, K>(G, e, n, x);
+                load_upto<GD, K, kKeep>(G, e, n, x);
     #pragma unroll
                 for (int c = 0; c < K; ++c) {
                     float y = x[c];
@@ -688,7 +699,7 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_kernel(NormTable tab, float
                     if constexpr (kStore) x[c] = y;
                     if (e + c < n) acc += sq(y);
                 }
-                if constexpr (kStore) store_upto<GD, K>(const_cast<void*>(G), e, n, x);
+                if constexpr (kStore) store_upto<GD, K, kKeep>(const_cast<void*>(G), e, n, x);
             }
         }
         const double block_total = block_sum<kNormBlock>(acc);
@@ -1275,7 +1286,7 @@ __device__ __forceinline__ float scale_one(float x, float unscale, float mul) {
     return round_to<D>(round_to<D>(x * unscale) * mul);
 }
 
-template <int D>
+template <int D, bool kKeep>
 __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale,
                                                             const float* __restrict__ grad_mul, int64_t block_base) {
     constexpr int K = scale_vec<D>();
@@ -1295,16 +1306,16 @@ __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale
             constexpr int U = scale_unroll<D>();
             float v[U][K];
 #pragma unroll
-            for (int u = 0; u < U; ++u) load_vec<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, v[u]);
+            for (int u = 0; u < U; ++u) load_vec<D, K, kKeep>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, v[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
 #pragma unroll
                 for (int c = 0; c < K; ++c) v[u][c] = scale_one<D>(v[u][c], unscale, mul);
-                store_vec<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, v[u]);
+                store_vec<D, K, kKeep>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, v[u]);
             }
         } else {
             u32x4_any* P = reinterpret_cast<u32x4_any*>(static_cast<uint16_t*>(X) + base) + threadIdx.x;
-            const u32x4 w = __builtin_nontemporal_load(P);
+            const u32x4 w = kKeep ? *P : __builtin_nontemporal_load(P);
             float y[8];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1319,19 +1330,20 @@ __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale
             }
 #pragma unroll
             for (int c = 0; c < 8; ++c) y[c] = y[c] * mul;
-            __builtin_nontemporal_store(pack8_rounded<D>(y), P);
+            if constexpr (kKeep) *P = pack8_rounded<D>(y);
+            else __builtin_nontemporal_store(pack8_rounded<D>(y), P);
         }
         return;
     }
     float v[scale_unroll<D>()][K];
 #pragma unroll
     for (int u = 0; u < scale_unroll<D>(); ++u)
-        load_upto<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
+        load_upto<D, K, kKeep>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
 #pragma unroll
     for (int u = 0; u < scale_unroll<D>(); ++u) {
 #pragma unroll
         for (int c = 0; c < K; ++c) v[u][c] = scale_one<D>(v[u][c], unscale, mul);
-        store_upto<D, K>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
+        store_upto<D, K, kKeep>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
     }
 }
 
@@ -1741,6 +1753,18 @@ float host_round_to(float x, int32_t dtype) {
     return x;
 }
 
+// Whether a launch over these gradients leaves them in the memory-side cache for the pass
+// that follows it in a step (the clip after the norm, the update after either): they have to
+// fit its 256 MB, and below 32 MB the L2 serves the next pass either way.  Kept and not
+// kept, whole tails: norm, clip and AdamW of 54 M fp32 elements (a 2-layer GPT-2 under DDP)
+// 418 and 433 us, of 30 M 226 and 239; norm and AdamW without a clip in place of 30 M 151
+// and 159; past 256 MB keeping slows the norm by 6% and saves nothing.
+bool keep_for_next_pass(const int64_t* numels, int32_t count, int32_t dtype) {
+    int64_t bytes = 0;
+    for (int32_t i = 0; i < count; ++i) bytes += numels[i] * dtype_size(dtype);
+    return bytes >= (int64_t(32) << 20) && bytes <= (int64_t(256) << 20);
+}
+
 // The optimizer dtype pairs (parameter, gradient) with a kernel.
 bool optimizer_dtypes_ok(int32_t param_dtype, int32_t grad_dtype) {
     return (param_dtype == F32 && (grad_dtype == F32 || grad_dtype == BF16)) ||
@@ -1943,18 +1967,25 @@ int32_t launch_sqnorm(const char* who, const NormTable& tab, int64_t chunks, int
             sqnorm_f64_kernel<<<grid, kNormBlock, 0, st>>>(tab, partials, first);
         });
     }
+    const bool keep = keep_for_next_pass(tab.n, tab.count, grad_dtype);
     return launch_sliced(who, chunks, kNormBlock, [&](int64_t first, dim3 grid) {
+#define HBT_SQNORM(GD, SCALED, STORE)                                                                                  \
+    do {                                                                                                               \
+        if (keep) sqnorm_kernel<GD, SCALED, STORE, true><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);  \
+        else sqnorm_kernel<GD, SCALED, STORE, false><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);      \
+    } while (0)
         if (grad_dtype == F32) {
-            if (scaled && store) sqnorm_kernel<F32, true, true><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
-            else if (scaled) sqnorm_kernel<F32, true><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
-            else sqnorm_kernel<F32, false><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
+            if (scaled && store) HBT_SQNORM(F32, true, true);
+            else if (scaled) HBT_SQNORM(F32, true, false);
+            else HBT_SQNORM(F32, false, false);
         } else if (grad_dtype == BF16) {
-            if (scaled) sqnorm_kernel<BF16, true><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
-            else sqnorm_kernel<BF16, false><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
+            if (scaled) HBT_SQNORM(BF16, true, false);
+            else HBT_SQNORM(BF16, false, false);
         } else {
-            if (scaled) sqnorm_kernel<F16, true><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
-            else sqnorm_kernel<F16, false><<<grid, kNormBlock, 0, st>>>(tab, unscale, partials, first);
+            if (scaled) HBT_SQNORM(F16, true, false);
+            else HBT_SQNORM(F16, false, false);
         }
+#undef HBT_SQNORM
     });
 }
 
@@ -2423,10 +2454,17 @@ int32_t hbt_scale_inplace(void* const* tensors, const int64_t* numels, int32_t c
     for (int i = count + 1; i <= kMaxT; ++i) tab.first_block[i] = blocks;
     hipStream_t st = as_stream(stream);
     const int threads = dtype == F32 ? scale_block<F32>() : scale_block<BF16>();
+    const bool keep = keep_for_next_pass(tab.n, tab.count, dtype);
     return launch_sliced("hbt_scale_inplace", blocks, threads, [&](int64_t first, dim3 grid) {
-        if (dtype == F32) scale_kernel<F32><<<grid, threads, 0, st>>>(tab, unscale, grad_mul, first);
-        else if (dtype == BF16) scale_kernel<BF16><<<grid, threads, 0, st>>>(tab, unscale, grad_mul, first);
-        else scale_kernel<F16><<<grid, threads, 0, st>>>(tab, unscale, grad_mul, first);
+#define HBT_SCALE(D)                                                                                 \
+    do {                                                                                             \
+        if (keep) scale_kernel<D, true><<<grid, threads, 0, st>>>(tab, unscale, grad_mul, first);    \
+        else scale_kernel<D, false><<<grid, threads, 0, st>>>(tab, unscale, grad_mul, first);        \
+    } while (0)
+        if (dtype == F32) HBT_SCALE(F32);
+        else if (dtype == BF16) HBT_SCALE(BF16);
+        else HBT_SCALE(F16);
+#undef HBT_SCALE
     });
 }
 

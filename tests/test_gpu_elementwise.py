@@ -621,3 +621,26 @@ def test_local_share_tile_the_real_elements_end_in(device, valid, pad, group):
         ref = math.fsum(float(x) * float(x) for x in expect[c * 32768 : min((c + 1) * 32768, valid)])
         assert abs(sums[c] - ref) <= 1e-12 * ref, c
     assert np.all(sums[-(-valid // 32768) :] == 0.0)
+
+
+@pytest.mark.parametrize("n", [(8 << 20) - 1, 8 << 20, 64 << 20, (64 << 20) + 1])
+def test_norm_and_scale_at_the_sizes_kept_for_the_next_pass(device, n):
+    """Around 32 and 256 MB of gradients, where a launch starts and stops leaving them in the
+    memory-side cache for the next pass: the same values and partials on both sides."""
+    lib = _native.library()
+    x = torch.randn(n, device=device, generator=torch.Generator(device=device).manual_seed(n))
+    stream = _native.stream_of(device)
+    partials = torch.empty(-(-n // 32768), dtype=torch.float64, device=device)
+    _native.check(lib.hbt_grad_sqnorm_partials(_native.pointer_array([x.data_ptr()]), _native.int64_array([n]),
+                                               _native.double_array([1.0]), 1, 0, 1.0, partials.data_ptr(), stream),
+                  "test.norm")
+    squares = x.double().square_()
+    whole = n // 32768 * 32768
+    expect = torch.cat([squares[:whole].view(-1, 32768).sum(1), squares[whole:].sum().view(1)])[: partials.numel()]
+    assert torch.allclose(partials, expect, rtol=1e-12, atol=0.0)
+    del squares, expect
+    mul = torch.tensor([0.3], device=device)
+    scaled = x.clone()
+    _native.check(lib.hbt_scale_inplace(_native.pointer_array([scaled.data_ptr()]), _native.int64_array([n]), 1, 0, 1.0,
+                                        mul.data_ptr(), stream), "test.scale")
+    assert torch.equal(scaled, x * mul)
