@@ -681,6 +681,7 @@ class CopyPlan:
     def __init__(self, device: torch.device) -> None:
         self.device = torch.device(device)
         self._rows: list[tuple[int, int, int]] = []
+        self._flat: ctypes.Array | None = None  # the rows as the launch takes them, kept for a repeated run
         # The tensors the rows address, held for the plan's lifetime.  A row records
         # only addresses: a temporary the caller made for it (a dense or device copy)
         # and dropped before run() would hand its memory to the next allocation on the
@@ -761,7 +762,9 @@ class CopyPlan:
         if len(self._rows) <= COPY_MAX_ROWS:
             # The table rides in the launch: nothing to build on the device or to keep.
             graph_recording()  # a capture that a replay could not repeat correctly is refused
-            flat = (ctypes.c_int64 * (3 * len(self._rows)))(*chain.from_iterable(self._rows))
+            flat = self._flat
+            if flat is None or len(flat) != 3 * len(self._rows):  # rows are only ever appended
+                flat = self._flat = (ctypes.c_int64 * (3 * len(self._rows)))(*chain.from_iterable(self._rows))
             with device_guard(self.device):
                 status = lib.hbt_copy_rows(flat, len(self._rows), src_code, dst_code, op, float(divisor),
                                            stream_of(self.device))
