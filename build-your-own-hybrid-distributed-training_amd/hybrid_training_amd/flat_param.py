@@ -63,6 +63,8 @@ __all__ = [
     "reshard_state_dict_pieces",
 ]
 
+_FLOATS = (torch.float32, torch.bfloat16, torch.float16, torch.float64)
+
 #: Tile sums (doubles, one per 256 shard elements) up to which the local share keeps them
 #: in the norm partials' allocation: shards of up to 2 Mi elements.
 _SHARED_TILE_SUMS = 8192
@@ -543,8 +545,7 @@ class FlatParamHandle:
         accumulated row once (``hbt_grad_local_share_accumulated``; a float64 reduce
         dtype adds first and then reduces).
         """
-        floats = (torch.float32, torch.bfloat16, torch.float16, torch.float64)
-        if self._reduce_dtype not in floats or self._master_dtype not in floats:
+        if self._reduce_dtype not in _FLOATS or self._master_dtype not in _FLOATS:
             raise UnsupportedFeatureError(
                 format_error(
                     "fsdp.reduce_scatter_gradient",
@@ -565,10 +566,11 @@ class FlatParamHandle:
                     observed=len(grads),
                 )
             )
+        in_dtype, padded = grads[0].dtype, self._padded_numel
         for g in grads:
-            _native.require_device_tensor(g, "fsdp.reduce_scatter_gradient")
-            if g.numel() != self._padded_numel or g.dtype not in floats \
-                    or g.dtype != grads[0].dtype or not g.is_contiguous():
+            if not g.is_cuda:
+                _native.require_device_tensor(g, "fsdp.reduce_scatter_gradient")
+            if g.numel() != padded or g.dtype != in_dtype or in_dtype not in _FLOATS or not g.is_contiguous():
                 raise ShardingError(
                     format_error(
                         "fsdp.reduce_scatter_gradient",
@@ -577,24 +579,24 @@ class FlatParamHandle:
                         observed=f"{g.numel()} {g.dtype}",
                     )
                 )
-        if grads[0].dtype == torch.float64 and self._reduce_dtype != torch.float64:
+        if in_dtype == torch.float64 and self._reduce_dtype != torch.float64:
             raise UnsupportedFeatureError(
                 format_error("fsdp.reduce_scatter_gradient",
                              "float64 gradients are reduced in float64 (the kernels narrow only after the sum)",
                              observed=f"reduce dtype {self._reduce_dtype}",
                              resolution="set reduce_dtype to float64, or compute in a narrower dtype")
             )
-        local = self.local_shard_range()
         source_rank = self._shard_group.local_rank
+        start = source_rank * self._shard_numel  # local_shard_range()'s
         rows = None  # accumulator rows the reduction adds the last micro-batch to
         if self._accumulate_without_reduction:
-            self._accumulate(grads, local.start)
+            self._accumulate(grads, start)
             return None
         if self._grad_accumulator is not None:
             if self._reduce_dtype == torch.float64:
                 # Reduce the accumulated sums: row q is rank q's total restricted to this
                 # rank's slice, so the local share reads it at rank offset 0.
-                self._accumulate(grads, local.start)
+                self._accumulate(grads, start)
                 accumulator, self._grad_accumulator = self._grad_accumulator, None
                 grads = list(accumulator.unbind(0))
                 source_rank = 0
@@ -604,7 +606,7 @@ class FlatParamHandle:
                 # rewritten and read again.  The kernel only reads them, so they are
                 # dropped once it has been queued: a refused launch keeps them.
                 rows = self._grad_accumulator
-        valid = max(0, min(self._shard_numel, self._total_numel - local.start))
+        valid = max(0, min(self._shard_numel, self._total_numel - start))
         divisor = float(group) if (self._config.average_gradients and group > 1) else 1.0
         # A float64 master over a narrower reduce dtype: reduce into float32, widen after.
         widen = self._master_dtype == torch.float64 and self._reduce_dtype != torch.float64
@@ -619,15 +621,17 @@ class FlatParamHandle:
             # A small shard's launch is bound by host time: the partials and the kernel's
             # tile sums share one allocation (a large shard's tile sums are freed at once).
             partials = torch.empty(n_partials + n_tiles, dtype=torch.float64, device=self._device)
-            tile_sums_ptr = partials.data_ptr() + 8 * n_partials
+            partials_ptr = partials.data_ptr()
+            tile_sums_ptr = partials_ptr + 8 * n_partials
         else:
             partials = torch.empty(n_partials, dtype=torch.float64, device=self._device)
+            partials_ptr = partials.data_ptr()
             tile_sums = torch.empty(n_tiles, dtype=torch.float64, device=self._device)
             tile_sums_ptr = tile_sums.data_ptr()
         lib = _native.library()
         args = (group, source_rank, self._shard_numel, valid, _native.dtype_code(grads[0].dtype),
                 _native.dtype_code(self._reduce_dtype), divisor, _native.dtype_code(out_dtype),
-                out.data_ptr(), partials.data_ptr(), tile_sums_ptr, _native.stream_of(self._device))
+                out.data_ptr(), partials_ptr, tile_sums_ptr, _native.stream_of(self._device))
         grad_ptrs = _native.pointer_array([g.data_ptr() for g in grads])
         with _native.device_guard(self._device):
             if rows is None:

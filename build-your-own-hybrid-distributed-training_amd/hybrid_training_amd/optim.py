@@ -104,13 +104,6 @@ class NormPartials:
         return self.segments.get((offset, length))
 
 
-def _cached_partials(grad: torch.Tensor, offset: int, length: int, unscale: float) -> torch.Tensor | None:
-    record = getattr(grad, NORM_PARTIALS_ATTR, None)
-    if record is None or unscale != 1.0:
-        return None
-    return record.lookup(grad, offset, length)
-
-
 def build_inner_optimizer(
     parameters: Iterable[nn.Parameter], config: OptimizerConfig
 ) -> torch.optim.Optimizer:
@@ -336,7 +329,7 @@ def _mul_ptr(result: NormResult | None, dtype: torch.dtype) -> int | None:
 
 
 def _pending_unscale(grad: torch.Tensor) -> float:
-    return float(getattr(grad, PENDING_UNSCALE_ATTR, 1.0))
+    return float(grad.__dict__.get(PENDING_UNSCALE_ATTR, 1.0))
 
 
 def gradient_norm_pass(
@@ -364,18 +357,21 @@ def gradient_norm_pass(
     """
     lib = _native.library()
     batches: dict[tuple[torch.dtype, float], list[tuple[torch.Tensor, int, int, float]]] = {}
-    for grad, offset, length, weight in segments:
-        if not is_host(grad):
+    for segment in segments:
+        grad = segment[0]
+        dtype = grad.dtype
+        unscale = grad.__dict__.get(PENDING_UNSCALE_ATTR, 1.0)
+        if not grad.is_cuda and not is_host(grad):
             _native.require_device_tensor(grad, "optim.gradient_norm")
-        if grad.dtype not in (torch.float32, torch.bfloat16, torch.float16, torch.float64):
+        if dtype not in _NORM_CHUNKS:
             raise UnsupportedFeatureError(
                 format_error(
                     "optim.gradient_norm",
                     "gradients must be float64, float32, bfloat16 or float16",
-                    observed=str(grad.dtype),
+                    observed=str(dtype),
                 )
             )
-        if grad.dtype == torch.float64 and _pending_unscale(grad) != 1.0:
+        if unscale != 1.0 and dtype == torch.float64:
             raise UnsupportedFeatureError(
                 format_error("optim.gradient_norm",
                              "a float64 gradient is unscaled in place before its norm, not read through "
@@ -385,10 +381,8 @@ def gradient_norm_pass(
             raise ShardingError(
                 format_error("optim.gradient_norm", "gradients must be dense", observed=tuple(grad.stride()))
             )
-        if length > 0:
-            batches.setdefault((grad.dtype, _pending_unscale(grad)), []).append(
-                (grad, offset, length, weight)
-            )
+        if segment[2] > 0:
+            batches.setdefault((dtype, float(unscale)), []).append(segment)
     # Every segment's partials in summation order: the ones its producer left, where they
     # lie, or a run of slots in a fresh array that this pass fills.
     slots = 0
@@ -401,20 +395,21 @@ def gradient_norm_pass(
         for item in items:
             grad, offset, length, weight = item
             count = -(-length // chunk_elems)
-            cached = _cached_partials(grad, offset, length, unscale)
+            record = grad.__dict__.get(NORM_PARTIALS_ATTR) if unscale == 1.0 else None
+            cached = None if record is None else record.lookup(grad, offset, length)
             if cached is not None and cached.numel() == count and cached.is_contiguous():
                 # Partials a producer wrote over exact zeros are the same +0.0 under any
                 # finite non-negative weight.
-                if 0.0 <= weight < float("inf") and _zero_segment(grad, offset, length):
+                if weight != 1.0 and 0.0 <= weight < float("inf") and (offset, length) in record.zero:
                     weight = 1.0
                 order.append((cached, 0, count, weight))
                 continue
             if tag and weight == 1.0 and unscale == 1.0:
                 fresh.append((grad, offset, length, slots, count))
-            if is_host(grad):
+            if not grad.is_cuda:
                 launches.append((dtype, unscale, [item], slots))
             else:
-                if not batch or len(batch) == _native.MAX_TENSORS_PER_LAUNCH or is_host(launches[-1][2][0][0]):
+                if not batch or len(batch) == _native.MAX_TENSORS_PER_LAUNCH or not launches[-1][2][0][0].is_cuda:
                     batch = []
                     launches.append((dtype, unscale, batch, slots))
                 batch.append(item)
@@ -427,7 +422,7 @@ def gradient_norm_pass(
     stream = _native.stream_of(device)
     with _native.device_guard(device):
         for dtype, unscale, items, first in launches:
-            if is_host(items[0][0]):
+            if not items[0][0].is_cuda:
                 _stream_sqnorm(lib, *items[0], dtype, unscale, partials, first, device)
             else:
                 _launch_sqnorm(lib, items, dtype, unscale, partials, first, stream)
@@ -443,12 +438,6 @@ def gradient_norm_pass(
         else:
             setattr(grad, NORM_PARTIALS_ATTR, NormPartials(grad.data_ptr(), grad._version, found, grad.dtype))
     return NormResult(scalars)
-
-
-def _zero_segment(grad: torch.Tensor, offset: int, length: int) -> bool:
-    """Whether ``grad``'s producer wrote the segment as exact zeros (and the record is valid)."""
-    record = getattr(grad, NORM_PARTIALS_ATTR, None)
-    return record is not None and record.lookup(grad, offset, length) is not None and (offset, length) in record.zero
 
 
 def _finalize(lib, order, partials, scalars, max_norm, device, stream) -> None:
@@ -487,12 +476,14 @@ def _finalize(lib, order, partials, scalars, max_norm, device, stream) -> None:
     _native.check(status, "optim.hbt_grad_norm_finalize_parts")
 
 
+#: Elements per norm partial.
+_NORM_CHUNKS = {torch.float32: 32768, torch.bfloat16: 65536, torch.float16: 65536, torch.float64: 16384}
+
+
 def norm_chunk_elems(dtype: torch.dtype) -> int:
     """Elements per norm partial: 32768 of an fp32 gradient, 65536 of a 2-byte one,
     16384 of a float64 one."""
-    if dtype == torch.float64:
-        return 16384
-    return 32768 if dtype == torch.float32 else 65536
+    return _NORM_CHUNKS.get(dtype, 65536)
 
 
 def _stream_sqnorm(lib, grad, offset, length, weight, dtype, unscale, partials, slot, device) -> None:
@@ -551,8 +542,8 @@ def scale_gradients(grads: Sequence[torch.Tensor], dtype: torch.dtype, unscale: 
                                            _native.dtype_code(dtype), unscale, grad_mul_ptr, stream)
         _native.check(status, operation)
 
-    resident = [g for g in grads if not is_host(g)]
-    hosted = [g for g in grads if is_host(g)]
+    resident = [g for g in grads if g.is_cuda]
+    hosted = [g for g in grads if not g.is_cuda]
     with _native.device_guard(device):
         for start in range(0, len(resident), _native.MAX_TENSORS_PER_LAUNCH):
             chunk = resident[start : start + _native.MAX_TENSORS_PER_LAUNCH]
@@ -1073,7 +1064,8 @@ class ShardedOptimizer:
             g = p.grad
             if g is None:
                 continue
-            _native.require_dense(g, "optim.scale_gradients")
+            if not g.is_contiguous():
+                _native.require_dense(g, "optim.scale_gradients")
             unscale = _pending_unscale(g) if unscale_attr else 1.0
             groups.setdefault((g.dtype, unscale), []).append(g)
         for (dtype, unscale), grads in groups.items():
@@ -1084,11 +1076,13 @@ class ShardedOptimizer:
                 if p.grad is not None and hasattr(p.grad, PENDING_UNSCALE_ATTR):
                     delattr(p.grad, PENDING_UNSCALE_ATTR)
 
+    def _has_pending_unscale(self) -> bool:
+        grads = [p.grad for p in self._parameters]
+        return any(g is not None and PENDING_UNSCALE_ATTR in g.__dict__ for g in grads)
+
     def materialize_pending(self) -> None:
         """Apply any deferred loss-scale and clip factors to ``.grad`` in place."""
-        has_unscale = any(
-            p.grad is not None and hasattr(p.grad, PENDING_UNSCALE_ATTR) for p in self._parameters
-        )
+        has_unscale = self._has_pending_unscale()
         mul = self._pending_mul if self._pending_valid() else None
         if has_unscale or mul is not None:
             # Scaling keeps every element's finiteness (a finite norm gives a finite
@@ -1132,7 +1126,13 @@ class ShardedOptimizer:
         self._pending_mul = result
         self._pending_signature = signature
         if not (self._defer_clip or self._clip_in_step):
-            self.materialize_pending()  # the reference's grad.mul_(coefficient), on the device
+            # The reference's grad.mul_(coefficient), on the device.  Nothing has run since the
+            # norm pass, so there is no change to look for, and scaling keeps every element's
+            # finiteness, so the pass's flag describes the clipped gradients.
+            self._scale_grads(result, unscale_attr=self._has_pending_unscale())
+            self._last_check = (_grad_signature(self._parameters), result)
+            self._pending_mul = None
+            self._pending_signature = None
         return result.norm
 
     def clip_and_step(self, max_norm: float) -> torch.Tensor:
@@ -1181,12 +1181,12 @@ class ShardedOptimizer:
         if self._host_resident:
             self._stream.synchronize()  # host parameters, gradients and state are final
         if write_back:
-            written = [p.grad for p in self._parameters if p.grad is not None]
-            if written and (grad_mul is not None or any(_pending_unscale(g) != 1.0 for g in written)):
+            written = [g for g in [p.grad for p in self._parameters] if g is not None]
+            scaled = [g for g in written if PENDING_UNSCALE_ATTR in g.__dict__]
+            if written and (grad_mul is not None or any(_pending_unscale(g) != 1.0 for g in scaled)):
                 increment_version(written)
-            for g in written:
-                if hasattr(g, PENDING_UNSCALE_ATTR):
-                    delattr(g, PENDING_UNSCALE_ATTR)
+            for g in scaled:
+                delattr(g, PENDING_UNSCALE_ATTR)
         self._pending_mul = None
         self._pending_signature = None
 
@@ -1202,6 +1202,9 @@ class ShardedOptimizer:
         grad = p.grad
         if grad is None:
             return None
+        if (p.is_cuda and grad.is_cuda and grad.is_contiguous() and p.is_contiguous() and grad.shape == p.shape
+                and (p.dtype, grad.dtype) in _native.OPTIMIZER_DTYPES):
+            return grad
         if is_host(p) != is_host(grad):
             raise ShardingError(
                 format_error("optim.ShardedOptimizer.step",
@@ -1228,36 +1231,41 @@ class ShardedOptimizer:
             )
         return grad
 
-    def _stepped_parameters(self) -> list[tuple[dict, nn.Parameter, torch.Tensor]]:
-        """``(group, parameter, gradient)`` of every parameter this step updates.
+    def _stepped_parameters(self) -> list[tuple[dict, nn.Parameter, torch.Tensor, dict | None]]:
+        """``(group, parameter, gradient, existing state or None)`` of every parameter this
+        step updates.
 
         Every parameter, its gradient and its existing state are checked here, before
         any state is created or any step counter advances, so a refused step leaves
         the optimizer as it was.
         """
         stepped = []
+        states = self._optimizer.state
         for group in self._optimizer.param_groups:
+            # the state the update reads: AdamW's moments, or SGD's buffer with momentum
+            read = (("exp_avg", "exp_avg_sq") if "betas" in group
+                    else ("momentum_buffer",) if float(group.get("momentum", 0.0)) != 0.0 else ())
             for p in group["params"]:
-                grad = self._checked_grad(self._device_param.get(id(p), p), group)
+                grad = self._checked_grad(self._device_param.get(id(p), p) if self._device_param else p, group)
                 if grad is None:
                     continue
-                # the state the update reads: AdamW's moments, or SGD's buffer with momentum
-                read = (("exp_avg", "exp_avg_sq") if "betas" in group
-                        else ("momentum_buffer",) if float(group.get("momentum", 0.0)) != 0.0 else ())
-                for key in read:
-                    value = self._optimizer.state[p].get(key) if p in self._optimizer.state else None
-                    if value is not None:
-                        _native.require_dense(value, "optim.ShardedOptimizer.step")
-                stepped.append((group, p, grad))
+                state = states.get(p)
+                if state:
+                    for key in read:
+                        value = state.get(key)
+                        if value is not None and not value.is_contiguous():
+                            _native.require_dense(value, "optim.ShardedOptimizer.step")
+                stepped.append((group, p, grad, state))
         return stepped
 
     def _run_adamw_step(self, grad_mul: NormResult | None, write_back: bool) -> None:
         lib = _native.library()
         recording = self._recording_check()
-        batches: dict[tuple, list[nn.Parameter]] = {}
-        for group, p, grad in self._stepped_parameters():
-            state = self._optimizer.state[p]
-            if len(state) == 0:
+        batches: dict[tuple, list[tuple[nn.Parameter, torch.Tensor, dict]]] = {}
+        formed: dict[tuple[int, float], tuple[float, ...]] = {}  # scalars per group and step count
+        for group, p, grad, state in self._stepped_parameters():
+            if not state:
+                state = self._optimizer.state[p]
                 if recording is not None:
                     raise _unrecordable("the first step creates the optimizer state")
                 # Same initial state as torch.optim.Adam._init_group.
@@ -1270,36 +1278,41 @@ class ShardedOptimizer:
                 step_t.fill_(step)  # step_t += 1
             else:
                 step = _next_step(step_t)  # the step each replay advances to
-            key = (_adamw_scalars(group, step), p.dtype, grad.dtype, _pending_unscale(grad))
-            batches.setdefault(key, []).append(p)
+            scalars = formed.get((id(group), step))
+            if scalars is None:
+                scalars = formed[(id(group), step)] = _adamw_scalars(group, step)
+            key = (scalars, p.dtype, grad.dtype, _pending_unscale(grad))
+            batches.setdefault(key, []).append((p, grad, state))
         stream = _native.stream_of(self._device)
         with _native.device_guard(self._device):
             for (scalars, pdtype, gdtype, unscale), batch in batches.items():
                 flags = _write_back_flag(write_back, grad_mul, unscale)
                 mul_ptr = _mul_ptr(grad_mul, gdtype)
-                for p in batch:
-                    if is_host(p):
+                for p, _, _ in batch:
+                    if not p.is_cuda:
                         self._streamed_adamw(lib, p, scalars, pdtype, gdtype, unscale, mul_ptr, flags)
-                params = [p for p in batch if not is_host(p)]
+                resident = [item for item in batch if item[0].is_cuda]
                 slot = None
-                if recording is not None and params:
+                if recording is not None and resident:
                     slot = recording.new_slot()
-                    recording.steps.append(_RecordedAdamW(self, slot, recording.record_address(slot), params,
-                                                          pdtype, unscale, scalars))
-                for start in range(0, len(params), _native.MAX_TENSORS_PER_LAUNCH):
-                    chunk = params[start : start + _native.MAX_TENSORS_PER_LAUNCH]
-                    states = [self._optimizer.state[p] for p in chunk]
+                    recording.steps.append(_RecordedAdamW(self, slot, recording.record_address(slot),
+                                                          [p for p, _, _ in resident], pdtype, unscale, scalars))
+                for start in range(0, len(resident), _native.MAX_TENSORS_PER_LAUNCH):
+                    chunk = resident[start : start + _native.MAX_TENSORS_PER_LAUNCH]
+                    params = [p for p, _, _ in chunk]
+                    first = [state["exp_avg"] for _, _, state in chunk]
+                    second = [state["exp_avg_sq"] for _, _, state in chunk]
                     status = _adamw_call(
                         lib, pdtype, gdtype,
-                        [p.data_ptr() for p in chunk],
-                        [p.grad.data_ptr() for p in chunk],
-                        [s["exp_avg"].data_ptr() for s in states],
-                        [s["exp_avg_sq"].data_ptr() for s in states],
-                        [p.numel() for p in chunk],
+                        [p.data_ptr() for p in params],
+                        [g.data_ptr() for _, g, _ in chunk],
+                        [m.data_ptr() for m in first],
+                        [v.data_ptr() for v in second],
+                        [p.numel() for p in params],
                         unscale, mul_ptr, scalars, flags, stream, slot,
                     )
                     _native.check(status, "optim.hbt_adamw_step")
-                    increment_version(chunk + [s["exp_avg"] for s in states] + [s["exp_avg_sq"] for s in states])
+                    increment_version(params + first + second)
 
     def _recording_check(self) -> "_native.GraphRecording | None":
         """The graph recording this step joins, after refusing what a replay cannot repeat."""
@@ -1371,7 +1384,7 @@ class ShardedOptimizer:
         lib = _native.library()
         recording = self._recording_check()
         batches: dict[tuple, list[nn.Parameter]] = {}
-        for group, p, grad in self._stepped_parameters():
+        for group, p, grad, _ in self._stepped_parameters():
             # Scalars exactly as torch forms them: Python doubles, rounded to fp32 (and
             # each alpha to a 2-byte parameter dtype inside the kernel's entry point), or
             # kept as doubles for float64 parameters.
