@@ -1195,20 +1195,23 @@ __device__ __forceinline__ double finalize_sum(int64_t count, Value&& value) {
     return block_sum<kFinalBlock>((a0 + a1) + (a2 + a3));
 }
 
-__device__ __forceinline__ void write_norm_outputs(double total, double max_norm, const NormOutputs& out) {
-    // clamp_min(0) keeps NaN; sqrt of fp64 is correctly rounded.
-    const double clamped = total < 0.0 ? 0.0 : total;
-    const double norm = sqrt(clamped);
-    if (out.sum != nullptr) out.sum[0] = total;
-    if (out.norm != nullptr) out.norm[0] = norm;
-    // The reference multiplies by the Python-double coefficient only when it is below 1:
-    // fp32, bf16 and fp16 gradients take it as torch passes it to their kernels, rounded
-    // to fp32; float64 gradients take the double itself.
-    double mul = 1.0;
+// clamp_min(0) keeps NaN; sqrt of fp64 is correctly rounded.
+__device__ __forceinline__ double norm_of(double total) { return sqrt(total < 0.0 ? 0.0 : total); }
+// The reference multiplies by the Python-double coefficient only when it is below 1:
+// fp32, bf16 and fp16 gradients take it as torch passes it to their kernels, rounded
+// to fp32; float64 gradients take the double itself.
+__device__ __forceinline__ double clip_multiplier(double norm, double max_norm) {
     if (max_norm > 0.0) {
         const double coef = max_norm / (norm + 1e-6);
-        if (coef < 1.0) mul = coef;
+        if (coef < 1.0) return coef;
     }
+    return 1.0;
+}
+__device__ __forceinline__ void write_norm_outputs(double total, double max_norm, const NormOutputs& out) {
+    const double norm = norm_of(total);
+    const double mul = clip_multiplier(norm, max_norm);
+    if (out.sum != nullptr) out.sum[0] = total;
+    if (out.norm != nullptr) out.norm[0] = norm;
     if (out.grad_mul != nullptr) out.grad_mul[0] = static_cast<float>(mul);
     if (out.grad_mul64 != nullptr) out.grad_mul64[0] = mul;
     if (out.nonfinite != nullptr) out.nonfinite[0] = isfinite(total) ? 0 : 1;
@@ -1233,21 +1236,21 @@ struct PartTable {
     int64_t first[HBT_MAX_NORM_PARTS + 1];
     int32_t parts;
 };
-__global__ __launch_bounds__(kFinalBlock) void norm_finalize_parts_kernel(PartTable tab, double max_norm,
-                                                                          NormOutputs out) {
+// The weighted sum over the table's arrays, valid in thread 0 of a kFinalBlock-lane workgroup.
+__device__ __forceinline__ double parts_sum(const PartTable& tab) {
     static_assert(HBT_MAX_NORM_PARTS < kFinalBlock, "one lane per part fills the LDS table");
     __shared__ const double* p[HBT_MAX_NORM_PARTS];
     __shared__ double w[HBT_MAX_NORM_PARTS];
     __shared__ int64_t first[HBT_MAX_NORM_PARTS + 1];
     const int t = static_cast<int>(threadIdx.x);
-    if (t < tab.parts) {
+    const int parts = tab.parts;
+    if (t < parts) {
         p[t] = tab.p[t];
         w[t] = tab.w[t];
     }
-    if (t <= tab.parts) first[t] = tab.first[t];
+    if (t <= parts) first[t] = tab.first[t];
     __syncthreads();
-    const int parts = tab.parts;
-    const double total = finalize_sum(first[parts], [&](int64_t i) {
+    return finalize_sum(first[parts], [&](int64_t i) {
         int lo = 0, hi = parts - 1;  // the last part that starts at or before i
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -1256,7 +1259,11 @@ __global__ __launch_bounds__(kFinalBlock) void norm_finalize_parts_kernel(PartTa
         }
         return p[lo][i - first[lo]] * w[lo];
     });
-    if (t == 0) write_norm_outputs(total, max_norm, out);
+}
+__global__ __launch_bounds__(kFinalBlock) void norm_finalize_parts_kernel(PartTable tab, double max_norm,
+                                                                          NormOutputs out) {
+    const double total = parts_sum(tab);
+    if (threadIdx.x == 0) write_norm_outputs(total, max_norm, out);
 }
 
 // ---- in-place scaling ---------------------------------------------------------------
@@ -1345,6 +1352,38 @@ __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale
         for (int c = 0; c < K; ++c) v[u][c] = scale_one<D>(v[u][c], unscale, mul);
         store_upto<D, K, kKeep>(X, base + (int64_t(u) * kScaleBlock + threadIdx.x) * K, n, v[u]);
     }
+}
+
+// The finalize and the in-place clip of a short list of gradients in one launch: every
+// workgroup sums the partials itself (the same sum in the same order, read from the cache),
+// workgroup 0 writes the outputs, and each scales its tiles of 4,096 elements by the
+// multiplier it formed, bitwise norm_finalize_parts_kernel followed by scale_kernel.  A step
+// over gradients this small is bound by its launches (about 4 us of host time each, and as
+// long on the device): the 929-element MLP tail
+// takes 58 us with the two and 53 us with the one.  Past kClipMax elements
+// the sums repeated by every workgroup cost what the launch saves.
+constexpr int64_t kClipTile = int64_t(kFinalBlock) * 4;
+template <int D>
+__global__ __launch_bounds__(kFinalBlock) void norm_clip_kernel(PartTable parts, ScaleTable tab, double max_norm,
+                                                                NormOutputs out) {
+    __shared__ float shared_mul;
+    const double total = parts_sum(parts);
+    if (threadIdx.x == 0) {
+        shared_mul = static_cast<float>(clip_multiplier(norm_of(total), max_norm));
+        if (blockIdx.x == 0) write_norm_outputs(total, max_norm, out);
+    }
+    __syncthreads();
+    const float mul = shared_mul;
+    if (mul == 1.0f) return;  // the gradients are left untouched, bits and all
+    const int64_t block = blockIdx.x;
+    const int t = owning_tensor(tab.first_block, tab.count, block);
+    const int64_t e = (block - tab.first_block[t]) * kClipTile + int64_t(threadIdx.x) * 4;
+    const int64_t n = tab.n[t];
+    float v[4];
+    load_upto<D, 4>(tab.x[t], e, n, v);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = round_to<D>(v[c] * mul);
+    store_upto<D, 4>(tab.x[t], e, n, v);
 }
 
 // ---- float64 parameters ---------------------------------------------------------------
@@ -2362,20 +2401,17 @@ int32_t hbt_grad_norm_finalize(const double* partials, int64_t count, double max
     return check_launch("hbt_grad_norm_finalize");
 }
 
-int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_t* counts, const double* weights,
-                                     int32_t parts, double max_norm, double* sum_out, double* norm_out,
-                                     float* grad_mul_out, double* grad_mul64_out, int32_t* nonfinite_out,
-                                     void* stream) {
-    clear_error();
+static int32_t build_part_table(const char* who, const double* const* partials, const int64_t* counts,
+                                const double* weights, int32_t parts, PartTable& tab) {
     if (parts < 0 || parts > HBT_MAX_NORM_PARTS ||
         (parts > 0 && (partials == nullptr || counts == nullptr || weights == nullptr))) {
-        set_error("hbt_grad_norm_finalize_parts: bad table (parts=%d of at most %d)", parts, HBT_MAX_NORM_PARTS);
+        set_error("%s: bad table (parts=%d of at most %d)", who, parts, HBT_MAX_NORM_PARTS);
         return HBT_ERR_INVALID_ARGUMENT;
     }
-    PartTable tab{};
+    tab = PartTable{};
     for (int i = 0; i < parts; ++i) {
         if (counts[i] < 0 || (counts[i] > 0 && partials[i] == nullptr)) {
-            set_error("hbt_grad_norm_finalize_parts: part %d has a bad pointer or count", i);
+            set_error("%s: part %d has a bad pointer or count", who, i);
             return HBT_ERR_INVALID_ARGUMENT;
         }
         if (counts[i] == 0) continue;  // the search wants strictly increasing starts
@@ -2384,9 +2420,78 @@ int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_
         tab.first[tab.parts + 1] = tab.first[tab.parts] + counts[i];
         ++tab.parts;
     }
+    return HBT_OK;
+}
+
+// A table of tensors scaled in place in tiles of `tile` elements; `blocks` counts the tiles.
+static int32_t build_scale_table(const char* who, void* const* tensors, const int64_t* numels, int32_t count,
+                                 int64_t tile, ScaleTable& tab, int64_t& blocks) {
+    if (count < 0 || count > kMaxT || (count > 0 && (tensors == nullptr || numels == nullptr))) {
+        set_error("%s: bad table (count=%d)", who, count);
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    tab = ScaleTable{};
+    tab.count = count;
+    blocks = 0;
+    for (int i = 0; i < count; ++i) {
+        if (numels[i] < 0 || (numels[i] > 0 && tensors[i] == nullptr)) {
+            set_error("%s: tensor %d has a bad pointer or numel", who, i);
+            return HBT_ERR_INVALID_ARGUMENT;
+        }
+        tab.x[i] = tensors[i];
+        tab.n[i] = numels[i];
+        tab.first_block[i] = blocks;
+        blocks += (numels[i] + tile - 1) / tile;
+    }
+    for (int i = count; i <= kMaxT; ++i) tab.first_block[i] = blocks;
+    return HBT_OK;
+}
+
+int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_t* counts, const double* weights,
+                                     int32_t parts, double max_norm, double* sum_out, double* norm_out,
+                                     float* grad_mul_out, double* grad_mul64_out, int32_t* nonfinite_out,
+                                     void* stream) {
+    clear_error();
+    PartTable tab{};
+    const int32_t status = build_part_table("hbt_grad_norm_finalize_parts", partials, counts, weights, parts, tab);
+    if (status != HBT_OK) return status;
     norm_finalize_parts_kernel<<<1, kFinalBlock, 0, as_stream(stream)>>>(
         tab, max_norm, NormOutputs{sum_out, norm_out, grad_mul_out, grad_mul64_out, nonfinite_out});
     return check_launch("hbt_grad_norm_finalize_parts");
+}
+
+int32_t hbt_grad_norm_clip(const double* const* partials, const int64_t* counts, const double* weights, int32_t parts,
+                           double max_norm, void* const* grads, const int64_t* numels, int32_t count, int32_t dtype,
+                           double* sum_out, double* norm_out, float* grad_mul_out, double* grad_mul64_out,
+                           int32_t* nonfinite_out, void* stream) {
+    clear_error();
+    if (dtype != F32 && dtype != BF16 && dtype != F16) {
+        set_error("hbt_grad_norm_clip: dtype %d is not F32, BF16 or F16", dtype);
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    PartTable tab{};
+    int32_t status = build_part_table("hbt_grad_norm_clip", partials, counts, weights, parts, tab);
+    if (status != HBT_OK) return status;
+    ScaleTable scale{};
+    int64_t blocks = 0;
+    status = build_scale_table("hbt_grad_norm_clip", grads, numels, count, kClipTile, scale, blocks);
+    if (status != HBT_OK) return status;
+    if (blocks > HBT_CLIP_MAX_ELEMENTS / kClipTile + kMaxT) {
+        set_error("hbt_grad_norm_clip: more than %lld elements (finalize, then hbt_scale_inplace)",
+                  static_cast<long long>(HBT_CLIP_MAX_ELEMENTS));
+        return HBT_ERR_UNSUPPORTED;
+    }
+    const NormOutputs out{sum_out, norm_out, grad_mul_out, grad_mul64_out, nonfinite_out};
+    hipStream_t st = as_stream(stream);
+    if (blocks == 0) {
+        norm_finalize_parts_kernel<<<1, kFinalBlock, 0, st>>>(tab, max_norm, out);
+    } else {
+        const dim3 grid(static_cast<unsigned>(blocks));
+        if (dtype == F32) norm_clip_kernel<F32><<<grid, kFinalBlock, 0, st>>>(tab, scale, max_norm, out);
+        else if (dtype == BF16) norm_clip_kernel<BF16><<<grid, kFinalBlock, 0, st>>>(tab, scale, max_norm, out);
+        else norm_clip_kernel<F16><<<grid, kFinalBlock, 0, st>>>(tab, scale, max_norm, out);
+    }
+    return check_launch("hbt_grad_norm_clip");
 }
 
 int32_t hbt_grad_norm_noalloc(const void* const* grads, const int64_t* numels, const double* weights,
@@ -2437,21 +2542,10 @@ int32_t hbt_scale_inplace(void* const* tensors, const int64_t* numels, int32_t c
         return HBT_ERR_INVALID_ARGUMENT;
     }
     ScaleTable tab{};
-    tab.count = count;
-    const int64_t tile = dtype == F32 ? scale_tile<F32>() : scale_tile<BF16>();
     int64_t blocks = 0;
-    for (int i = 0; i < count; ++i) {
-        if (numels[i] < 0 || (numels[i] > 0 && tensors[i] == nullptr)) {
-            set_error("hbt_scale_inplace: tensor %d has a bad pointer or numel", i);
-            return HBT_ERR_INVALID_ARGUMENT;
-        }
-        tab.x[i] = tensors[i];
-        tab.n[i] = numels[i];
-        tab.first_block[i] = blocks;
-        blocks += (numels[i] + tile - 1) / tile;
-    }
-    tab.first_block[count] = blocks;
-    for (int i = count + 1; i <= kMaxT; ++i) tab.first_block[i] = blocks;
+    const int32_t status = build_scale_table("hbt_scale_inplace", tensors, numels, count,
+                                             dtype == F32 ? scale_tile<F32>() : scale_tile<BF16>(), tab, blocks);
+    if (status != HBT_OK) return status;
     hipStream_t st = as_stream(stream);
     const int threads = dtype == F32 ? scale_block<F32>() : scale_block<BF16>();
     const bool keep = keep_for_next_pass(tab.n, tab.count, dtype);

@@ -17,6 +17,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import struct
 import threading
 from collections import OrderedDict
 from collections.abc import Iterable, Sequence
@@ -44,6 +45,7 @@ __all__ = [
     "SGD_MOMENTUM",
     "SGD_NESTEROV",
     "SGD_WEIGHT_DECAY",
+    "CLIP_MAX_ELEMENTS",
     "CopyPlan",
     "DTYPE_BF16",
     "DTYPE_F16",
@@ -70,6 +72,7 @@ ABI_VERSION = 19
 MAX_TENSORS_PER_LAUNCH = 16
 MAX_LOCAL_RANKS = 64
 MAX_NORM_PARTS = 128
+CLIP_MAX_ELEMENTS = 1048576
 #: Doubles of working storage hbt_scale_inplace_sqnorm takes per partial for 2-byte gradients.
 PIECES_PER_NORM_CHUNK = 128
 
@@ -152,6 +155,11 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
         (_ptr_array, _i64_array, _f64_array, _c_i32, _c_f64, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
          _c_void_p),
     ),
+    "hbt_grad_norm_clip": (
+        _c_i32,
+        (_ptr_array, _i64_array, _f64_array, _c_i32, _c_f64, _ptr_array, _i64_array, _c_i32, _c_i32, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p),
+    ),
     "hbt_grad_norm_noalloc": (
         _c_i32,
         (_ptr_array, _i64_array, _f64_array, _c_i32, _c_i32, _c_f32, _c_f64, _c_void_p, _c_void_p,
@@ -162,7 +170,7 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
         _c_i32,
         (_c_void_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p),
     ),
-    "hbt_copy_rows": (_c_i32, (_i64_array, _c_i32, _c_i32, _c_i32, _c_i32, _c_f32, _c_void_p)),
+    "hbt_copy_rows": (_c_i32, (_c_void_p, _c_i32, _c_i32, _c_i32, _c_i32, _c_f32, _c_void_p)),
     "hbt_grad_local_share": (
         _c_i32,
         (_ptr_array, _c_i32, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p, _c_void_p),
@@ -681,7 +689,7 @@ class CopyPlan:
     def __init__(self, device: torch.device) -> None:
         self.device = torch.device(device)
         self._rows: list[tuple[int, int, int]] = []
-        self._flat: ctypes.Array | None = None  # the rows as the launch takes them, kept for a repeated run
+        self._flat: bytes | None = None  # the rows as the launch takes them, kept for a repeated run
         # The tensors the rows address, held for the plan's lifetime.  A row records
         # only addresses: a temporary the caller made for it (a dense or device copy)
         # and dropped before run() would hand its memory to the next allocation on the
@@ -762,11 +770,12 @@ class CopyPlan:
         if len(self._rows) <= COPY_MAX_ROWS:
             # The table rides in the launch: nothing to build on the device or to keep.
             graph_recording()  # a capture that a replay could not repeat correctly is refused
+            count = len(self._rows)
             flat = self._flat
-            if flat is None or len(flat) != 3 * len(self._rows):  # rows are only ever appended
-                flat = self._flat = (ctypes.c_int64 * (3 * len(self._rows)))(*chain.from_iterable(self._rows))
+            if flat is None or len(flat) != 24 * count:  # rows are only ever appended
+                flat = self._flat = struct.pack(f"{3 * count}q", *chain.from_iterable(self._rows))
             with device_guard(self.device):
-                status = lib.hbt_copy_rows(flat, len(self._rows), src_code, dst_code, op, float(divisor),
+                status = lib.hbt_copy_rows(flat, count, src_code, dst_code, op, float(divisor),
                                            stream_of(self.device))
             check(status, "native.hbt_copy_rows")
             bump_versions(self._dests.values())

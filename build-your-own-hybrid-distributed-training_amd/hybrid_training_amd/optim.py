@@ -338,6 +338,7 @@ def gradient_norm_pass(
     *,
     max_norm: float,
     tag: bool = False,
+    clip: Sequence[torch.Tensor] = (),
 ) -> NormResult:
     """Weighted fp64 squared norm of gradient segments, plus the clip multiplier.
 
@@ -348,7 +349,9 @@ def gradient_norm_pass(
     order.  With ``tag``, every segment of weight 1 read without a pending factor
     leaves its partials on its gradient (:class:`NormPartials`), so a later pass over
     the unchanged gradient, such as the clip after the loss scaler's overflow check,
-    reuses them instead of reading the gradient again.
+    reuses them instead of reading the gradient again.  With ``clip``, gradients that
+    :func:`_clips_in_one_launch` accepts, the finalize also multiplies those in place by the
+    clip multiplier, in the same launch.
 
     A gradient in host memory (a parameter shard kept on the host) is uploaded through
     the device's :class:`~hybrid_training_amd.host_staging.HostStream` and summed there
@@ -426,7 +429,7 @@ def gradient_norm_pass(
                 _stream_sqnorm(lib, *items[0], dtype, unscale, partials, first, device)
             else:
                 _launch_sqnorm(lib, items, dtype, unscale, partials, first, stream)
-        _finalize(lib, order, partials, scalars, max_norm, device, stream)
+        _finalize(lib, order, partials, scalars, max_norm, device, stream, clip)
     records: dict[int, tuple[torch.Tensor, dict[tuple[int, int], torch.Tensor]]] = {}
     for grad, offset, length, slot, count in fresh:
         records.setdefault(id(grad), (grad, {}))[1][(offset, length)] = partials[slot : slot + count]
@@ -440,7 +443,23 @@ def gradient_norm_pass(
     return NormResult(scalars)
 
 
-def _finalize(lib, order, partials, scalars, max_norm, device, stream) -> None:
+def _clips_in_one_launch(grads: Sequence[torch.Tensor]) -> bool:
+    """Whether the norm's finalize may clip ``grads`` itself (``hbt_grad_norm_clip``): dense
+    gradients of one fp32, bf16 or fp16 dtype on the device without a pending factor, few
+    and small enough that a launch costs more than summing their partials again in every
+    workgroup."""
+    if not grads or len(grads) > _native.MAX_TENSORS_PER_LAUNCH:
+        return False
+    dtype, total = grads[0].dtype, 0
+    for g in grads:
+        total += g.numel()
+        if (total > _native.CLIP_MAX_ELEMENTS or g.dtype != dtype or not g.is_cuda or not g.is_contiguous()
+                or PENDING_UNSCALE_ATTR in g.__dict__):
+            return False
+    return dtype in (torch.float32, torch.bfloat16, torch.float16)
+
+
+def _finalize(lib, order, partials, scalars, max_norm, device, stream, clip=()) -> None:
     """Sum the partials of ``order`` into ``scalars`` (:class:`NormResult`'s layout) in one
     launch: over one array when they lie one after another with weight 1, else over the
     list of arrays.  Lists past ``MAX_NORM_PARTS`` arrays are gathered into one first."""
@@ -465,6 +484,15 @@ def _finalize(lib, order, partials, scalars, max_norm, device, stream) -> None:
         parts = [(whole.data_ptr(), first, 1.0)]
     out = scalars.data_ptr()
     outputs = (out, out + 8, out + 24, out + 16, out + 28, stream)
+    if clip:
+        status = lib.hbt_grad_norm_clip(
+            _native.pointer_array([p for p, _, _ in parts]), _native.int64_array([n for _, n, _ in parts]),
+            _native.double_array([w for _, _, w in parts]), len(parts), float(max_norm),
+            _native.pointer_array([g.data_ptr() for g in clip]), _native.int64_array([g.numel() for g in clip]),
+            len(clip), _native.dtype_code(clip[0].dtype), *outputs)
+        _native.check(status, "optim.hbt_grad_norm_clip")
+        increment_version(clip)
+        return
     if len(parts) <= 1 and all(weight == 1.0 for _, _, weight in parts):
         address, count, _ = parts[0] if parts else (None, 0, 1.0)
         status = lib.hbt_grad_norm_finalize(address, count, float(max_norm), *outputs)
@@ -1049,10 +1077,12 @@ class ShardedOptimizer:
         self._last_check: tuple[tuple[tuple[int, int, int], ...], NormResult | torch.Tensor] | None = None
 
     # -- norm and clip ---------------------------------------------------------------
-    def _norm(self, max_norm: float) -> tuple[NormResult, tuple[tuple[int, int, int], ...]]:
-        """The norm pass over the current gradients, and their signature."""
+    def _norm(self, max_norm: float, clip: Sequence[torch.Tensor] = ()) -> tuple[NormResult,
+                                                                              tuple[tuple[int, int, int], ...]]:
+        """The norm pass over the current gradients, with ``clip`` clipped by it, and their
+        signature after it."""
         segments = [s for c in self._contributions for s in c.segments()]
-        result = gradient_norm_pass(segments, self._device, max_norm=max_norm)
+        result = gradient_norm_pass(segments, self._device, max_norm=max_norm, clip=clip)
         signature = _grad_signature(self._parameters)
         self._last_check = (signature, result)
         return result, signature
@@ -1120,12 +1150,17 @@ class ShardedOptimizer:
         """
         if self._pending_mul is not None:
             self.materialize_pending()
+        in_place = max_norm > 0 and not (self._defer_clip or self._clip_in_step)
+        if in_place:
+            grads = [g for g in [p.grad for p in self._parameters] if g is not None]
+            if _clips_in_one_launch(grads):
+                return self._norm(max_norm, grads)[0].norm
         result, signature = self._norm(max_norm)
         if max_norm <= 0:
             return result.norm
         self._pending_mul = result
         self._pending_signature = signature
-        if not (self._defer_clip or self._clip_in_step):
+        if in_place:
             # The reference's grad.mul_(coefficient), on the device.  Nothing has run since the
             # norm pass, so there is no change to look for, and scaling keeps every element's
             # finiteness, so the pass's flag describes the clipped gradients.

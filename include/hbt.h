@@ -190,6 +190,23 @@ int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_
                                      void* stream);
 
 /* ------------------------------------------------------------------------------
+ * Stage 2 and the in-place clip of a short list of gradients in one launch.
+ *
+ * Replaces: the clip coefficient and the grad.mul_ loop of ShardedOptimizer.clip_grad_norm
+ *   (optim/sharded_optimizer.py:331-337) where launches cost more than the gradients do.
+ * Writes what hbt_grad_norm_finalize_parts writes, and multiplies the `count` gradients of
+ * `dtype` (F32, BF16 or F16; at most HBT_MAX_TENSORS_PER_LAUNCH of them and, rounded up to
+ * 4,096 each, HBT_CLIP_MAX_ELEMENTS elements together, else HBT_ERR_UNSUPPORTED) in place by
+ * the fp32 multiplier, rounded to the dtype, untouched when it is 1: bitwise that call followed
+ * by hbt_scale_inplace with its multiplier.  The gradients must not overlap the partials.
+ * ---------------------------------------------------------------------------- */
+#define HBT_CLIP_MAX_ELEMENTS 1048576
+int32_t hbt_grad_norm_clip(const double* const* partials, const int64_t* counts, const double* weights, int32_t parts,
+                           double max_norm, void* const* grads, const int64_t* numels, int32_t count, int32_t dtype,
+                           double* sum_out, double* norm_out, float* grad_mul_out, double* grad_mul64_out,
+                           int32_t* nonfinite_out, void* stream);
+
+/* ------------------------------------------------------------------------------
  * Weighted squared norm and clip coefficient with no allocation and no workspace.
  *
  * This entry point has no counterpart in the reference.  It is for callers that

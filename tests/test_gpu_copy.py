@@ -434,8 +434,8 @@ def test_copy_rows_refuses_what_it_cannot_move(device):
     ok = (buf.data_ptr(), buf.data_ptr() + 16, 4)
 
     def status(rows, count=None, src=0, dst=0, op=0):
-        return lib.hbt_copy_rows(_native.int64_array([v for r in rows for v in r]), len(rows) if count is None else count,
-                                 src, dst, op, 2.0, stream)
+        flat = np.array(rows, dtype=np.int64).reshape(-1)
+        return lib.hbt_copy_rows(flat.ctypes.data, len(rows) if count is None else count, src, dst, op, 2.0, stream)
 
     assert status([ok]) == 0 and status([(0, 0, 0)] * 3) == 0 and status([], 0) == 0
     assert status([ok], count=_native.COPY_MAX_ROWS + 1) == -1

@@ -655,3 +655,70 @@ def test_norm_from_partials_in_many_arrays(device, tensors):
     assert torch.equal(first.scalars.view(torch.int64), again.scalars.view(torch.int64))
     ref = float(sum(w * g.double().square().sum() for g, _, _, w in segments))
     assert abs(float(first.sum) - ref) <= 1e-12 * ref
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sizes", [[1], [929], [4095, 4096, 4097], [0, 5, 0, 70_001], [3] * 16, [1 << 20]])
+@pytest.mark.parametrize("case", ["clipped", "below", "inf", "nan"])
+def test_norm_clip_is_the_finalize_and_the_scale(device, dtype, sizes, case):
+    """The one-launch finalize and clip: gradients and every output bitwise the finalize over
+    the same partials followed by the in-place scale, with a norm above and below the limit
+    (left untouched, NaN payloads and signed zeros included) and a non-finite one."""
+    lib = _native.library()
+    code, stream = _native.dtype_code(dtype), _native.stream_of(device)
+    gen = torch.Generator(device=device).manual_seed(len(sizes))
+    store = (torch.randn(sum(sizes) + 1, device=device, generator=gen) * 0.1).to(dtype)
+    store[-1] = float("inf") if case == "inf" else float("nan") if case == "nan" else -0.0
+    grads, at = [], 1  # one element in: off every vector boundary
+    for n in sizes:
+        grads.append(store[at : at + n])
+        at += n
+    chunk = 32768 if dtype == torch.float32 else 65536
+    counts = [-(-n // chunk) for n in sizes]
+    partials = [torch.empty(max(1, c), dtype=torch.float64, device=device) for c in counts]
+    for g, p in zip(grads, partials):
+        _native.check(lib.hbt_grad_sqnorm_partials(
+            _native.pointer_array([g.data_ptr()]), _native.int64_array([g.numel()]), _native.double_array([1.0]), 1,
+            code, 1.0, p.data_ptr(), stream), "test.norm")
+    max_norm = 1e9 if case == "below" else 1e-3
+    before = store.clone()
+    table = (_native.pointer_array([p.data_ptr() for p in partials]), _native.int64_array(counts),
+             _native.double_array([1.0] * len(counts)), len(counts), max_norm)
+    outs = [torch.full((4,), 9.0, dtype=torch.float64, device=device) for _ in range(2)]
+
+    def pointers(o):
+        p = o.data_ptr()
+        return p, p + 8, p + 24, p + 16, p + 28, stream
+
+    ptrs, numels = _native.pointer_array([g.data_ptr() for g in grads]), _native.int64_array(sizes)
+    _native.check(lib.hbt_grad_norm_finalize_parts(*table, *pointers(outs[0])), "test.finalize")
+    _native.check(lib.hbt_scale_inplace(ptrs, numels, len(sizes), code, 1.0, outs[0].data_ptr() + 24, stream),
+                  "test.scale")
+    expected = store.clone()
+    store.copy_(before)
+    _native.check(lib.hbt_grad_norm_clip(*table, ptrs, numels, len(sizes), code, *pointers(outs[1])), "test.clip")
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    assert torch.equal(outs[0].view(torch.int64), outs[1].view(torch.int64))
+    assert torch.equal(store.view(bits), expected.view(bits))
+    if case == "below":
+        assert torch.equal(store.view(bits), before.view(bits))
+
+
+@pytest.mark.parametrize("n", [_native.CLIP_MAX_ELEMENTS, _native.CLIP_MAX_ELEMENTS + 1])
+def test_clip_on_both_sides_of_the_one_launch_limit(device, n):
+    """Optimizers whose gradients just fit the one-launch clip, and just do not: the norm, the
+    clipped gradient, its version counter and a following step are the same reference's."""
+    gen = torch.Generator(device=device).manual_seed(3)
+    param = torch.nn.Parameter(torch.randn(n, device=device, generator=gen) * 0.02)
+    grad = torch.randn(n, device=device, generator=gen)
+    param.grad = grad.clone()
+    opt = ShardedOptimizer([param], OptimizerConfig(learning_rate=1e-3), norm_group=GroupHandle.trivial(), device=device)
+    version = param.grad._version
+    norm = opt.clip_grad_norm(0.5)
+    ref = grad.double().square().sum().sqrt()
+    assert abs(float(norm) - float(ref)) <= 1e-12 * float(ref)
+    mul = float(np.float32(0.5 / (float(norm) + 1e-6)))
+    assert torch.equal(param.grad, grad * mul) and param.grad._version > version
+    assert int(opt.last_nonfinite_flag().item()) == 0
+    opt.step()
+    assert float(opt.clip_grad_norm(10.0)) == pytest.approx(0.5, rel=1e-5)
