@@ -720,10 +720,12 @@ struct ShareRanks {
     const uint8_t* g[HBT_MAX_LOCAL_RANKS];
 };
 // The no_sync accumulator rows of the reduction that ends the accumulation: row q holds
-// rank q's accumulated gradient over this rank's slice, in the reduce dtype.
+// rank q's accumulated gradient over this rank's slice, in the reduce dtype, or, after one
+// micro-batch, that micro-batch's gradient itself in its own dtype.
 struct ShareAcc {
     const uint8_t* a[HBT_MAX_LOCAL_RANKS];
 };
+enum ShareRows : int { kNoRows, kReduceRows, kInputRows };
 
 constexpr int kShareBlock = 64;
 constexpr int64_t kShareTile = int64_t(kShareBlock) * 4;  // 256 elements, one wave
@@ -763,7 +765,9 @@ constexpr int kShareIssue = 2;
 constexpr int64_t kShareBurstTiles = 8192;
 // With the accumulator rows (kAcc) each rank is two loads, its gradient and its row;
 // waiting after every rank's pair streamed fastest (against every two, four or eight
-// ranks, or all gradients before the rows).
+// ranks, or all gradients before the rows).  Rows held in the input dtype after a single
+// micro-batch are half the bytes: 5 bf16 ranks of 24.9 M elements 147 us over fp32 rows,
+// 97 us over held ones (598 MB).
 constexpr int kShareAccIssue = 1;
 
 // Where tile t's sum is stored among a launch's `tiles` tile sums.  Workgroup b owns
@@ -849,27 +853,30 @@ __device__ __forceinline__ float stored(float x) {
     return round_to<RD>(x);
 }
 
-// Rank q's element in the reduce dtype: the gradient cast to RD and, when kAcc, added to
+// Rank q's element in the reduce dtype: the gradient cast to RD and, when kAdd, added to
 // the accumulated one as the reference's final no_sync step adds them before reducing,
 // formed exactly as accumulate_kernel forms and stores R(acc + R(grad)), so the fused
 // reduction equals an accumulate launch followed by a reduction of the rows bit for bit,
 // NaNs included.
-template <int ID, int RD, bool kAcc>
+template <int ID, int RD, bool kAdd>
 __device__ __forceinline__ float share_input(float g, float a) {
     const float x = share_cast<ID, RD>(g);
-    if constexpr (kAcc) return stored<RD>(a + x);
+    if constexpr (kAdd) return stored<RD>(a + x);
     return x;
 }
 
 // One 256-element tile of the local share, run by the 64 lanes of one wave (`lane` is
 // this thread's lane): writes the tile's outputs and returns this lane's part of the tile's
 // squared norm.
-template <int ID, int kG, bool kRecip, int RD, int OD, bool kAcc>
+template <int ID, int kG, bool kRecip, int RD, int OD, ShareRows kRows>
 __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const ShareAcc& accs, int32_t group_size,
                                              int64_t offset, int64_t shard_numel, int64_t valid_numel, float divisor,
                                              float recip, int32_t burst, void* __restrict__ out, int64_t tile,
                                              int lane) {
     constexpr int64_t IB = bytes_of<ID>();
+    constexpr bool kAcc = kRows != kNoRows;
+    constexpr int AD = kRows == kInputRows ? ID : RD;  // the rows' dtype
+    static_assert(kRows != kInputRows || RD == F32, "a row in the input dtype widens exactly");
     const int64_t base = tile * kShareTile;
     double acc = 0.0;
     if (base < valid_numel && valid_numel >= kShareTile) {
@@ -888,7 +895,7 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
 #pragma unroll
             for (int q = 0; q < kG; ++q) {
                 load_vec<ID, 4>(ranks.g[q] + offset * IB, e, x[q]);
-                if constexpr (kAcc) load_vec<RD, 4>(accs.a[q], e, a[q]);
+                if constexpr (kAcc) load_vec<AD, 4>(accs.a[q], e, a[q]);
                 if ((q + 1) % (kAcc ? kShareAccIssue : kShareIssue) == 0 && q + 1 < kG && !burst) wait_vmem();
             }
 #pragma unroll
@@ -906,7 +913,7 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
             float a[2][4] = {};
             const auto load = [&](int32_t q, int slot) {
                 load_vec<ID, 4>(ranks.g[q] + offset * IB, e, x[slot]);
-                if constexpr (kAcc) load_vec<RD, 4>(accs.a[q], e, a[slot]);
+                if constexpr (kAcc) load_vec<AD, 4>(accs.a[q], e, a[slot]);
             };
             const auto term = [&](int slot, int c) {
                 return round_to<RD>(share_div<kRecip>(share_input<ID, RD, kAcc>(x[slot][c], a[slot][c]), divisor, recip));
@@ -955,11 +962,11 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
         for (int64_t e = base + lane; e < end; e += kShareBlock) {
             float v = 0.0f;
             if (e < valid_numel) {
-                const float a0 = kAcc ? load_one<RD>(accs.a[0], e) : 0.0f;
+                const float a0 = kAcc ? load_one<AD>(accs.a[0], e) : 0.0f;
                 v = round_to<RD>(share_div<kRecip>(share_input<ID, RD, kAcc>(load_one<ID>(ranks.g[0], offset + e), a0),
                                                    divisor, recip));
                 for (int32_t q = 1; q < group_size; ++q) {
-                    const float aq = kAcc ? load_one<RD>(accs.a[q], e) : 0.0f;
+                    const float aq = kAcc ? load_one<AD>(accs.a[q], e) : 0.0f;
                     const float x = share_input<ID, RD, kAcc>(load_one<ID>(ranks.g[q], offset + e), aq);
                     v = round_to<RD>(v + round_to<RD>(share_div<kRecip>(x, divisor, recip)));
                 }
@@ -972,13 +979,13 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
     return acc;
 }
 
-template <int ID, int kG, bool kRecip, int RD, int OD, bool kAcc = false>
+template <int ID, int kG, bool kRecip, int RD, int OD, ShareRows kRows = kNoRows>
 __global__ __launch_bounds__(kShareBlock) void local_share_tiles_kernel(
     ShareRanks ranks, ShareAcc accs, int32_t group_size, int64_t offset, int64_t shard_numel, int64_t valid_numel,
     float divisor, float recip, int32_t burst, void* __restrict__ out, double* __restrict__ tile_sums,
     int64_t block_base) {
     const int64_t tile = block_base + blockIdx.x;
-    double acc = share_tile<ID, kG, kRecip, RD, OD, kAcc>(ranks, accs, group_size, offset, shard_numel, valid_numel,
+    double acc = share_tile<ID, kG, kRecip, RD, OD, kRows>(ranks, accs, group_size, offset, shard_numel, valid_numel,
                                                           divisor, recip, burst, out, tile,
                                                           static_cast<int>(threadIdx.x));
     if (tile_sums == nullptr) return;
@@ -1005,7 +1012,7 @@ __global__ __launch_bounds__(kSmallShareTiles * kShareBlock) void local_share_sm
     const int wave = static_cast<int>(threadIdx.x) / kShareBlock;  // the launch has one wave per tile
     const int lane = static_cast<int>(threadIdx.x) % kShareBlock;
     const ShareAcc none{};
-    const double s = wave_sum(share_tile<ID, kG, kRecip, RD, OD, false>(
+    const double s = wave_sum(share_tile<ID, kG, kRecip, RD, OD, kNoRows>(
         ranks, none, group_size, offset, shard_numel, valid_numel, divisor, recip, 1, out, wave, lane));
     if (lane == 0) sums[wave] = s;
     __syncthreads();
@@ -1671,6 +1678,10 @@ __global__ __launch_bounds__(kNormBlock) void sqnorm_f64_kernel(NormTable tab, d
 // acc = R(acc + R(grad)), R rounding to the accumulator's dtype (the reduce dtype): the
 // gradient's cast to that dtype (Tensor.to) and one addition computed in fp32 and
 // rounded once (add_).  kAssign writes R(grad) instead: the first micro-batch's clone.
+// kHeld takes the first micro-batch from where it is held in its own 2-byte dtype and
+// writes an fp32 acc = held + grad: a bf16 or fp16 value widens exactly, so the sum is the
+// one over its fp32 copy, bit for bit, and neither that copy's write nor its read is made.
+// Bound by HBM: 8 bytes an element so, 10 where acc is read and written in fp32.
 // The scale kernel's shape: half-wave workgroups, two 4-element vectors per lane,
 // 256 accumulator elements per workgroup.
 constexpr int kAccumBlock = 32;  // half-wave workgroups, two 4-element vectors per lane
@@ -1679,13 +1690,14 @@ constexpr int64_t kAccumTile = int64_t(kAccumBlock) * 2 * 4;
 struct AccumTable {
     void* acc[kMaxT];
     const void* grad[kMaxT];
+    const void* held[kMaxT];
     int64_t n[kMaxT];
     int64_t first_block[kMaxT + 1];
     int32_t count;
 };
 
 // GD: the gradient's dtype; AD: the accumulator's.
-template <int GD, int AD, bool kAssign>
+template <int GD, int AD, bool kAssign, bool kHeld = false>
 __global__ __launch_bounds__(kAccumBlock) void accumulate_kernel(AccumTable tab, int64_t block_base) {
     const int64_t block = block_base + blockIdx.x;
     const int t = owning_tensor(tab.first_block, tab.count, block);
@@ -1693,6 +1705,9 @@ __global__ __launch_bounds__(kAccumBlock) void accumulate_kernel(AccumTable tab,
     const int64_t n = tab.n[t];
     void* acc = tab.acc[t];
     const void* grad = tab.grad[t];
+    static_assert(!kHeld || (AD == F32 && !kAssign), "a held gradient widens exactly into an fp32 sum");
+    constexpr int SD = kHeld ? GD : AD;  // what is added to
+    const void* sum = kHeld ? tab.held[t] : acc;
     if (base + kAccumTile <= n) {
         float a[2][4], g[2][4];
 #pragma unroll
@@ -1703,7 +1718,7 @@ __global__ __launch_bounds__(kAccumBlock) void accumulate_kernel(AccumTable tab,
         }
         if constexpr (!kAssign) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u) load_vec<AD, 4>(acc, base + (int64_t(u) * kAccumBlock + threadIdx.x) * 4, a[u]);
+            for (int u = 0; u < 2; ++u) load_vec<SD, 4>(sum, base + (int64_t(u) * kAccumBlock + threadIdx.x) * 4, a[u]);
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -1720,7 +1735,7 @@ __global__ __launch_bounds__(kAccumBlock) void accumulate_kernel(AccumTable tab,
     for (int u = 0; u < 2; ++u) {
         const int64_t e = base + (int64_t(u) * kAccumBlock + threadIdx.x) * 4;
         load_upto<GD, 4>(grad, e, n, g[u]);
-        if constexpr (!kAssign) load_upto<AD, 4>(acc, e, n, a[u]);
+        if constexpr (!kAssign) load_upto<SD, 4>(sum, e, n, a[u]);
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -2061,11 +2076,12 @@ int32_t noalloc_scratch(const char* who, double** out) {
 
 // Shared by hbt_grad_local_share, hbt_grad_local_share_sqnorm (tile_scratch and
 // partials null for the former) and hbt_grad_local_share_accumulated (accumulators
-// non-null: row q, in the reduce dtype, is added to rank q's gradient first).
+// non-null: row q, in the reduce dtype, is added to rank q's gradient first) and
+// hbt_grad_local_share_held (the rows in the input dtype).
 int32_t local_share(const char* who, const void* const* rank_grads, int32_t group_size, int32_t rank,
                     int64_t shard_numel, int64_t valid_numel, int32_t in_dtype, int32_t reduce_dtype,
                     float divisor, int32_t out_dtype, void* out, double* partials, double* tile_scratch,
-                    hipStream_t st, const void* const* accumulators = nullptr) {
+                    hipStream_t st, const void* const* accumulators = nullptr, bool held = false) {
     if (rank_grads == nullptr || out == nullptr || group_size < 1 || group_size > HBT_MAX_LOCAL_RANKS ||
         rank < 0 || rank >= group_size || shard_numel < 0 || valid_numel < 0 || valid_numel > shard_numel) {
         set_error("%s: bad arguments (group_size=%d rank=%d shard=%lld valid=%lld)", who, group_size, rank,
@@ -2090,6 +2106,11 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
     if (with_acc && f64) {
         set_error("%s: an accumulated reduction in reduce dtype F64 is not fused; add the last micro-batch "
                   "with hbt_grad_accumulate and reduce the accumulator", who);
+        return HBT_ERR_UNSUPPORTED;
+    }
+    if (held && (reduce_dtype != F32 || in_dtype == F32)) {
+        set_error("%s: rows held in the input dtype are 2-byte gradients reduced in F32 (input %d, reduce %d)", who,
+                  in_dtype, reduce_dtype);
         return HBT_ERR_UNSUPPORTED;
     }
     ShareRanks ranks{};
@@ -2124,12 +2145,16 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
         if (small)                                                                                             \
             local_share_small_kernel<ID, G, R, RD, OD><<<dim3(1), dim3(small_threads), 0, st>>>(                 \
                 ranks, group_size, offset, shard_numel, valid_numel, divisor, recip, out, partials);    \
+        else if (held)                                                                                         \
+            local_share_tiles_kernel<ID, G, R, RD, OD, (RD == F32 && ID != F32 ? kInputRows : kReduceRows)>      \
+                <<<grid, kShareBlock, 0, st>>>(ranks, accs, group_size, offset, shard_numel, valid_numel,        \
+                                               divisor, recip, burst, out, tile_scratch, first);               \
         else if (with_acc)                                                                                     \
-            local_share_tiles_kernel<ID, G, R, RD, OD, true><<<grid, kShareBlock, 0, st>>>(                      \
+            local_share_tiles_kernel<ID, G, R, RD, OD, kReduceRows><<<grid, kShareBlock, 0, st>>>(               \
                 ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
                 tile_scratch, first);                                                                          \
         else                                                                                                   \
-            local_share_tiles_kernel<ID, G, R, RD, OD, false><<<grid, kShareBlock, 0, st>>>(                     \
+            local_share_tiles_kernel<ID, G, R, RD, OD, kNoRows><<<grid, kShareBlock, 0, st>>>(                   \
                 ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
                 tile_scratch, first);                                                                          \
     } while (0)
@@ -2562,36 +2587,40 @@ int32_t hbt_scale_inplace(void* const* tensors, const int64_t* numels, int32_t c
     });
 }
 
-int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads, const int64_t* numels,
-                            int32_t count, int32_t acc_dtype, int32_t grad_dtype, int32_t flags, void* stream) {
+// Both forms of the accumulation; held is null for hbt_grad_accumulate.
+static int32_t accumulate(const char* who, void* const* accumulators, const void* const* held,
+                          const void* const* grads, const int64_t* numels, int32_t count, int32_t acc_dtype,
+                          int32_t grad_dtype, int32_t flags, void* stream) {
     clear_error();
     if (count < 0 || count > kMaxT ||
         (count > 0 && (accumulators == nullptr || grads == nullptr || numels == nullptr))) {
-        set_error("hbt_grad_accumulate: bad table (count=%d)", count);
+        set_error("%s: bad table (count=%d)", who, count);
         return HBT_ERR_INVALID_ARGUMENT;
     }
     const auto float_code = [](int32_t d) { return d == F32 || d == BF16 || d == F16; };
     const bool f64 = acc_dtype == HBT_DTYPE_F64;
     if (!(float_code(acc_dtype) || f64) || !(float_code(grad_dtype) || (f64 && grad_dtype == HBT_DTYPE_F64))) {
-        set_error("hbt_grad_accumulate: dtypes (accumulator %d, gradient %d) must be F32, BF16 or F16 "
+        set_error("%s: dtypes (accumulator %d, gradient %d) must be F32, BF16 or F16 "
                   "(or an F64 accumulator, whose gradient may also be F64)",
-                  acc_dtype, grad_dtype);
+                  who, acc_dtype, grad_dtype);
         return HBT_ERR_INVALID_ARGUMENT;
     }
     if ((flags & ~HBT_ACCUMULATE_ASSIGN) != 0) {
-        set_error("hbt_grad_accumulate: unknown flags 0x%x", static_cast<unsigned>(flags));
+        set_error("%s: unknown flags 0x%x", who, static_cast<unsigned>(flags));
         return HBT_ERR_INVALID_ARGUMENT;
     }
     AccumTable tab{};
     tab.count = count;
     int64_t blocks = 0;
     for (int i = 0; i < count; ++i) {
-        if (numels[i] < 0 || (numels[i] > 0 && (accumulators[i] == nullptr || grads[i] == nullptr))) {
-            set_error("hbt_grad_accumulate: pair %d has a bad pointer or numel", i);
+        if (numels[i] < 0 || (numels[i] > 0 && (accumulators[i] == nullptr || grads[i] == nullptr ||
+                                                (held != nullptr && held[i] == nullptr)))) {
+            set_error("%s: pair %d has a bad pointer or numel", who, i);
             return HBT_ERR_INVALID_ARGUMENT;
         }
         tab.acc[i] = accumulators[i];
         tab.grad[i] = grads[i];
+        tab.held[i] = held == nullptr ? nullptr : held[i];
         tab.n[i] = numels[i];
         tab.first_block[i] = blocks;
         blocks += (numels[i] + kAccumTile - 1) / kAccumTile;
@@ -2600,7 +2629,7 @@ int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads,
     for (int i = count + 1; i <= kMaxT; ++i) tab.first_block[i] = blocks;
     hipStream_t st = as_stream(stream);
     const bool assign = (flags & HBT_ACCUMULATE_ASSIGN) != 0;
-    return launch_sliced("hbt_grad_accumulate", blocks, kAccumBlock, [&](int64_t first, dim3 grid) {
+    return launch_sliced(who, blocks, kAccumBlock, [&](int64_t first, dim3 grid) {
 #define HBT_ACC(GD, AD)                                                                        \
     do {                                                                                       \
         if (assign) accumulate_kernel<GD, AD, true><<<grid, kAccumBlock, 0, st>>>(tab, first); \
@@ -2617,7 +2646,10 @@ int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads,
         if (assign) accumulate_f64_kernel<SB, SH, true><<<grid, kAccumBlock, 0, st>>>(tab, first); \
         else accumulate_f64_kernel<SB, SH, false><<<grid, kAccumBlock, 0, st>>>(tab, first);       \
     } while (0)
-        if (f64) {
+        if (held != nullptr) {
+            if (grad_dtype == BF16) accumulate_kernel<BF16, F32, false, true><<<grid, kAccumBlock, 0, st>>>(tab, first);
+            else accumulate_kernel<F16, F32, false, true><<<grid, kAccumBlock, 0, st>>>(tab, first);
+        } else if (f64) {
             if (grad_dtype == HBT_DTYPE_F64) HBT_ACC64(8, false);
             else if (grad_dtype == F32) HBT_ACC64(4, false);
             else if (grad_dtype == BF16) HBT_ACC64(2, false);
@@ -2633,6 +2665,26 @@ int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads,
 #undef HBT_ACC64
 #undef HBT_ACC
     });
+}
+
+int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads, const int64_t* numels,
+                            int32_t count, int32_t acc_dtype, int32_t grad_dtype, int32_t flags, void* stream) {
+    return accumulate("hbt_grad_accumulate", accumulators, nullptr, grads, numels, count, acc_dtype, grad_dtype, flags,
+                      stream);
+}
+
+int32_t hbt_grad_accumulate_held(void* const* accumulators, const void* const* held, const void* const* grads,
+                                 const int64_t* numels, int32_t count, int32_t dtype, void* stream) {
+    clear_error();
+    if (held == nullptr && count > 0) {
+        set_error("hbt_grad_accumulate_held: null table of held gradients");
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    if (dtype != BF16 && dtype != F16) {
+        set_error("hbt_grad_accumulate_held: held gradients of dtype %d are not BF16 or F16", dtype);
+        return HBT_ERR_UNSUPPORTED;
+    }
+    return accumulate("hbt_grad_accumulate_held", accumulators, held, grads, numels, count, F32, dtype, 0, stream);
 }
 
 int32_t hbt_grad_local_share(const void* const* rank_grads, int32_t group_size, int32_t rank,
@@ -2672,6 +2724,23 @@ int32_t hbt_grad_local_share_accumulated(const void* const* rank_grads, const vo
     return local_share("hbt_grad_local_share_accumulated", rank_grads, group_size, rank, shard_numel, valid_numel,
                        in_dtype, reduce_dtype, divisor, out_dtype, out, partials, tile_scratch, as_stream(stream),
                        accumulators);
+}
+
+int32_t hbt_grad_local_share_held(const void* const* rank_grads, const void* const* held, int32_t group_size,
+                                  int32_t rank, int64_t shard_numel, int64_t valid_numel, int32_t in_dtype,
+                                  int32_t reduce_dtype, float divisor, int32_t out_dtype, void* out, double* partials,
+                                  double* tile_scratch, void* stream) {
+    clear_error();
+    if (held == nullptr) {
+        set_error("hbt_grad_local_share_held: null table of held gradients");
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    if ((partials == nullptr) != (tile_scratch == nullptr)) {
+        set_error("hbt_grad_local_share_held: partials and tile scratch must both be given or both null");
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    return local_share("hbt_grad_local_share_held", rank_grads, group_size, rank, shard_numel, valid_numel, in_dtype,
+                       reduce_dtype, divisor, out_dtype, out, partials, tile_scratch, as_stream(stream), held, true);
 }
 
 static int32_t sgd_step_impl(const char* who, void* const* params, void* const* grads, void* const* momentum_buffers,

@@ -68,7 +68,7 @@ __all__ = [
     "stream_of",
 ]
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 MAX_TENSORS_PER_LAUNCH = 16
 MAX_LOCAL_RANKS = 64
 MAX_NORM_PARTS = 128
@@ -185,6 +185,11 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
         (_ptr_array, _ptr_array, _c_i32, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p,
          _c_void_p, _c_void_p, _c_void_p),
     ),
+    "hbt_grad_local_share_held": (
+        _c_i32,
+        (_ptr_array, _ptr_array, _c_i32, _c_i32, _c_i64, _c_i64, _c_i32, _c_i32, _c_f32, _c_i32, _c_void_p,
+         _c_void_p, _c_void_p, _c_void_p),
+    ),
     "hbt_scale_inplace": (
         _c_i32,
         (_ptr_array, _i64_array, _c_i32, _c_i32, _c_f32, _c_void_p, _c_void_p),
@@ -196,6 +201,10 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
     "hbt_grad_accumulate": (
         _c_i32,
         (_ptr_array, _ptr_array, _i64_array, _c_i32, _c_i32, _c_i32, _c_i32, _c_void_p),
+    ),
+    "hbt_grad_accumulate_held": (
+        _c_i32,
+        (_ptr_array, _ptr_array, _ptr_array, _i64_array, _c_i32, _c_i32, _c_void_p),
     ),
     "hbt_adamw_step_f64": (
         _c_i32,

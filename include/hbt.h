@@ -401,6 +401,22 @@ int32_t hbt_grad_local_share_accumulated(const void* const* rank_grads, const vo
                                          void* out, double* partials, double* tile_scratch, void* stream);
 
 /* ------------------------------------------------------------------------------
+ * The same reduction after a single accumulated micro-batch, whose gradients are held in
+ * their own dtype.
+ *
+ * Replaces: the final micro-batch of FlatParamHandle.reduce_scatter_gradient under
+ *   no_sync (parallel/fsdp.py:747-769) where one was accumulated before it.
+ * It is hbt_grad_local_share_accumulated with held[q] (row q of the rows that
+ * hbt_copy_rows copied them into) in in_dtype, BF16 or F16, and reduce_dtype F32; others
+ * return HBT_ERR_UNSUPPORTED.  A 2-byte value widens exactly, so the outputs are bitwise
+ * those over rows widened to F32, which take twice the bytes to write and to read.
+ * ---------------------------------------------------------------------------- */
+int32_t hbt_grad_local_share_held(const void* const* rank_grads, const void* const* held, int32_t group_size,
+                                  int32_t rank, int64_t shard_numel, int64_t valid_numel, int32_t in_dtype,
+                                  int32_t reduce_dtype, float divisor, int32_t out_dtype, void* out, double* partials,
+                                  double* tile_scratch, void* stream);
+
+/* ------------------------------------------------------------------------------
  * FSDP no_sync gradient accumulation over up to HBT_MAX_TENSORS_PER_LAUNCH
  * (accumulator, gradient) pairs.
  *
@@ -422,6 +438,18 @@ int32_t hbt_grad_local_share_accumulated(const void* const* rank_grads, const vo
 #define HBT_ACCUMULATE_ASSIGN 1
 int32_t hbt_grad_accumulate(void* const* accumulators, const void* const* grads, const int64_t* numels,
                             int32_t count, int32_t acc_dtype, int32_t grad_dtype, int32_t flags, void* stream);
+
+/* ------------------------------------------------------------------------------
+ * The second micro-batch over held first ones.
+ *
+ * Replaces: accumulator.add_(grad) of the accumulate branch of
+ *   FlatParamHandle.reduce_scatter_gradient (parallel/fsdp.py:738-749).
+ * F32 accumulators[k] = held[k] + grads[k], both numels[k] elements of `dtype` (BF16 or F16; others return HBT_ERR_UNSUPPORTED):
+ * bitwise hbt_grad_accumulate of the gradients over F32 copies of the held ones.  The
+ * accumulators overlap neither.
+ * ---------------------------------------------------------------------------- */
+int32_t hbt_grad_accumulate_held(void* const* accumulators, const void* const* held, const void* const* grads,
+                                 const int64_t* numels, int32_t count, int32_t dtype, void* stream);
 
 /* ------------------------------------------------------------------------------
  * In-place gradient scaling: x = (x * unscale) * (*grad_mul), each product rounded to

@@ -302,6 +302,56 @@ def test_local_share_accumulated_is_accumulate_then_share(device, group, in_dtyp
         assert f64 == -2 and b"F64" in lib.hbt_last_error()  # HBT_ERR_UNSUPPORTED
 
 
+@pytest.mark.parametrize("group", [1, 2, 5, 8, 9])
+@pytest.mark.parametrize("in_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("master", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shard, off", [(1, 0), (255, 1), (4096, 0), (3 * 32768 + 301, 1)])
+def test_held_rows_are_their_widened_copies(device, group, in_dtype, master, shard, off):
+    """A first micro-batch held in its own dtype: ``hbt_grad_local_share_held`` and
+    ``hbt_grad_accumulate_held`` are bitwise ``hbt_grad_local_share_accumulated`` and
+    ``hbt_grad_accumulate`` over float32 copies of the held rows, NaN, infinities, -0.0
+    and subnormals included."""
+    lib = _native.library()
+    gen = torch.Generator(device=device).manual_seed(shard + group)
+    valid = max(1, shard - 77)
+    rank = group - 1
+    grads = [(torch.randn(group * shard + off, device=device, generator=gen) * 0.3).to(in_dtype)[off:]
+             for _ in range(group)]
+    held = [(torch.randn(shard + off, device=device, generator=gen) * 0.7).to(in_dtype)[off:] for _ in range(group)]
+    for e, value in enumerate((float("nan"), float("inf"), -float("inf"), -0.0, 1e-7, 6e4)):
+        if e < shard:
+            held[0][e] = value
+    wide = [h.float() for h in held]
+    code_in, code_out = _native.dtype_code(in_dtype), _native.dtype_code(master)
+    stream = ctypes.c_void_p(_native.stream_of(device))
+    count = -(-valid // 32768) + -(-(shard - valid) // 32768)
+    tiles = -(-shard // 256)
+
+    def pointers(tensors, extra=0):
+        return _native.pointer_array([t.data_ptr() + extra for t in tensors])
+
+    def reduced(call, rows):
+        out = torch.empty(shard, dtype=master, device=device)
+        partials = torch.zeros(count + 1, dtype=torch.float64, device=device)
+        scratch = torch.empty(tiles, dtype=torch.float64, device=device)
+        _native.check(call(pointers(grads), pointers(rows), group, rank, shard, valid, code_in, 0, float(group),
+                           code_out, out.data_ptr(), partials.data_ptr(), scratch.data_ptr(), stream), "test.share")
+        return _bits(out), partials.cpu().numpy().view(np.int64)
+
+    expect, got = reduced(lib.hbt_grad_local_share_accumulated, wide), reduced(lib.hbt_grad_local_share_held, held)
+    assert np.array_equal(expect[0], got[0]) and np.array_equal(expect[1], got[1])
+
+    sums = [torch.empty(shard, device=device) for _ in range(group)]
+    sizes = _native.int64_array([shard] * group)
+    offset = rank * shard * in_dtype.itemsize
+    _native.check(lib.hbt_grad_accumulate_held(pointers(sums), pointers(held), pointers(grads, offset), sizes, group,
+                                               code_in, stream), "test.accumulate_held")
+    _native.check(lib.hbt_grad_accumulate(pointers(wide), pointers(grads, offset), sizes, group, 0, code_in, 0, stream),
+                  "test.accumulate")
+    for a, b in zip(wide, sums):
+        assert np.array_equal(_bits(a), _bits(b))
+
+
 _SMALL_DTYPES = [(torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.float32, torch.float32),
                  (torch.bfloat16, torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16, torch.float32),
                  (torch.float32, torch.float32, torch.bfloat16)]

@@ -368,6 +368,32 @@ def test_no_sync_accumulation_matches_oracle(device, group, in_dtype, micro, red
         assert h.reduction_count == 2
 
 
+@pytest.mark.parametrize("dtypes", [(torch.bfloat16, torch.float32), (torch.float16, torch.bfloat16),
+                                    (torch.bfloat16, torch.float16, torch.float16),
+                                    (torch.bfloat16, torch.bfloat16, torch.float32)])
+def test_no_sync_accumulation_over_changing_dtypes(device, dtypes):
+    """Micro-batches of different dtypes, the first of them 2-byte and held in its own
+    dtype: bitwise the oracle's float32 accumulation, and the held rows are the gradients
+    of their call, not of a later one that reuses the buffer."""
+    group = 2
+    handles = _mp_handles(group, device, "float32")
+    padded, shard = handles[0].padded_numel, handles[0].shard_numel
+    gen = torch.Generator(device=device).manual_seed(len(dtypes))
+    grads = [[(torch.randn(padded, device=device, generator=gen) * 1e-2).to(d) for _ in range(group)] for d in dtypes]
+    totals = [oracle.no_sync_accumulate([m[q].float().cpu().numpy() for m in grads], "float32") for q in range(group)]
+    for rank, h in enumerate(handles):
+        h.set_accumulate_without_reduction(True)
+        for batch in grads[:-1]:
+            passed = [g.clone() for g in batch]
+            assert h.reduce_scatter_gradient(passed[rank], peer_grads=passed) is None
+            for g in passed:
+                g.zero_()
+        h.set_accumulate_without_reduction(False)
+        out = h.reduce_scatter_gradient(grads[-1][rank], peer_grads=grads[-1])
+        expect = oracle.local_share(totals, rank, shard, max(0, min(shard, 1857 - rank * shard)), float(group), "float32")
+        assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32)), rank
+
+
 def test_load_local_pieces_round_trip(device):
     named, originals, handles = _handles(MLP_23_32_32_1, 4, device)
     state = {name: torch.randn_like(orig) for (name, _), orig in zip(named, originals)}

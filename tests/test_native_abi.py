@@ -124,6 +124,14 @@ def test_invalid_arguments_are_rejected_before_any_launch():
     assert lib.hbt_copy_chunk_elems(1, 2) == 512 and lib.hbt_copy_chunk_elems(3, 3) == 128
     assert lib.hbt_grad_accumulate(None, None, None, 0, 0, 0, 2, None) == -1  # unknown flag
     assert lib.hbt_grad_accumulate(None, None, None, 1, 0, 0, 0, None) == -1  # null table
+    # rows held in the input dtype: 2-byte gradients reduced in float32 only
+    one = _native.pointer_array([4096])
+    assert lib.hbt_grad_accumulate_held(None, None, None, None, 0, 1, None) == 0  # empty table
+    assert lib.hbt_grad_accumulate_held(one, None, one, _native.int64_array([1]), 1, 1, None) == -1
+    assert lib.hbt_grad_accumulate_held(one, one, one, _native.int64_array([1]), 1, 0, None) == -2
+    for in_dtype, reduce_dtype in ((0, 0), (1, 1), (2, 3)):
+        assert lib.hbt_grad_local_share_held(one, one, 1, 0, 1, 1, in_dtype, reduce_dtype, 1.0, 0, fake, None, None,
+                                             None) == -2
     assert lib.hbt_grad_norm_finalize(None, 5, 1.0, None, None, None, None, None, None) == -1
     # float64 steps and scaling: table and flag checks on the host
     assert lib.hbt_adamw_step_f64(None, None, None, None, None, 99, 1.0, None,
