@@ -64,6 +64,21 @@ int32_t launch_sliced(const char* who, int64_t blocks, int threads, Launch&& lau
     return HBT_OK;
 }
 
+// ---- XCD order -----------------------------------------------------------------------
+// The dispatcher deals consecutive workgroups to the 8 XCDs in turn, each with its own L2.
+// Where workgroup b moves piece b of a stream whose pieces do not start on cache lines, the
+// line that two pieces share is fetched by two XCDs.  xcd_order gives kRun consecutive
+// pieces to workgroups of one XCD, close in time, so all but one such line in kRun comes
+// from the L2: a bijection of [0, count), the identity past the last whole 8 * kRun pieces.
+template <int kRun>
+__device__ __forceinline__ int64_t xcd_order(int64_t b, int64_t count) {
+    constexpr int64_t kGroup = 8 * kRun;
+    const int64_t group = b / kGroup * kGroup;
+    if (group + kGroup > count) return b;
+    const uint32_t r = static_cast<uint32_t>(b - group);
+    return group + (r % 8u) * kRun + r / 8u;
+}
+
 // ---- dtype helpers -------------------------------------------------------------------
 inline int dtype_size(int32_t dtype) {
     switch (dtype) {

@@ -769,6 +769,15 @@ constexpr int64_t kShareBurstTiles = 8192;
 // micro-batch are half the bytes: 5 bf16 ranks of 24.9 M elements 147 us over fp32 rows,
 // 97 us over held ones (598 MB).
 constexpr int kShareAccIssue = 1;
+// Rows held in the input dtype are narrow loads again and go out two ranks at a time.
+constexpr int kShareHeldIssue = 2;
+// Consecutive tiles that one XCD reduces where a rank's slice does not start on a cache
+// line (xcd_order): each 512 B of bf16 then touches 5 lines, the fifth shared with the next
+// tile.  With one tile and with 8, 16 and 32, and pairs for held rows: 5 bf16 ranks of
+// 24.9 M elements held and reduced 188, 169, 168 and 166 us.  Slices on lines keep the
+// dispatch order, which streams them faster (a Llama-3-8B layer of 8 ranks 88.6 us, 92 us
+// in runs of 4 or 16).
+constexpr int kShareRun = 32;
 
 // Where tile t's sum is stored among a launch's `tiles` tile sums.  Workgroup b owns
 // tile b, and the dispatcher deals consecutive workgroups to the 8 XCDs in turn, each
@@ -876,6 +885,7 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
     constexpr int64_t IB = bytes_of<ID>();
     constexpr bool kAcc = kRows != kNoRows;
     constexpr int AD = kRows == kInputRows ? ID : RD;  // the rows' dtype
+    constexpr int kIssue = kRows == kNoRows ? kShareIssue : (kRows == kInputRows ? kShareHeldIssue : kShareAccIssue);
     static_assert(kRows != kInputRows || RD == F32, "a row in the input dtype widens exactly");
     const int64_t base = tile * kShareTile;
     double acc = 0.0;
@@ -896,7 +906,7 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
             for (int q = 0; q < kG; ++q) {
                 load_vec<ID, 4>(ranks.g[q] + offset * IB, e, x[q]);
                 if constexpr (kAcc) load_vec<AD, 4>(accs.a[q], e, a[q]);
-                if ((q + 1) % (kAcc ? kShareAccIssue : kShareIssue) == 0 && q + 1 < kG && !burst) wait_vmem();
+                if ((q + 1) % kIssue == 0 && q + 1 < kG && !burst) wait_vmem();
             }
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -982,15 +992,17 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
 template <int ID, int kG, bool kRecip, int RD, int OD, ShareRows kRows = kNoRows>
 __global__ __launch_bounds__(kShareBlock) void local_share_tiles_kernel(
     ShareRanks ranks, ShareAcc accs, int32_t group_size, int64_t offset, int64_t shard_numel, int64_t valid_numel,
-    float divisor, float recip, int32_t burst, void* __restrict__ out, double* __restrict__ tile_sums,
-    int64_t block_base) {
-    const int64_t tile = block_base + blockIdx.x;
+    float divisor, float recip, int32_t burst, int32_t off_lines, void* __restrict__ out,
+    double* __restrict__ tile_sums, int64_t block_base) {
+    const int64_t tiles = (shard_numel + kShareTile - 1) / kShareTile;
+    int64_t tile = block_base + blockIdx.x;
+    if (off_lines) tile = xcd_order<kShareRun>(tile, tiles);
     double acc = share_tile<ID, kG, kRecip, RD, OD, kRows>(ranks, accs, group_size, offset, shard_numel, valid_numel,
                                                           divisor, recip, burst, out, tile,
                                                           static_cast<int>(threadIdx.x));
     if (tile_sums == nullptr) return;
     acc = wave_sum(acc);
-    if (threadIdx.x == 0) tile_sums[tile_sum_slot(tile, (shard_numel + kShareTile - 1) / kShareTile)] = acc;
+    if (threadIdx.x == 0) tile_sums[off_lines ? tile : tile_sum_slot(tile, tiles)] = acc;
 }
 
 // A shard of at most kSmallShareTiles tiles and its norm partials in one launch: one
@@ -1156,10 +1168,11 @@ __global__ __launch_bounds__(kShareBlock) void local_share_f64_tiles_kernel(
 // Chunk c < valid_chunks: the sum of its kTiles tile sums (those below valid_tiles), lane
 // l adding tiles l, l + 64, ... in order before the butterfly; padding chunks: 0, the
 // square sum of zeros.  `tiles` is the tile count of the launch that wrote the sums
-// (their slots, tile_sum_slot); a chunk's sums lie in 8 runs of kTiles / 8 slots.
+// (their slots, tile_sum_slot, or with in_order their own index: kShareRun tiles of one XCD
+// fill whole lines); a chunk's sums lie in 8 runs of kTiles / 8 slots.
 template <int kTiles>
 __global__ __launch_bounds__(kShareBlock) void tile_sums_to_partials_kernel(
-    const double* __restrict__ tile_sums, int64_t tiles, int64_t valid_tiles, int64_t valid_chunks,
+    const double* __restrict__ tile_sums, int64_t tiles, int64_t valid_tiles, int64_t valid_chunks, int32_t in_order,
     double* __restrict__ partials, int64_t block_base) {
     const int64_t chunk = block_base + blockIdx.x;
     double acc = 0.0;
@@ -1168,7 +1181,7 @@ __global__ __launch_bounds__(kShareBlock) void tile_sums_to_partials_kernel(
 #pragma unroll
         for (int k = 0; k < kTiles / kShareBlock; ++k) {
             const int64_t a = first + int64_t(k) * kShareBlock;
-            if (a < valid_tiles) acc += tile_sums[tile_sum_slot(a, tiles)];
+            if (a < valid_tiles) acc += tile_sums[in_order ? a : tile_sum_slot(a, tiles)];
         }
     }
     acc = wave_sum(acc);
@@ -2116,12 +2129,17 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
     ShareRanks ranks{};
     ShareAcc accs{};
     const int64_t offset = int64_t(rank) * shard_numel;
+    const int elem = dtype_size(in_dtype);
+    constexpr uintptr_t kLine = 128;  // a cache line
+    int32_t off_lines = 0;
     for (int q = 0; q < group_size; ++q) {
         if (rank_grads[q] == nullptr && valid_numel > 0) {
             set_error("%s: rank %d gradient pointer is null", who, q);
             return HBT_ERR_INVALID_ARGUMENT;
         }
         ranks.g[q] = static_cast<const uint8_t*>(rank_grads[q]);
+        const uintptr_t read = reinterpret_cast<uintptr_t>(rank_grads[q]) + static_cast<uintptr_t>(offset * elem);
+        if ((read & (kLine - 1)) != 0) off_lines = 1;
         if (with_acc) {
             if (accumulators[q] == nullptr && valid_numel > 0) {
                 set_error("%s: rank %d accumulator pointer is null", who, q);
@@ -2148,14 +2166,14 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
         else if (held)                                                                                         \
             local_share_tiles_kernel<ID, G, R, RD, OD, (RD == F32 && ID != F32 ? kInputRows : kReduceRows)>      \
                 <<<grid, kShareBlock, 0, st>>>(ranks, accs, group_size, offset, shard_numel, valid_numel,        \
-                                               divisor, recip, burst, out, tile_scratch, first);               \
+                                               divisor, recip, burst, off_lines, out, tile_scratch, first);    \
         else if (with_acc)                                                                                     \
             local_share_tiles_kernel<ID, G, R, RD, OD, kReduceRows><<<grid, kShareBlock, 0, st>>>(               \
-                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
+                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, off_lines, out,    \
                 tile_scratch, first);                                                                          \
         else                                                                                                   \
             local_share_tiles_kernel<ID, G, R, RD, OD, kNoRows><<<grid, kShareBlock, 0, st>>>(                   \
-                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, out,    \
+                ranks, accs, group_size, offset, shard_numel, valid_numel, divisor, recip, burst, off_lines, out,    \
                 tile_scratch, first);                                                                          \
     } while (0)
 // Groups of 1 to 8 ranks have their own instantiations, every rank's load issued before
@@ -2239,17 +2257,18 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
     const int64_t valid_chunks = (valid_numel + chunk - 1) / chunk;
     const int64_t pad_chunks = (shard_numel - valid_numel + chunk - 1) / chunk;
     const int64_t valid_tiles = (valid_numel + kShareTile - 1) / kShareTile;
+    const int32_t in_order = off_lines && !f64;
     return launch_sliced(who, valid_chunks + pad_chunks, kShareBlock, [&](int64_t first, dim3 grid) {
         if (out_dtype == HBT_DTYPE_F64) {
             static_assert(kNormF64Chunk % kShareTile == 0, "a float64 norm chunk is whole tiles");
             tile_sums_to_partials_kernel<static_cast<int>(kNormF64Chunk / kShareTile)><<<grid, kShareBlock, 0, st>>>(
-                tile_scratch, tiles, valid_tiles, valid_chunks, partials, first);
+                tile_scratch, tiles, valid_tiles, valid_chunks, in_order, partials, first);
         } else if (out_dtype == F32) {
             tile_sums_to_partials_kernel<tiles_per_norm_chunk<F32>()><<<grid, kShareBlock, 0, st>>>(
-                tile_scratch, tiles, valid_tiles, valid_chunks, partials, first);
+                tile_scratch, tiles, valid_tiles, valid_chunks, in_order, partials, first);
         } else {
             tile_sums_to_partials_kernel<tiles_per_norm_chunk<BF16>()><<<grid, kShareBlock, 0, st>>>(
-                tile_scratch, tiles, valid_tiles, valid_chunks, partials, first);
+                tile_scratch, tiles, valid_tiles, valid_chunks, in_order, partials, first);
         }
     });
 }

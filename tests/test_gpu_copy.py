@@ -442,3 +442,27 @@ def test_copy_rows_refuses_what_it_cannot_move(device):
     assert status([(buf.data_ptr(), 0, 4)]) == -1 and status([(ok[0], ok[1], -1)]) == -1
     assert status([ok], src=9) == -1 and status([ok], op=7) == -1
     assert status([ok], src=3, dst=0, op=1) == -2
+
+
+@pytest.mark.parametrize("chunks", [63, 64, 65, 129])
+@pytest.mark.parametrize("src, dst", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                      (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("src_off, dst_off", [(1, 0), (3, 3), (0, 5), (8, 65)])
+def test_records_off_the_destinations_lines(device, chunks, src, dst, src_off, dst_off):
+    """A record whose source and destination lines differ moves its chunks in groups of 64;
+    lengths around a whole number of groups, and a second record that agrees on lines."""
+    codes = _native.dtype_code(src), _native.dtype_code(dst)
+    chunk = int(_native.library().hbt_copy_chunk_elems(*codes))
+    gen = torch.Generator(device=device).manual_seed(chunks)
+    for n in (chunks * chunk - 1, chunks * chunk, chunks * chunk + 7):
+        source = torch.randn(n + src_off + 128, device=device, generator=gen).to(src)
+        target = torch.full((n + dst_off + 9,), 7.0, dtype=dst, device=device)
+        other = torch.zeros(chunk + 3, dtype=dst, device=device)
+        plan = _native.CopyPlan(device)
+        plan.add(source, src_off, target, dst_off, n)
+        plan.add(source, 0, other, 0, chunk + 3)
+        plan.run(src_dtype=src, dst_dtype=dst)
+        expect = torch.full_like(target, 7.0)
+        expect[dst_off : dst_off + n] = source[src_off : src_off + n].to(dst)
+        assert torch.equal(target, expect), n
+        assert torch.equal(other, source[: chunk + 3].to(dst))

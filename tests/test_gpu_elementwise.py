@@ -694,3 +694,34 @@ def test_norm_and_scale_at_the_sizes_kept_for_the_next_pass(device, n):
     _native.check(lib.hbt_scale_inplace(_native.pointer_array([scaled.data_ptr()]), _native.int64_array([n]), 1, 0, 1.0,
                                         mul.data_ptr(), stream), "test.scale")
     assert torch.equal(scaled, x * mul)
+
+
+@pytest.mark.parametrize("shard", [255, 65_536, 65_537, 3 * 65_536 + 257])
+@pytest.mark.parametrize("rows", [False, True])
+def test_local_share_off_cache_lines_is_the_same(device, shard, rows):
+    """Slices that start off a cache line are reduced in another order of tiles (whole and
+    partial groups of 256 tiles): outputs and norm partials are bitwise those of the same
+    values on lines."""
+    lib = _native.library()
+    group = 3
+    gen = torch.Generator(device=device).manual_seed(shard)
+    values = [torch.randn(shard, device=device, generator=gen).bfloat16() for _ in range(group)]
+    accumulated = [torch.randn(shard, device=device, generator=gen) for _ in range(group)]
+    results = []
+    for off in (0, 1, 40):
+        grads = [torch.cat([torch.zeros(off, dtype=torch.bfloat16, device=device), v]) for v in values]
+        out = torch.empty(shard, device=device)
+        partials = torch.zeros(-(-shard // 32768), dtype=torch.float64, device=device)
+        scratch = torch.full((-(-shard // 256),), float("nan"), dtype=torch.float64, device=device)
+        pointers = _native.pointer_array([g.data_ptr() + 2 * off for g in grads])
+        args = (group, 0, shard, shard, 1, 0, 3.0, 0, out.data_ptr(), partials.data_ptr(), scratch.data_ptr(),
+                ctypes.c_void_p(_native.stream_of(device)))
+        if rows:
+            status = lib.hbt_grad_local_share_accumulated(
+                pointers, _native.pointer_array([a.data_ptr() for a in accumulated]), *args)
+        else:
+            status = lib.hbt_grad_local_share_sqnorm(pointers, *args)
+        _native.check(status, "test.share")
+        results.append((_bits(out), partials.cpu().numpy().view(np.int64)))
+    for got in results[1:]:
+        assert np.array_equal(results[0][0], got[0]) and np.array_equal(results[0][1], got[1])
