@@ -739,6 +739,26 @@ __device__ __forceinline__ float share_div(float x, float divisor, float recip) 
     if constexpr (kRecip) return x * recip;
     return x / divisor;
 }
+// x / d for an integer d of at most HBT_MAX_LOCAL_RANKS and r = 1 / d rounded to nearest, in
+// four operations where the division takes a dozen: the residual of x * r is exact, and one
+// correction by it rounds correctly (Markstein's division, IBM J. Res. Dev. 34(1), 1990),
+// which holds for all 2^23 significands of every such d, tried one by one on the CPU; at
+// other exponents the same significands are scaled, down to kQuickMin, below which the
+// residual could underflow.  div_fixup gives zeros, infinities and NaN what a division does.
+// A reduction of 2-byte gradients over 3, 5, 6 or 7 ranks was bound by its divisions: 5 bf16
+// ranks of 24.9 M elements 78 us with x / d and 64 us so, 7 ranks of 31.2 M 101 and 90; fp32
+// gradients and accumulated rows stream no faster either way.
+constexpr float kQuickMin = 0x1p-80f;
+__device__ __forceinline__ float quick_div(float x, float d, float r) {
+    float q = x * r;
+    q = __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
+    return __builtin_amdgcn_div_fixupf(q, d, x);
+}
+// 1 / d where quick_div serves d, else 0.
+float quick_reciprocal(float divisor) {
+    const bool served = divisor >= 1.0f && divisor <= float(HBT_MAX_LOCAL_RANKS) && divisor == std::floor(divisor);
+    return served ? 1.0f / divisor : 0.0f;
+}
 
 // The reference's AVG reduce-scatter in reduce dtype RD over inputs of dtype ID: the
 // gradient is cast to RD unless it already has that dtype (Tensor.to), each division
@@ -909,14 +929,31 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
                 if ((q + 1) % kIssue == 0 && q + 1 < kG && !burst) wait_vmem();
             }
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                sum[c] = round_to<RD>(share_div<kRecip>(share_input<ID, RD, kAcc>(x[0][c], a[0][c]), divisor, recip));
+            for (int q = 0; q < kG; ++q) {
 #pragma unroll
-                for (int q = 1; q < kG; ++q) {
-                    const float xq = share_input<ID, RD, kAcc>(x[q][c], a[kAcc ? q : 0][c]);
-                    sum[c] = round_to<RD>(sum[c] + round_to<RD>(share_div<kRecip>(xq, divisor, recip)));
-                }
+                for (int c = 0; c < 4; ++c) x[q][c] = share_input<ID, RD, kAcc>(x[q][c], a[kAcc ? q : 0][c]);
             }
+            const auto average = [&](auto&& divide) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    sum[c] = round_to<RD>(divide(x[0][c]));
+#pragma unroll
+                    for (int q = 1; q < kG; ++q) sum[c] = round_to<RD>(sum[c] + round_to<RD>(divide(x[q][c])));
+                }
+            };
+            // A wave whose values quick_div all serves takes it (recip holds 1 / divisor then, or 0).
+            bool quick = !kRecip && recip != 0.0f;
+            if constexpr (!kRecip) {
+                uint32_t least = 0xFFFFFFFFu;  // the smallest magnitude that is not zero
+#pragma unroll
+                for (int q = 0; q < kG; ++q) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) least = min(least, (__float_as_uint(x[q][c]) << 1) - 1u);
+                }
+                quick = quick && __all(least >= (__float_as_uint(kQuickMin) << 1) - 1u);
+            }
+            if (quick) average([&](float v) { return quick_div(v, divisor, recip); });
+            else average([&](float v) { return share_div<kRecip>(v, divisor, recip); });
         } else {
             // Any other group: two ranks' loads in flight at a time.
             float x[2][4];
@@ -2151,8 +2188,9 @@ int32_t local_share(const char* who, const void* const* rank_grads, int32_t grou
     const int64_t tiles = (shard_numel + kShareTile - 1) / kShareTile;
     if (tiles == 0) return HBT_OK;
     // An exact power of two (or 1) divides as a multiply by its exact reciprocal.
-    const float recip = exact_reciprocal(divisor);
+    float recip = exact_reciprocal(divisor);
     const bool recip_exact = recip != 0.0f;
+    if (!recip_exact && !f64) recip = quick_reciprocal(divisor);
     // A small shard's share and partials take one launch (local_share_small_kernel).
     const bool small = partials != nullptr && !with_acc && !f64 && tiles <= kSmallShareTiles;
     const int32_t burst = tiles <= kShareBurstTiles;

@@ -725,3 +725,37 @@ def test_local_share_off_cache_lines_is_the_same(device, shard, rows):
         results.append((_bits(out), partials.cpu().numpy().view(np.int64)))
     for got in results[1:]:
         assert np.array_equal(results[0][0], got[0]) and np.array_equal(results[0][1], got[1])
+
+
+@pytest.mark.parametrize("divisor", [3.0, 5.0, 6.0, 7.0, 11.0, 63.0, 2.5, 65.0])
+def test_local_share_divides_as_a_division_does(device, divisor):
+    """Every significand of one binade, and the values around the ranges where a division by
+    a rank count is formed from its reciprocal: subnormals, 2^-80, the largest, zeros,
+    infinities and NaN, alone in a tile of ordinary values and in tiles of their own."""
+    lib = _native.library()
+    ordinary = np.arange(1 << 23, dtype=np.uint32) | np.uint32(0x3F800000)
+    edge = []
+    for exponent in (0, 1, 2, 23, 24, 25, 45, 46, 47, 48, 125, 128, 252, 253, 254, 255):
+        base = exponent << 23
+        edge += [base, base + 1, base + 0x2AAAAA, base + 0x7FFFFF]
+    edge = np.array(edge, dtype=np.uint32)
+    edge = np.concatenate([edge, edge | np.uint32(0x80000000)])
+    planted = ordinary.copy()[: 256 * edge.size]
+    planted[77 :: 256] = edge
+    values = np.concatenate([ordinary, np.resize(edge, 1024), planted]).view(np.float32)
+    x = torch.from_numpy(values).to(device)
+    zeros = torch.zeros_like(x)
+    out = torch.empty_like(x)
+    for group in (1, 2):  # x / d, and x / d + 0 / d
+        status = lib.hbt_grad_local_share(_native.pointer_array([x.data_ptr(), zeros.data_ptr()][:group]), group, 0,
+                                          x.numel(), x.numel(), 0, 0, divisor, 0, out.data_ptr(),
+                                          ctypes.c_void_p(_native.stream_of(device)))
+        _native.check(status, "test.share")
+        with np.errstate(all="ignore"):
+            expect = values / np.float32(divisor)
+            if group == 2:
+                expect = expect + np.float32(0.0)
+        got = out.cpu().numpy()
+        nan = np.isnan(expect)
+        assert np.array_equal(np.isnan(got), nan)
+        assert np.array_equal(got.view(np.int32)[~nan], expect.view(np.int32)[~nan])
