@@ -292,8 +292,10 @@ __device__ __forceinline__ void CopyAny<SB, DB, OP, H>::run(const Record& rec, i
 
     const int64_t line = ((kLineBytes - (static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst)) & (kLineBytes - 1u))) &
                           (kLineBytes - 1u)) / DB;
-    // The source of the first whole line starts off a line, so every chunk's does.
-    if (src != nullptr && ((reinterpret_cast<uintptr_t>(src) + line * SB) & (kLineBytes - 1u)) != 0)
+    // The source of the first whole line starts off a line, so every chunk's does.  Widening
+    // chunks read 2 KB for the 4 KB they write, and the order those leave in counts for more: a
+    // 275 M-element bf16 to fp32 reshard 291 us in runs and 281 us without.
+    if (SB >= DB && src != nullptr && ((reinterpret_cast<uintptr_t>(src) + line * SB) & (kLineBytes - 1u)) != 0)
         c = xcd_order<kCopyRun>(c, (n + kChunk - 1) / kChunk);
     const int64_t e0 = c == 0 ? 0 : line + c * kChunk;
     const int64_t past = line + (c + 1) * kChunk;
