@@ -814,8 +814,8 @@ def bench_fsdp(steps: int, warmup: int) -> int:
     no_sync: one micro-batch's accumulation of rank 0's slices of the 8 bf16 gradients
     into its fp32 accumulator (read 4 + 2 B, write 4 B per accumulated element).  no_sync
     end: the call after the accumulation, which adds the last micro-batch to the 8
-    accumulated rows and reduces them in one pass (read 8 x (4 + 2) B + write 4 B per
-    shard element), the first micro-batch set up outside the timed events.
+    accumulated fp32 rows and reduces them in one pass (read 8 x (4 + 2) B + write 4 B per
+    shard element), two micro-batches before it set up outside the timed events.
     """
     import torch
 
@@ -934,8 +934,9 @@ def bench_fsdp(steps: int, warmup: int) -> int:
           _secondary_traffic("fsdp", ["gradient local share with norm partials", "fused clip + AdamW in the tail"],
                              [1, 1]), cpu.get("tail"))
 
-    # no_sync: the first micro-batch copies rank 0's slice of each rank's gradient into
-    # the fp32 accumulator (untimed); each timed micro-batch adds the eight slices to it.
+    # no_sync: the first micro-batch copies rank 0's slice of each rank's gradient and the
+    # second, among the warmup, forms the fp32 accumulator; each timed micro-batch adds the
+    # eight slices to it.
     owner.set_accumulate_without_reduction(True)
     owner.reduce_scatter_gradient(grads[0], peer_grads=grads)
 
@@ -956,7 +957,8 @@ def bench_fsdp(steps: int, warmup: int) -> int:
 
     def end_of_accumulation(events=None):
         owner.set_accumulate_without_reduction(True)
-        owner.reduce_scatter_gradient(grads[0], peer_grads=grads)  # the first micro-batch, untimed
+        for _ in range(2):  # untimed: the second forms the fp32 rows
+            owner.reduce_scatter_gradient(grads[0], peer_grads=grads)
         owner.set_accumulate_without_reduction(False)
         if events is not None:
             events[0].record(stream)
