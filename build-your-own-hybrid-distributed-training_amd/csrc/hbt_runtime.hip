@@ -56,10 +56,10 @@ extern "C" {
 const char* hbt_last_error(void) { return hbt::g_last_error.c_str(); }
 
 // Bumped whenever an exported signature or a table layout changes.
-int32_t hbt_abi_version(void) { return 20; }
+int32_t hbt_abi_version(void) { return 21; }
 
-// Entry points declared in include/hbt.h (hbt_last_error .. hbt_scale_inplace_f64).
-int32_t hbt_symbol_count(void) { return 39; }
+// Entry points declared in include/hbt.h (hbt_last_error .. hbt_exchange_capture_mode).
+int32_t hbt_symbol_count(void) { return 40; }
 
 int64_t hbt_grid_slices(int64_t blocks, int32_t threads, int64_t* first, int64_t* count, int64_t capacity) {
     if (threads <= 0) return -1;
@@ -71,6 +71,18 @@ int64_t hbt_grid_slices(int64_t blocks, int32_t threads, int64_t* first, int64_t
         if (count != nullptr) count[k] = blocks - start < per ? blocks - start : per;
     }
     return slices;
+}
+
+int32_t hbt_exchange_capture_mode(int32_t mode, int32_t* previous) {
+    hbt::clear_error();
+    if (mode < hipStreamCaptureModeGlobal || mode > hipStreamCaptureModeRelaxed) {
+        hbt::set_error("hbt_exchange_capture_mode: unknown mode %d", mode);
+        return HBT_ERR_INVALID_ARGUMENT;
+    }
+    hipStreamCaptureMode exchanged = static_cast<hipStreamCaptureMode>(mode);
+    const int32_t status = hbt::check_hip(hipThreadExchangeStreamCaptureMode(&exchanged), "hbt_exchange_capture_mode");
+    if (status == HBT_OK && previous != nullptr) *previous = static_cast<int32_t>(exchanged);
+    return status;
 }
 
 }  // extern "C"

@@ -68,7 +68,7 @@ __all__ = [
     "stream_of",
 ]
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 MAX_TENSORS_PER_LAUNCH = 16
 MAX_LOCAL_RANKS = 64
 MAX_NORM_PARTS = 128
@@ -87,6 +87,8 @@ COPY_ALIGNED = 1
 COPY_HINTS = 2
 #: Chunks per entry of a copy plan's hint table (HBT_COPY_HINTS).
 COPY_HINT_STRIDE = 256
+#: hipStreamCaptureModeRelaxed, for hbt_exchange_capture_mode.
+CAPTURE_MODE_RELAXED = 2
 #: Rows of a plan whose table travels in the launch's arguments (hbt_copy_rows).
 COPY_MAX_ROWS = 112
 ACCUMULATE_ASSIGN = 1
@@ -279,6 +281,7 @@ EXPORTED_SYMBOLS: dict[str, tuple[object, tuple[object, ...]]] = {
         (_c_void_p, _c_f64, _c_f64, _c_f64, _c_f64, _c_f64, _c_f64, _c_f64, _c_f64),
     ),
     "hbt_sgd_scalar_record_f64": (_c_i32, (_c_void_p, _c_f64, _c_f64, _c_f64, _c_f64, _c_f64, _c_i32)),
+    "hbt_exchange_capture_mode": (_c_i32, (_c_i32, ctypes.POINTER(_c_i32))),
     "hbt_write_words": (_c_i32, (_c_void_p, ctypes.POINTER(ctypes.c_uint32), _c_i64, _c_void_p)),
 }
 
@@ -371,6 +374,34 @@ def graph_recording() -> GraphRecording | None:
                          resolution="record the step with hybrid_training_amd.StepGraph")
         )
     return recording
+
+
+def capturing() -> bool:
+    """Whether launches on the current stream are being captured into a HIP graph, by a
+    recording or a bare ``torch.cuda.graph``."""
+    return _RECORDING.get() is not None or (
+        torch.cuda.is_initialized() and _IS_CAPTURING is not None and _IS_CAPTURING())
+
+
+@contextlib.contextmanager
+def outside_capture(device: torch.device):
+    """Run the block's allocations and launches on a stream of their own beside the capture
+    in progress, complete when the block ends.
+
+    The calling thread takes part in captures in relaxed mode meanwhile (as torch's allocator
+    does for its own calls): allocating and waiting are refused to a capturing thread
+    otherwise.  The block must not use the captured stream.
+    """
+    lib = library()
+    previous = ctypes.c_int32(0)
+    check(lib.hbt_exchange_capture_mode(CAPTURE_MODE_RELAXED, ctypes.byref(previous)), "native.outside_capture")
+    try:
+        side = torch.cuda.Stream(device)
+        with torch.cuda.stream(side):
+            yield
+        side.synchronize()
+    finally:
+        check(lib.hbt_exchange_capture_mode(previous.value, None), "native.outside_capture")
 
 
 def set_graph_recording(recording: GraphRecording | None):

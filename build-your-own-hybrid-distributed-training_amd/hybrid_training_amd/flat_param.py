@@ -605,10 +605,9 @@ class FlatParamHandle:
                 # (hbt_grad_local_share_accumulated): the rows are read once, not
                 # rewritten and read again.  The kernel only reads them, so they are
                 # dropped once it has been queued: a refused launch keeps them.
+                if self._grad_accumulator.dtype not in (self._reduce_dtype, in_dtype):
+                    self._widen_held()
                 rows = self._grad_accumulator
-                if rows.dtype != self._reduce_dtype and rows.dtype != in_dtype:
-                    rows = self._accumulator_rows(group, self._reduce_dtype)
-                    self._widen(self._grad_accumulator, rows)
         valid = max(0, min(self._shard_numel, self._total_numel - start))
         divisor = float(group) if (self._config.average_gradients and group > 1) else 1.0
         # A float64 master over a narrower reduce dtype: reduce into float32, widen after.
@@ -684,28 +683,33 @@ class FlatParamHandle:
         half the bytes written and read: 5 bf16 ranks' 24.9 M elements accumulated and
         reduced in 178 us, with float32 rows in 274.  A second addition holds the
         2-byte and the float32 rows together until it has been queued.
+
+        Under a capture nothing is held: a replayed first micro-batch writes float32 rows
+        and a replayed addition adds to the rows it was recorded over, as often as it is
+        replayed.  Rows held before the capture are widened before it goes on.
         """
         shard = self._shard_numel
         dtype = grads[0].dtype
         lib = _native.library()
         stream = _native.stream_of(self._device)
         sources = [g.data_ptr() + start * g.element_size() for g in grads]
-        if self._grad_accumulator is None:
-            if self._reduce_dtype == torch.float32 and dtype in (torch.bfloat16, torch.float16):
+        rows, held, flags = self._grad_accumulator, None, 0
+        if rows is None:
+            if (self._reduce_dtype == torch.float32 and dtype in (torch.bfloat16, torch.float16)
+                    and not _native.capturing()):
                 rows = self._accumulator_rows(len(grads), dtype)
                 plan = _native.CopyPlan.from_rows(
                     self._device, [(s, rows[q].data_ptr(), shard) for q, s in enumerate(sources)])
                 plan.run(src_dtype=dtype, dst_dtype=dtype)
                 self._grad_accumulator = rows
                 return
-            rows, held, flags = self._accumulator_rows(len(grads), self._reduce_dtype), None, _native.ACCUMULATE_ASSIGN
-        else:
-            rows, held, flags = self._grad_accumulator, None, 0
-            if rows.dtype != self._reduce_dtype:
+            rows, flags = self._accumulator_rows(len(grads), self._reduce_dtype), _native.ACCUMULATE_ASSIGN
+        elif rows.dtype != self._reduce_dtype:
+            if rows.dtype == dtype and not _native.capturing():
                 held, rows = rows, self._accumulator_rows(len(grads), self._reduce_dtype)
-                if held.dtype != dtype:
-                    self._widen(held, rows)
-                    held = None
+            else:
+                self._widen_held()
+                rows = self._grad_accumulator
         with _native.device_guard(self._device):
             for first in range(0, len(grads), _native.MAX_TENSORS_PER_LAUNCH):
                 batch = range(first, min(first + _native.MAX_TENSORS_PER_LAUNCH, len(grads)))
@@ -730,11 +734,29 @@ class FlatParamHandle:
         shard = self._shard_numel
         return torch.empty((group, -(-shard // 64) * 64), dtype=dtype, device=self._device)[:, :shard]
 
-    def _widen(self, held: torch.Tensor, rows: torch.Tensor) -> None:
-        """Held first micro-batches as the accumulator's rows."""
+    def _widen_held(self) -> None:
+        """Turn held first micro-batches into the accumulator's rows.
+
+        During a capture the rows are made outside it, in ordinary memory and complete when
+        this returns: a replay adds to them, so their first value may not be a recorded
+        launch's, and a block of the graph's own pool may also be an earlier temporary's.
+        The held gradients were queued before the capture, which ``torch.cuda.graph`` starts
+        with a synchronization.
+        """
+        held = self._grad_accumulator
+        if not _native.capturing():
+            self._grad_accumulator = self._widened(held)
+            return
+        with _native.outside_capture(self._device):
+            self._grad_accumulator = self._widened(held)
+
+    def _widened(self, held: torch.Tensor) -> torch.Tensor:
+        """The accumulator's rows over held first micro-batches, on the current stream."""
+        rows = self._accumulator_rows(len(held), self._reduce_dtype)
         plan = _native.CopyPlan.from_rows(
             self._device, [(h.data_ptr(), r.data_ptr(), self._shard_numel) for h, r in zip(held, rows)])
         plan.run(src_dtype=held.dtype, dst_dtype=rows.dtype)
+        return rows
 
     def set_accumulate_without_reduction(self, value: bool) -> None:
         """Enable or disable ``no_sync`` accumulation for this unit (``fsdp.py:791-797``).

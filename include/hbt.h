@@ -614,6 +614,19 @@ int32_t hbt_sgd_scalar_record_f64(void* record, double unscale, double weight_de
  * ---------------------------------------------------------------------------- */
 int32_t hbt_write_words(void* dst, const uint32_t* words, int64_t count, void* stream);
 
+/* ------------------------------------------------------------------------------
+ * How the calling thread takes part in HIP graph captures.
+ *
+ * Replaces: nothing the reference runs; the accumulate branch of
+ *   FlatParamHandle.reduce_scatter_gradient (parallel/fsdp.py:738-745) needs it where a
+ *   capture begins between two micro-batches.
+ * Sets the thread's capture mode (0 global, 1 thread-local, 2 relaxed: the values of
+ * hipStreamCaptureMode) by hipThreadExchangeStreamCaptureMode and, if `previous` is
+ * non-NULL, writes the mode it replaces.  In relaxed mode a thread may allocate, and launch
+ * on and wait for a stream that is not captured, while another stream of its is.
+ * ---------------------------------------------------------------------------- */
+int32_t hbt_exchange_capture_mode(int32_t mode, int32_t* previous);
+
 #ifdef __cplusplus
 }
 #endif

@@ -476,3 +476,95 @@ def test_recorded_no_sync_cycle(world):
         graph.replay()
         torch.cuda.synchronize()
         _assert_same(eager, graphed, norms, graph.output, k)
+
+
+_BF16_POLICY = MixedPrecisionConfig(enabled=True, param_dtype="bfloat16", reduce_dtype="float32", master_dtype="float32")
+
+
+def _micro_batches(tails: list[_Tail], count: int) -> list[list[torch.Tensor]]:
+    gen = torch.Generator(device=DEV).manual_seed(41)
+    out = []
+    for _ in range(count):
+        batch = [torch.randn(g.shape, device=DEV, generator=gen).to(g.dtype) for g in tails[0].grads]
+        for g in batch:
+            g[TOTAL:] = 0.0
+        out.append(batch)
+    return out
+
+
+def _reduce(tail: _Tail, batch: list[torch.Tensor], accumulate: bool) -> list[torch.Tensor | None]:
+    out = []
+    for r, h in enumerate(tail.handles):
+        h.set_accumulate_without_reduction(accumulate)
+        out.append(h.reduce_scatter_gradient(batch[r], peer_grads=batch))
+    return out
+
+
+def test_recorded_micro_batches_replay_any_number_of_times():
+    """The first 2-byte micro-batch, a further one and the reduction recorded apart: the
+    further one replayed twice adds twice, and the next cycle starts over."""
+    config = OptimizerConfig(learning_rate=1e-3)
+    eager, graphed = (_Tail(2, config, mp=_BF16_POLICY) for _ in range(2))
+    batches = _micro_batches([eager], 8)
+    static = graphed.grads
+    first, further = (StepGraph(lambda: _reduce(graphed, static, True)) for _ in range(2))
+    last = StepGraph(lambda: _reduce(graphed, static, False))
+    assert not any(h.has_pending_accumulation for h in graphed.handles)
+    for cycle in (batches[:4], batches[4:]):
+        for graph, batch in zip((first, further, further, last), cycle):
+            for g, value in zip(static, batch):
+                g.copy_(value)
+            graph.replay()
+        for batch in cycle[:-1]:
+            _reduce(eager, batch, True)
+        for expect, got in zip(_reduce(eager, cycle[-1], False), last.output):
+            assert torch.equal(expect, got)
+
+
+@pytest.mark.parametrize("bare", [False, True])
+@pytest.mark.parametrize("narrow_then_wide", [False, True])
+def test_micro_batches_recorded_after_an_eager_one(bare, narrow_then_wide):
+    """A 2-byte micro-batch accumulated eagerly, then a recorded one replayed twice and an
+    eager reduction: the sums of all four, whatever the recording allocates before it."""
+    config = OptimizerConfig(learning_rate=1e-3)
+    eager, graphed = (_Tail(2, config, mp=_BF16_POLICY) for _ in range(2))
+    batches = _micro_batches([eager], 4)
+    if narrow_then_wide:
+        batches = batches[:1] + [[g.float() for g in batch] for batch in batches[1:]]
+    static = [torch.empty_like(g) for g in batches[1]]
+    _reduce(graphed, batches[0], True)
+
+    def step() -> None:
+        for _ in range(3):  # temporaries whose blocks a later allocation of the recording may take
+            torch.full((1 << 16,), 7.0, device=DEV)
+        _reduce(graphed, static, True)
+
+    if bare:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step()
+    else:
+        graph = StepGraph(step)
+    for batch in batches[1:3]:
+        for g, value in zip(static, batch):
+            g.copy_(value)
+        graph.replay()
+    for batch in batches[:3]:
+        _reduce(eager, batch, True)
+    for expect, got in zip(_reduce(eager, batches[3], False), _reduce(graphed, batches[3], False)):
+        assert torch.equal(expect, got)
+
+
+def test_a_bare_capture_takes_a_first_micro_batch():
+    """Nothing a replay of an accumulation needs changes between replays, so a bare
+    ``torch.cuda.graph`` may record it."""
+    eager, graphed = (_Tail(2, OptimizerConfig(learning_rate=1e-3), mp=_BF16_POLICY) for _ in range(2))
+    batches = _micro_batches([eager], 2)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _reduce(graphed, batches[0], True)
+    for _ in range(2):
+        graph.replay()
+    _reduce(eager, batches[0], True)
+    for expect, got in zip(_reduce(eager, batches[1], False), _reduce(graphed, batches[1], False)):
+        assert torch.equal(expect, got)

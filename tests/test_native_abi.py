@@ -298,3 +298,10 @@ def test_c_host_compiles_against_the_header_and_links(tmp_path):
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout + run.stderr
     assert lib.hbt_abi_version() == _native.ABI_VERSION
+
+
+def test_capture_mode_is_checked_before_the_runtime_is_asked():
+    lib = _native.library()
+    for mode in (-1, 3):
+        assert lib.hbt_exchange_capture_mode(mode, None) == -1
+        assert b"unknown mode" in lib.hbt_last_error()
