@@ -38,6 +38,7 @@ a shard on the device by streaming it through (``optim.ShardedOptimizer``).
 
 from __future__ import annotations
 
+import contextlib
 import dataclasses
 from collections.abc import Sequence
 from dataclasses import dataclass
@@ -234,6 +235,7 @@ class FlatParamHandle:
         # no_sync accumulation: row q holds rank q's accumulated gradient restricted to
         # this rank's slice, the only part of it this rank's reduce-scatter reads.
         self._grad_accumulator: torch.Tensor | None = None
+        self._accumulator_stream = 0  # the stream the rows were allocated on
         self._full: torch.Tensor | None = None
         self._is_sharded = True
         if not keep_originals:
@@ -589,6 +591,7 @@ class FlatParamHandle:
         source_rank = self._shard_group.local_rank
         start = source_rank * self._shard_numel  # local_shard_range()'s
         rows = None  # accumulator rows the reduction adds the last micro-batch to
+        dropped = None  # accumulator rows that nothing reads after this reduction
         if self._accumulate_without_reduction:
             self._accumulate(grads, start)
             return None
@@ -597,8 +600,8 @@ class FlatParamHandle:
                 # Reduce the accumulated sums: row q is rank q's total restricted to this
                 # rank's slice, so the local share reads it at rank offset 0.
                 self._accumulate(grads, start)
-                accumulator, self._grad_accumulator = self._grad_accumulator, None
-                grads = list(accumulator.unbind(0))
+                dropped, self._grad_accumulator = self._grad_accumulator, None
+                grads = list(dropped.unbind(0))
                 source_rank = 0
             else:
                 # The last micro-batch is added to the rows inside the reduction
@@ -649,7 +652,9 @@ class FlatParamHandle:
                     what = "fsdp.hbt_grad_local_share_held"
         _native.check(status, what)
         if rows is not None:
-            self._grad_accumulator = None
+            dropped, self._grad_accumulator = rows, None
+        if dropped is not None:
+            self._free_behind_this_stream(dropped)
         # The squared-norm partials of the shard's real and padding segments ride on
         # the gradient, so the next clip_grad_norm does not read it again.
         segments = {}
@@ -701,7 +706,7 @@ class FlatParamHandle:
                 plan = _native.CopyPlan.from_rows(
                     self._device, [(s, rows[q].data_ptr(), shard) for q, s in enumerate(sources)])
                 plan.run(src_dtype=dtype, dst_dtype=dtype)
-                self._grad_accumulator = rows
+                self._grad_accumulator, self._accumulator_stream = rows, stream
                 return
             rows, flags = self._accumulator_rows(len(grads), self._reduce_dtype), _native.ACCUMULATE_ASSIGN
         elif rows.dtype != self._reduce_dtype:
@@ -727,12 +732,21 @@ class FlatParamHandle:
                                                      _native.dtype_code(dtype), flags, stream)
                     what = "fsdp.hbt_grad_accumulate"
                 _native.check(status, what)
-        self._grad_accumulator = rows
+        if held is not None:
+            self._free_behind_this_stream(held)
+        if rows is not self._grad_accumulator:
+            self._grad_accumulator, self._accumulator_stream = rows, stream
 
     def _accumulator_rows(self, group: int, dtype: torch.dtype) -> torch.Tensor:
         """One row per rank, each starting on a 64-element boundary."""
         shard = self._shard_numel
         return torch.empty((group, -(-shard // 64) * 64), dtype=dtype, device=self._device)[:, :shard]
+
+    def _free_behind_this_stream(self, rows: torch.Tensor) -> None:
+        """Rows about to be dropped, whose last reader was queued on the current stream: their
+        memory is reused after it, also where they were allocated on another stream."""
+        if self._accumulator_stream != _native.stream_of(self._device):
+            rows.record_stream(torch.cuda.current_stream(self._device))
 
     def _widen_held(self) -> None:
         """Turn held first micro-batches into the accumulator's rows.
@@ -743,12 +757,10 @@ class FlatParamHandle:
         The held gradients were queued before the capture, which ``torch.cuda.graph`` starts
         with a synchronization.
         """
-        held = self._grad_accumulator
-        if not _native.capturing():
-            self._grad_accumulator = self._widened(held)
-            return
-        with _native.outside_capture(self._device):
-            self._grad_accumulator = self._widened(held)
+        with _native.outside_capture(self._device) if _native.capturing() else contextlib.nullcontext():
+            held, rows = self._grad_accumulator, self._widened(self._grad_accumulator)
+            self._free_behind_this_stream(held)
+            self._grad_accumulator, self._accumulator_stream = rows, _native.stream_of(self._device)
 
     def _widened(self, held: torch.Tensor) -> torch.Tensor:
         """The accumulator's rows over held first micro-batches, on the current stream."""

@@ -394,6 +394,41 @@ def test_no_sync_accumulation_over_changing_dtypes(device, dtypes):
         assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32)), rank
 
 
+@pytest.mark.parametrize("further", [torch.bfloat16, torch.float16, None])
+def test_accumulated_rows_outlive_their_readers_on_another_stream(device, further):
+    """Rows allocated on one stream and read last on another, by a further micro-batch (of the
+    held dtype, or of one that has the rows widened first) or by the reduction: an allocation
+    on the first stream meanwhile does not get their memory."""
+    group = 2
+    handles = _mp_handles(group, device, "float32")
+    gen = torch.Generator(device=device).manual_seed(5)
+    grads = [[(torch.randn(h.padded_numel, device=device, generator=gen) * 1e-2).to(d) for h in handles]
+             for d in (torch.bfloat16, further or torch.bfloat16)]
+    h = handles[0]
+    h.set_accumulate_without_reduction(True)
+    h.reduce_scatter_gradient(grads[0][0], peer_grads=grads[0])
+    held = h._grad_accumulator.data_ptr()
+    nbytes = h._grad_accumulator.untyped_storage().nbytes()
+    h.set_accumulate_without_reduction(further is not None)
+    main, side = torch.cuda.current_stream(device), torch.cuda.Stream(device)
+    side.wait_stream(main)
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(100_000_000)
+        out = h.reduce_scatter_gradient(grads[1][0], peer_grads=grads[1])
+    fresh = [torch.full((nbytes,), 255, dtype=torch.uint8, device=device) for _ in range(8)]
+    assert held not in [t.data_ptr() for t in fresh]
+    main.wait_stream(side)
+    batches = grads
+    if further is not None:
+        h.set_accumulate_without_reduction(False)
+        out = h.reduce_scatter_gradient(grads[0][0], peer_grads=grads[0])
+        batches = grads + grads[:1]
+    totals = [oracle.no_sync_accumulate([m[q].float().cpu().numpy() for m in batches], "float32") for q in range(group)]
+    shard = h.shard_numel
+    expect = oracle.local_share(totals, 0, shard, min(shard, 1857), float(group), "float32")
+    assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32))
+
+
 def test_load_local_pieces_round_trip(device):
     named, originals, handles = _handles(MLP_23_32_32_1, 4, device)
     state = {name: torch.randn_like(orig) for (name, _), orig in zip(named, originals)}
