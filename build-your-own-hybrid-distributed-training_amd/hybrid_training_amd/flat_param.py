@@ -70,6 +70,9 @@ _FLOATS = (torch.float32, torch.bfloat16, torch.float16, torch.float64)
 #: in the norm partials' allocation: shards of up to 2 Mi elements.
 _SHARED_TILE_SUMS = 8192
 
+#: Elements of a held micro-batch uploaded at a time when it was moved to host memory.
+_WIDEN_PIECE = 1 << 19
+
 
 @dataclass(frozen=True)
 class ShardedTensorPiece:
@@ -687,7 +690,8 @@ class FlatParamHandle:
         next (the second addition, or the reduction) widens it and gives the same bits, for
         half the bytes written and read: 5 bf16 ranks' 24.9 M elements accumulated and
         reduced in 178 us, with float32 rows in 274.  A second addition holds the
-        2-byte and the float32 rows together until it has been queued.
+        2-byte and the float32 rows together until it has been queued; where the device
+        has no room for both, the 2-byte ones wait in host memory.
 
         Under a capture nothing is held: a replayed first micro-batch writes float32 rows
         and a replayed addition adds to the rows it was recorded over, as often as it is
@@ -711,8 +715,9 @@ class FlatParamHandle:
             rows, flags = self._accumulator_rows(len(grads), self._reduce_dtype), _native.ACCUMULATE_ASSIGN
         elif rows.dtype != self._reduce_dtype:
             if rows.dtype == dtype and not _native.capturing():
-                held, rows = rows, self._accumulator_rows(len(grads), self._reduce_dtype)
-            else:
+                with contextlib.suppress(torch.OutOfMemoryError):
+                    held, rows = rows, self._accumulator_rows(len(grads), self._reduce_dtype)
+            if held is None:
                 self._widen_held()
                 rows = self._grad_accumulator
         with _native.device_guard(self._device):
@@ -764,11 +769,36 @@ class FlatParamHandle:
 
     def _widened(self, held: torch.Tensor) -> torch.Tensor:
         """The accumulator's rows over held first micro-batches, on the current stream."""
-        rows = self._accumulator_rows(len(held), self._reduce_dtype)
-        plan = _native.CopyPlan.from_rows(
-            self._device, [(h.data_ptr(), r.data_ptr(), self._shard_numel) for h, r in zip(held, rows)])
-        plan.run(src_dtype=held.dtype, dst_dtype=rows.dtype)
+        try:
+            rows = self._accumulator_rows(len(held), self._reduce_dtype)
+        except torch.OutOfMemoryError:
+            return self._widened_through_host(held)
+        self._widen([(h.data_ptr(), r.data_ptr(), self._shard_numel) for h, r in zip(held, rows)], held.dtype)
         return rows
+
+    def _widened_through_host(self, held: torch.Tensor) -> torch.Tensor:
+        """:meth:`_widened` where the device holds the float32 rows but not the held ones
+        beside them, which give their memory back first.  Without room for the rows alone the
+        held ones are put back and the allocator's error is raised."""
+        waiting = [row.cpu() for row in held]
+        storage = held.untyped_storage()
+        nbytes = storage.nbytes()
+        storage.resize_(0)
+        try:
+            rows = self._accumulator_rows(len(held), self._reduce_dtype)
+        except torch.OutOfMemoryError:
+            storage.resize_(nbytes)
+            for row, host in zip(held, waiting):
+                row.copy_(host)
+            raise
+        for row, host in zip(rows, waiting):
+            for start in range(0, self._shard_numel, _WIDEN_PIECE):
+                piece = host[start : start + _WIDEN_PIECE].to(self._device)
+                self._widen([(piece.data_ptr(), row[start:].data_ptr(), piece.numel())], held.dtype)
+        return rows
+
+    def _widen(self, rows: list[tuple[int, int, int]], dtype: torch.dtype) -> None:
+        _native.CopyPlan.from_rows(self._device, rows).run(src_dtype=dtype, dst_dtype=self._reduce_dtype)
 
     def set_accumulate_without_reduction(self, value: bool) -> None:
         """Enable or disable ``no_sync`` accumulation for this unit (``fsdp.py:791-797``).

@@ -429,6 +429,44 @@ def test_accumulated_rows_outlive_their_readers_on_another_stream(device, furthe
     assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32))
 
 
+@pytest.mark.parametrize("room", [True, False])
+@pytest.mark.parametrize("further", [torch.bfloat16, torch.float16])
+def test_no_sync_accumulation_without_room_for_both_rows(device, monkeypatch, room, further):
+    """No device memory for the float32 rows beside the held 2-byte ones: they replace them
+    where they fit alone; where they do not, the call fails and loses nothing."""
+    from hybrid_training_amd import flat_param
+
+    monkeypatch.setattr(flat_param, "_WIDEN_PIECE", 100)
+    group = 2
+    handles = _mp_handles(group, device, "float32")
+    h = handles[0]
+    gen = torch.Generator(device=device).manual_seed(9)
+    grads = [[(torch.randn(h.padded_numel, device=device, generator=gen) * 1e-2).to(d) for _ in range(group)]
+             for d in (torch.bfloat16, further, torch.bfloat16)]
+    h.set_accumulate_without_reduction(True)
+    h.reduce_scatter_gradient(grads[0][0], peer_grads=grads[0])
+    allocate = h._accumulator_rows
+
+    def scarce(count, dtype):
+        if dtype == torch.float32 and (not room or h._grad_accumulator.untyped_storage().nbytes()):
+            raise torch.OutOfMemoryError("no room")
+        return allocate(count, dtype)
+
+    monkeypatch.setattr(h, "_accumulator_rows", scarce)
+    if not room:
+        for _ in range(2):
+            with pytest.raises(torch.OutOfMemoryError):
+                h.reduce_scatter_gradient(grads[1][0], peer_grads=grads[1])
+        monkeypatch.setattr(h, "_accumulator_rows", allocate)
+    h.reduce_scatter_gradient(grads[1][0], peer_grads=grads[1])
+    h.set_accumulate_without_reduction(False)
+    out = h.reduce_scatter_gradient(grads[2][0], peer_grads=grads[2])
+    totals = [oracle.no_sync_accumulate([m[q].float().cpu().numpy() for m in grads], "float32") for q in range(group)]
+    shard = h.shard_numel
+    expect = oracle.local_share(totals, 0, shard, min(shard, 1857), float(group), "float32")
+    assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32))
+
+
 def test_load_local_pieces_round_trip(device):
     named, originals, handles = _handles(MLP_23_32_32_1, 4, device)
     state = {name: torch.randn_like(orig) for (name, _), orig in zip(named, originals)}
