@@ -416,6 +416,12 @@ class FlatParamHandle:
                     observed=[int(s.numel()) for s in peer_shards],
                 )
             )
+        # Every consumer addresses all of them by one element size.
+        if any(s.dtype != peer_shards[0].dtype for s in peer_shards):
+            raise ShardingError(
+                format_error(operation, "peer shards must share one dtype",
+                             expected=str(peer_shards[0].dtype), observed=[str(s.dtype) for s in peer_shards])
+            )
         return list(peer_shards)
 
     def gather_full(self, peer_shards: Sequence[torch.Tensor] | None = None) -> torch.Tensor:

@@ -467,6 +467,20 @@ def test_no_sync_accumulation_without_room_for_both_rows(device, monkeypatch, ro
     assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32))
 
 
+@pytest.mark.parametrize("dtypes", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("call", ["gather_full", "unshard", "full_tensors"])
+def test_peer_shards_of_several_dtypes_are_refused(device, dtypes, call):
+    """One launch addresses every shard by the first one's element size: refused before it."""
+    h = _mp_handles(2, device, "float32")[0]
+    shards = [torch.zeros(h.shard_numel, dtype=d, device=device) for d in dtypes]
+    with pytest.raises(ShardingError, match="share one dtype"):
+        getattr(h, call)(shards)
+    full = h.gather_full([s.float() for s in shards])
+    h.reshard()
+    with pytest.raises(ShardingError, match="share one dtype"):
+        h.refill(full, shards)
+
+
 def test_load_local_pieces_round_trip(device):
     named, originals, handles = _handles(MLP_23_32_32_1, 4, device)
     state = {name: torch.randn_like(orig) for (name, _), orig in zip(named, originals)}
