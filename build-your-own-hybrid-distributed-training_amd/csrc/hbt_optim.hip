@@ -1417,7 +1417,7 @@ __global__ __launch_bounds__(64) void scale_kernel(ScaleTable tab, float unscale
 // multiplier it formed, bitwise norm_finalize_parts_kernel followed by scale_kernel.  A step
 // over gradients this small is bound by its launches (about 4 us of host time each, and as
 // long on the device): the 929-element MLP tail
-// takes 58 us with the two and 53 us with the one.  Past kClipMax elements
+// takes 58 us with the two and 53 us with the one.  Past HBT_CLIP_MAX_ELEMENTS elements
 // the sums repeated by every workgroup cost what the launch saves.
 constexpr int64_t kClipTile = int64_t(kFinalBlock) * 4;
 template <int D>
@@ -2558,10 +2558,14 @@ int32_t hbt_grad_norm_clip(const double* const* partials, const int64_t* counts,
     int64_t blocks = 0;
     status = build_scale_table("hbt_grad_norm_clip", grads, numels, count, kClipTile, scale, blocks);
     if (status != HBT_OK) return status;
-    if (blocks > HBT_CLIP_MAX_ELEMENTS / kClipTile + kMaxT) {
-        set_error("hbt_grad_norm_clip: more than %lld elements (finalize, then hbt_scale_inplace)",
-                  static_cast<long long>(HBT_CLIP_MAX_ELEMENTS));
-        return HBT_ERR_UNSUPPORTED;
+    int64_t room = HBT_CLIP_MAX_ELEMENTS;
+    for (int i = 0; i < count; ++i) {
+        if (numels[i] > room) {
+            set_error("hbt_grad_norm_clip: more than %lld elements (finalize, then hbt_scale_inplace)",
+                      static_cast<long long>(HBT_CLIP_MAX_ELEMENTS));
+            return HBT_ERR_UNSUPPORTED;
+        }
+        room -= numels[i];
     }
     const NormOutputs out{sum_out, norm_out, grad_mul_out, grad_mul64_out, nonfinite_out};
     hipStream_t st = as_stream(stream);

@@ -195,10 +195,10 @@ int32_t hbt_grad_norm_finalize_parts(const double* const* partials, const int64_
  * Replaces: the clip coefficient and the grad.mul_ loop of ShardedOptimizer.clip_grad_norm
  *   (optim/sharded_optimizer.py:331-337) where launches cost more than the gradients do.
  * Writes what hbt_grad_norm_finalize_parts writes, and multiplies the `count` gradients of
- * `dtype` (F32, BF16 or F16; at most HBT_MAX_TENSORS_PER_LAUNCH of them and, rounded up to
- * 4,096 each, HBT_CLIP_MAX_ELEMENTS elements together, else HBT_ERR_UNSUPPORTED) in place by
- * the fp32 multiplier, rounded to the dtype, untouched when it is 1: bitwise that call followed
- * by hbt_scale_inplace with its multiplier.  The gradients must not overlap the partials.
+ * `dtype` (F32, BF16 or F16; at most HBT_MAX_TENSORS_PER_LAUNCH of them, and at most
+ * HBT_CLIP_MAX_ELEMENTS elements together, else HBT_ERR_UNSUPPORTED) in place by the fp32
+ * multiplier, rounded to the dtype, untouched when it is 1: bitwise that call followed by
+ * hbt_scale_inplace with its multiplier.  The gradients must not overlap the partials.
  * ---------------------------------------------------------------------------- */
 #define HBT_CLIP_MAX_ELEMENTS 1048576
 int32_t hbt_grad_norm_clip(const double* const* partials, const int64_t* counts, const double* weights, int32_t parts,

@@ -305,3 +305,13 @@ def test_capture_mode_is_checked_before_the_runtime_is_asked():
     for mode in (-1, 3):
         assert lib.hbt_exchange_capture_mode(mode, None) == -1
         assert b"unknown mode" in lib.hbt_last_error()
+
+
+@pytest.mark.parametrize("sizes", [[1 << 20, 1], [1 << 19, 1 << 19, 0, 1], [(1 << 20) + 1], [1 << 62, 1 << 62]])
+def test_the_one_launch_clip_refuses_more_elements_than_it_states(sizes):
+    """``HBT_CLIP_MAX_ELEMENTS`` counts the elements themselves, refused before any launch."""
+    lib = _native.library()
+    pointers = _native.pointer_array([4096] * len(sizes))
+    assert lib.hbt_grad_norm_clip(None, None, None, 0, 1.0, pointers, _native.int64_array(sizes), len(sizes), 0,
+                                  None, None, None, None, None, None) == -2
+    assert str(_native.CLIP_MAX_ELEMENTS).encode() in lib.hbt_last_error()
