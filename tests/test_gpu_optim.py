@@ -722,3 +722,81 @@ def test_clip_on_both_sides_of_the_one_launch_limit(device, n):
     assert int(opt.last_nonfinite_flag().item()) == 0
     opt.step()
     assert float(opt.clip_grad_norm(10.0)) == pytest.approx(0.5, rel=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("extra", [0, 77])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_kept_launches_are_the_streamed_ones(device, dtype, extra, off):
+    """The norm, the in-place scale and the in-place unscale with partials of 32 MB and a little
+    more, which stay in the memory-side cache, against the same values in two launches, which
+    stream: bitwise, on and off the vectors; the values are torch's and the norm is within
+    1e-12 of 64 bits."""
+    lib = _native.library()
+    n = (32 << 20) // dtype.itemsize + extra
+    norm_chunk = 32768 if dtype == torch.float32 else 65536
+    half = n // 2 // norm_chunk * norm_chunk
+    gen = torch.Generator(device=device).manual_seed(extra + off)
+    values = (torch.randn(n + off, device=device, generator=gen) * 0.1).to(dtype)
+    mul = torch.tensor([0.3], device=device)
+    stream = _native.stream_of(device)
+    code, chunks = _native.dtype_code(dtype), -(-n // norm_chunk)
+    results = []
+    for cuts in ((0, n), (0, half, n)):
+        scaled, unscaled = values.clone(), values.clone()
+        partials = torch.full((3, chunks), -1.0, dtype=torch.float64, device=device)
+        scratch = torch.empty(chunks * _native.PIECES_PER_NORM_CHUNK, dtype=torch.float64, device=device)
+        for first, last in zip(cuts, cuts[1:]):
+            sizes, weight = _native.int64_array([last - first]), _native.double_array([1.0])
+
+            def at(t):
+                return _native.pointer_array([t.data_ptr() + (off + first) * t.element_size()])
+
+            rows = [row.data_ptr() + 8 * (first // norm_chunk) for row in partials]
+            for row, unscale in zip(rows, (1.0, 0.3)):
+                _native.check(lib.hbt_grad_sqnorm_partials(at(values), sizes, weight, 1, code, unscale, row, stream),
+                              "test.norm")
+            _native.check(lib.hbt_scale_inplace(at(scaled), sizes, 1, code, 0.7, mul.data_ptr(), stream), "test.scale")
+            _native.check(lib.hbt_scale_inplace_sqnorm(at(unscaled), sizes, 1, code, 0.3, rows[2],
+                                                       scratch.data_ptr(), stream), "test.unscale")
+        results.append((partials.view(torch.int64), scaled, unscaled))
+    for kept, streamed in zip(*results):
+        assert torch.equal(kept, streamed)
+    partials, scaled, unscaled = results[0]
+    # torch's multiplies on the CPU: on the GPU it rounds a half product once, not twice
+    lead, x = values[:off].cpu(), values[off:].cpu()
+    assert torch.equal(unscaled.cpu(), torch.cat([lead, x * 0.3]))
+    assert torch.equal(scaled.cpu(), torch.cat([lead, ((x * 0.7).float() * mul.cpu()).to(dtype)]))
+    sums = partials.view(torch.float64).sum(1)
+    for got, expect in zip(sums, (values[off:], unscaled[off:], unscaled[off:])):
+        assert abs(float(got) - float(expect.double().square().sum())) <= 1e-12 * float(got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_norm_clip_weighs_each_array(device, dtype):
+    """Partials of unequal weights, some of no elements: gradients and outputs bitwise the
+    finalize's and the in-place scale's over the same table."""
+    lib = _native.library()
+    gen = torch.Generator(device=device).manual_seed(8)
+    counts, weights = [3, 0, 1, 1029], [0.125, 7.0, 3.0, 0.5]
+    partials = [torch.rand(max(1, c), dtype=torch.float64, device=device, generator=gen) for c in counts]
+    values = (torch.randn(5000, device=device, generator=gen)).to(dtype)
+    table = (_native.pointer_array([p.data_ptr() for p in partials]), _native.int64_array(counts),
+             _native.double_array(weights), len(counts), 0.75)
+    code, stream, sizes = _native.dtype_code(dtype), _native.stream_of(device), _native.int64_array([5000])
+    outs = [torch.full((4,), 9.0, dtype=torch.float64, device=device) for _ in range(2)]
+    clipped = [values.clone() for _ in range(2)]
+
+    def outputs(o):
+        p = o.data_ptr()
+        return p, p + 8, p + 24, p + 16, p + 28, stream
+
+    _native.check(lib.hbt_grad_norm_finalize_parts(*table, *outputs(outs[0])), "test.finalize")
+    _native.check(lib.hbt_scale_inplace(_native.pointer_array([clipped[0].data_ptr()]), sizes, 1, code, 1.0,
+                                        outs[0].data_ptr() + 24, stream), "test.scale")
+    _native.check(lib.hbt_grad_norm_clip(*table, _native.pointer_array([clipped[1].data_ptr()]), sizes, 1, code,
+                                         *outputs(outs[1])), "test.clip")
+    assert torch.equal(outs[0].view(torch.int64), outs[1].view(torch.int64))
+    assert torch.equal(clipped[0], clipped[1]) and not torch.equal(clipped[0], values)
+    expect = sum(w * float(p[:c].sum()) for p, c, w in zip(partials, counts, weights))
+    assert abs(float(outs[0][0]) - expect) <= 1e-12 * expect
