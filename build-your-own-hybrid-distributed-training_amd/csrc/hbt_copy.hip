@@ -14,6 +14,9 @@
 // lines of the destination, so that only a record's first and last chunk write part of a
 // line, and reads its units where they lie with unaligned vector loads.  A load never
 // touches a byte outside the source interval.
+#include <algorithm>
+#include <cstring>
+
 #include "hbt_common.hpp"
 
 namespace hbt {
@@ -235,24 +238,29 @@ __device__ __forceinline__ Record owning_record(const int64_t* __restrict__ tabl
     return Record{rec[0], rec[1], rec[2], rec[3]};
 }
 
-// A plan of up to HBT_COPY_MAX_ROWS records in the launch's own arguments, with a hint for
-// every 2^shift chunks (kRowHints of them cover the plan), four to a word: the record that
-// owns the first of them.  A plan built for
-// one use, such as an unpack into fresh tensors, then needs no table built in pinned memory
-// and uploaded ahead of the launch: 52 GPT-2 tensors rebuilt from 5 ragged shards (542 MB, 101 us of
-// kernel) took 406 us a call with the table and took 115 us without, the rows counted by
-// arithmetic; a Llama-3-8B layer gathered from 8 shards 199 and 197 us.  3.9 KB, inside the 4 KB a launch's arguments may take.
+// A plan of up to kRows records in the launch's own arguments, with a hint for every 2^shift
+// chunks (kRowHints of them cover the plan), four to a word: the record that owns the first
+// of them.  A plan built for one use, such as an unpack into fresh tensors, then needs no
+// table built in pinned memory and uploaded ahead of the launch: 52 GPT-2 tensors rebuilt from
+// 5 ragged shards (542 MB, 101 us of kernel) took 406 us a call with the table and took 115 us
+// without, the rows counted by arithmetic; a Llama-3-8B layer gathered from 8 shards 199 and
+// 197 us.  HBT_COPY_MAX_ROWS records are 3.9 KB, inside the 4 KB a launch's arguments may take;
+// the host writes them at every launch, so a plan of at most kFewRows records takes 0.8 KB:
+// the call 3.1 us in place of 4.5, where one over a device table takes 3.2.
+constexpr int kFewRows = 16;
 constexpr int kRowHints = 256;
 constexpr uint32_t kHintSplit = 128;  // set when another record starts among the hint's chunks
+template <int kRows>
 struct RowTable {
-    Record rec[HBT_COPY_MAX_ROWS];
+    Record rec[kRows];
     uint32_t hint[kRowHints / 4];
     int32_t count;
     int32_t shift;
 };
 static_assert(HBT_COPY_MAX_ROWS <= kHintSplit, "a hint is one byte: a record and the split bit");
-static_assert(sizeof(RowTable) + 32 <= 4096, "the arguments of a launch");
-__device__ __forceinline__ Record owning_record(const RowTable& rows, int64_t chunk) {
+static_assert(sizeof(RowTable<HBT_COPY_MAX_ROWS>) + 32 <= 4096, "the arguments of a launch");
+template <int kRows>
+__device__ __forceinline__ Record owning_record(const RowTable<kRows>& rows, int64_t chunk) {
     const uint32_t j = static_cast<uint32_t>(chunk >> rows.shift);
     const uint32_t hint = (rows.hint[j >> 2] >> (8 * (j & 3u))) & 0xFFu;
     int r = static_cast<int>(hint & (kHintSplit - 1u));
@@ -600,21 +608,23 @@ __global__ __launch_bounds__(kCopyBlock) void copy_table_kernel(const int64_t* _
     const Record rec = owning_record(table, count, chunk, hints);
     Mover::run(rec, chunk - rec.first, divisor);
 }
-template <typename Mover>
-__global__ __launch_bounds__(kCopyBlock) void copy_rows_kernel(RowTable rows, typename Mover::Divisor divisor,
+template <typename Mover, int kRows>
+__global__ __launch_bounds__(kCopyBlock) void copy_rows_kernel(RowTable<kRows> rows, typename Mover::Divisor divisor,
                                                                int64_t chunk_base) {
     const int64_t chunk = chunk_base + static_cast<int64_t>(blockIdx.x);
     const Record rec = owning_record(rows, chunk);
     Mover::run(rec, chunk - rec.first, divisor);
 }
 
-// Where a launch finds its records: a device table, or the arguments (rows non-null).
+// Where a launch finds its records: a device table, or the arguments (few or rows non-null,
+// few where the plan fits it).
 struct Plan {
     const char* who;
     const int64_t* table;
     int64_t count;
     const int64_t* hints;
-    const RowTable* rows;
+    const RowTable<kFewRows>* few;
+    const RowTable<HBT_COPY_MAX_ROWS>* rows;
     int64_t chunks;
     bool aligned;
     hipStream_t stream;
@@ -622,8 +632,10 @@ struct Plan {
 template <typename Mover>
 int32_t launch_mover(const Plan& p, typename Mover::Divisor divisor) {
     return launch_sliced(p.who, p.chunks, kCopyBlock, [&](int64_t first, dim3 grid) {
-        if (p.rows != nullptr) {
-            copy_rows_kernel<Mover><<<grid, kCopyBlock, 0, p.stream>>>(*p.rows, divisor, first);
+        if (p.few != nullptr) {
+            copy_rows_kernel<Mover, kFewRows><<<grid, kCopyBlock, 0, p.stream>>>(*p.few, divisor, first);
+        } else if (p.rows != nullptr) {
+            copy_rows_kernel<Mover, HBT_COPY_MAX_ROWS><<<grid, kCopyBlock, 0, p.stream>>>(*p.rows, divisor, first);
         } else {
             copy_table_kernel<Mover><<<grid, kCopyBlock, 0, p.stream>>>(p.table, p.count, divisor, first, p.hints);
         }
@@ -748,7 +760,7 @@ int32_t hbt_copy_intervals(const int64_t* table, int64_t count, int64_t total_ch
     if (!copy_op_ok("hbt_copy_intervals", src_dtype, dst_dtype, op)) return HBT_ERR_INVALID_ARGUMENT;
     // The hints follow the count records of 4 int64 each.
     const int64_t* hints = (flags & HBT_COPY_HINTS) != 0 ? table + 4 * count : nullptr;
-    return launch_plan(Plan{"hbt_copy_intervals", table, count, hints, nullptr, total_chunks, aligned, as_stream(stream)},
+    return launch_plan(Plan{"hbt_copy_intervals", table, count, hints, nullptr, nullptr, total_chunks, aligned, as_stream(stream)},
                        src_dtype, dst_dtype, op, divisor);
 }
 
@@ -768,7 +780,8 @@ int32_t hbt_copy_rows(const int64_t* rows, int32_t count, int32_t src_dtype, int
     const int64_t chunk = hbt_copy_chunk_elems(src_dtype, dst_dtype);
     const uint64_t ssz = static_cast<uint64_t>(dtype_size(src_dtype)), dsz = static_cast<uint64_t>(dtype_size(dst_dtype));
     const uint64_t src_align = 16 * ssz / (ssz > dsz ? ssz : dsz);
-    RowTable tab{};
+    RowTable<HBT_COPY_MAX_ROWS> tab;  // what the plan does not fill is never read
+    tab.count = 0;
     int64_t chunks = 0;
     bool aligned = true;
     for (int32_t i = 0; i < count; ++i) {
@@ -783,15 +796,25 @@ int32_t hbt_copy_rows(const int64_t* rows, int32_t count, int32_t src_dtype, int
         chunks += (n * scale + chunk - 1) / chunk;
     }
     if (chunks == 0) return HBT_OK;
+    tab.shift = 0;
     while (((chunks - 1) >> tab.shift) >= kRowHints) ++tab.shift;
+    std::memset(tab.hint, 0, sizeof tab.hint);
     int r = 0;
     for (int64_t j = 0; j <= (chunks - 1) >> tab.shift; ++j) {
         while (r + 1 < tab.count && tab.rec[r + 1].first <= (j << tab.shift)) ++r;
         const bool split = r + 1 < tab.count && tab.rec[r + 1].first < ((j + 1) << tab.shift);
         tab.hint[j >> 2] |= (static_cast<uint32_t>(r) | (split ? kHintSplit : 0u)) << (8 * (j & 3));
     }
-    return launch_plan(Plan{"hbt_copy_rows", nullptr, tab.count, nullptr, &tab, chunks, aligned, as_stream(stream)},
-                       src_dtype, dst_dtype, op, divisor);
+    Plan plan{"hbt_copy_rows", nullptr, tab.count, nullptr, nullptr, &tab, chunks, aligned, as_stream(stream)};
+    RowTable<kFewRows> few;
+    if (tab.count <= kFewRows) {
+        std::copy(tab.rec, tab.rec + tab.count, few.rec);
+        std::memcpy(few.hint, tab.hint, sizeof few.hint);
+        few.count = tab.count;
+        few.shift = tab.shift;
+        plan.few = &few;
+    }
+    return launch_plan(plan, src_dtype, dst_dtype, op, divisor);
 }
 
 }  // extern "C"

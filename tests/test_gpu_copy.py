@@ -466,3 +466,30 @@ def test_records_off_the_destinations_lines(device, chunks, src, dst, src_off, d
         expect[dst_off : dst_off + n] = source[src_off : src_off + n].to(dst)
         assert torch.equal(target, expect), n
         assert torch.equal(other, source[: chunk + 3].to(dst))
+
+
+@pytest.mark.parametrize("count", [15, 16, 17])
+@pytest.mark.parametrize("spread", [1, 3000])
+@pytest.mark.parametrize(("sdt", "ddt"), [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                          (torch.float64, torch.float16)])
+def test_plans_around_a_few_rows(device, count, spread, sdt, ddt):
+    """Plans of as many records as the small argument table holds, one fewer and one more, with
+    rows of no elements among them and records of one chunk and of many."""
+    lib = _native.library()
+    rng = np.random.default_rng(count + spread)
+    sizes = [int(n) for n in rng.integers(1, spread + 1, size=count)]
+    sizes[0], sizes[count // 2], sizes[-1] = 1, 40 * spread, max(1, spread)
+    src = (torch.randn(sum(sizes), dtype=torch.float32, device=device) * 3).to(sdt)
+    dst = torch.full((sum(sizes) + count,), 7.0, dtype=ddt, device=device)
+    expected, source = dst.cpu(), src.cpu().to(ddt)
+    rows, at, to = [], 0, 0
+    for k, n in enumerate(sizes):
+        rows.append((src.data_ptr() + at * src.element_size(), dst.data_ptr() + to * dst.element_size(), n))
+        if k % 5 == 2:
+            rows.append((0, 0, 0))  # skipped: counts against neither table
+        expected[to : to + n] = source[at : at + n]
+        at, to = at + n, to + n + 1
+    flat = np.array(rows, dtype=np.int64).reshape(-1)
+    _native.check(lib.hbt_copy_rows(flat.ctypes.data, len(rows), _native.dtype_code(sdt), _native.dtype_code(ddt), 0,
+                                    1.0, _native.stream_of(device)), "test.copy_rows")
+    assert np.array_equal(_bits(dst), _bits(expected))
