@@ -405,9 +405,7 @@ class FlatParamHandle:
                     )
                 )
             return [self.flat_param.detach()]
-        if len(peer_shards) != self._shard_group.size or any(
-            s.numel() != self._shard_numel for s in peer_shards
-        ):
+        if [s.numel() for s in peer_shards] != [self._shard_numel] * self._shard_group.size:
             raise ShardingError(
                 format_error(
                     operation,
@@ -416,11 +414,11 @@ class FlatParamHandle:
                     observed=[int(s.numel()) for s in peer_shards],
                 )
             )
-        # Every consumer addresses all of them by one element size.
-        if any(s.dtype != peer_shards[0].dtype for s in peer_shards):
+        dtypes = [s.dtype for s in peer_shards]
+        if dtypes.count(dtypes[0]) != len(dtypes):  # every consumer addresses them by one element size
             raise ShardingError(
-                format_error(operation, "peer shards must share one dtype",
-                             expected=str(peer_shards[0].dtype), observed=[str(s.dtype) for s in peer_shards])
+                format_error(operation, "peer shards must share one dtype", expected=str(dtypes[0]),
+                             observed=[str(d) for d in dtypes])
             )
         return list(peer_shards)
 
