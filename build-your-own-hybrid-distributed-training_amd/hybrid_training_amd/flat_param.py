@@ -70,8 +70,21 @@ _FLOATS = (torch.float32, torch.bfloat16, torch.float16, torch.float64)
 #: in the norm partials' allocation: shards of up to 2 Mi elements.
 _SHARED_TILE_SUMS = 8192
 
+#: Elements of all ranks' slices from which a first 2-byte micro-batch is held in its own
+#: dtype: below, an accumulation is bound by the host, and holding costs it another allocation
+#: (one accumulated micro-batch and two, held and as float32 rows, 8 bf16 ranks: of 8 M
+#: elements 34 and 32 us, 50 and 43; of 16 M 34 and 40, 55 and 65; of 64 M 87 and 133, 189 and
+#: 228; 2 ranks: 31 and 30, 45 and 38; 33 and 42, 59 and 67; 104 and 146, 204 and 242).
+_HELD_MIN_ELEMENTS = 12 << 20
+
 #: Elements of a held micro-batch uploaded at a time when it was moved to host memory.
 _WIDEN_PIECE = 1 << 19
+
+
+def _row_addresses(rows: torch.Tensor) -> list[int]:
+    """The device address of every row of an accumulator."""
+    base, step = rows.data_ptr(), rows.stride(0) * rows.element_size()
+    return [base + q * step for q in range(rows.shape[0])]
 
 
 @dataclass(frozen=True)
@@ -650,7 +663,7 @@ class FlatParamHandle:
                 status = lib.hbt_grad_local_share_sqnorm(grad_ptrs, *args)
                 what = "fsdp.hbt_grad_local_share_sqnorm"
             else:
-                row_ptrs = _native.pointer_array([rows[q].data_ptr() for q in range(group)])
+                row_ptrs = _native.pointer_array(_row_addresses(rows))
                 if rows.dtype == self._reduce_dtype:
                     status = lib.hbt_grad_local_share_accumulated(grad_ptrs, row_ptrs, *args)
                     what = "fsdp.hbt_grad_local_share_accumulated"
@@ -690,7 +703,7 @@ class FlatParamHandle:
         rounded to the reduce dtype (``add_``).
 
         A first micro-batch of 2-byte gradients under a float32 reduce dtype is held in its
-        own dtype: its widening is exact wherever it happens, so the kernel that reads it
+        own dtype where its bytes count (``_HELD_MIN_ELEMENTS``): its widening is exact wherever it happens, so the kernel that reads it
         next (the second addition, or the reduction) widens it and gives the same bits, for
         half the bytes written and read: 5 bf16 ranks' 24.9 M elements accumulated and
         reduced in 178 us, with float32 rows in 274.  A second addition holds the
@@ -709,10 +722,10 @@ class FlatParamHandle:
         rows, held, flags = self._grad_accumulator, None, 0
         if rows is None:
             if (self._reduce_dtype == torch.float32 and dtype in (torch.bfloat16, torch.float16)
-                    and not _native.capturing()):
+                    and len(grads) * shard >= _HELD_MIN_ELEMENTS and not _native.capturing()):
                 rows = self._accumulator_rows(len(grads), dtype)
                 plan = _native.CopyPlan.from_rows(
-                    self._device, [(s, rows[q].data_ptr(), shard) for q, s in enumerate(sources)])
+                    self._device, [(source, row, shard) for source, row in zip(sources, _row_addresses(rows))])
                 plan.run(src_dtype=dtype, dst_dtype=dtype)
                 self._grad_accumulator, self._accumulator_stream = rows, stream
                 return
@@ -724,19 +737,22 @@ class FlatParamHandle:
             if held is None:
                 self._widen_held()
                 rows = self._grad_accumulator
+        row_addresses = _row_addresses(rows)
+        held_addresses = None if held is None else _row_addresses(held)
+        step = _native.MAX_TENSORS_PER_LAUNCH
         with _native.device_guard(self._device):
-            for first in range(0, len(grads), _native.MAX_TENSORS_PER_LAUNCH):
-                batch = range(first, min(first + _native.MAX_TENSORS_PER_LAUNCH, len(grads)))
-                sums = _native.pointer_array([rows[q].data_ptr() for q in batch])
-                added = _native.pointer_array([sources[q] for q in batch])
-                sizes = _native.int64_array([shard] * len(batch))
-                if held is not None:
+            for first in range(0, len(grads), step):
+                sums = _native.pointer_array(row_addresses[first : first + step])
+                added = _native.pointer_array(sources[first : first + step])
+                count = min(step, len(grads) - first)
+                sizes = _native.int64_array([shard] * count)
+                if held_addresses is not None:
                     status = lib.hbt_grad_accumulate_held(
-                        sums, _native.pointer_array([held[q].data_ptr() for q in batch]), added, sizes, len(batch),
+                        sums, _native.pointer_array(held_addresses[first : first + step]), added, sizes, count,
                         _native.dtype_code(dtype), stream)
                     what = "fsdp.hbt_grad_accumulate_held"
                 else:
-                    status = lib.hbt_grad_accumulate(sums, added, sizes, len(batch),
+                    status = lib.hbt_grad_accumulate(sums, added, sizes, count,
                                                      _native.dtype_code(self._reduce_dtype),
                                                      _native.dtype_code(dtype), flags, stream)
                     what = "fsdp.hbt_grad_accumulate"
@@ -777,7 +793,7 @@ class FlatParamHandle:
             rows = self._accumulator_rows(len(held), self._reduce_dtype)
         except torch.OutOfMemoryError:
             return self._widened_through_host(held)
-        self._widen([(h.data_ptr(), r.data_ptr(), self._shard_numel) for h, r in zip(held, rows)], held.dtype)
+        self._widen([(h, r, self._shard_numel) for h, r in zip(_row_addresses(held), _row_addresses(rows))], held.dtype)
         return rows
 
     def _widened_through_host(self, held: torch.Tensor) -> torch.Tensor:

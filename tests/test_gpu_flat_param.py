@@ -27,6 +27,7 @@ from hybrid_training_amd import (
     optimizer_parameter_layout,
     reshard_state_dict_pieces,
 )
+from hybrid_training_amd import flat_param
 from hybrid_training_amd.errors import UnsupportedFeatureError
 from hybrid_training_amd.optim import NORM_PARTIALS_ATTR
 
@@ -394,11 +395,29 @@ def test_no_sync_accumulation_over_changing_dtypes(device, dtypes):
         assert np.array_equal(out.cpu().numpy().view(np.int32), expect.view(np.int32)), rank
 
 
+@pytest.mark.parametrize("dtypes", [(torch.bfloat16,) * 2, (torch.bfloat16,) * 3, (torch.float16,) * 4,
+                                    (torch.bfloat16, torch.float32), (torch.float16, torch.bfloat16),
+                                    (torch.bfloat16, torch.float16, torch.float16)])
+@pytest.mark.parametrize("above", [-1, 0, 1])
+def test_held_micro_batches_from_the_smallest_size_on(device, monkeypatch, dtypes, above):
+    """A first 2-byte micro-batch is held from ``_HELD_MIN_ELEMENTS`` on and widened below;
+    bitwise the oracle's float32 accumulation on both sides."""
+    h = _mp_handles(2, device, "float32")[0]
+    elements = 2 * h.shard_numel
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", elements - above)
+    grad = torch.zeros(h.padded_numel, dtype=dtypes[0], device=device)
+    h.set_accumulate_without_reduction(True)
+    h.reduce_scatter_gradient(grad, peer_grads=[grad, grad])
+    assert h._grad_accumulator.dtype == (dtypes[0] if above >= 0 else torch.float32)
+    test_no_sync_accumulation_over_changing_dtypes(device, dtypes)
+
+
 @pytest.mark.parametrize("further", [torch.bfloat16, torch.float16, None])
-def test_accumulated_rows_outlive_their_readers_on_another_stream(device, further):
+def test_accumulated_rows_outlive_their_readers_on_another_stream(device, monkeypatch, further):
     """Rows allocated on one stream and read last on another, by a further micro-batch (of the
     held dtype, or of one that has the rows widened first) or by the reduction: an allocation
     on the first stream meanwhile does not get their memory."""
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", 0)
     group = 2
     handles = _mp_handles(group, device, "float32")
     gen = torch.Generator(device=device).manual_seed(5)
@@ -434,8 +453,7 @@ def test_accumulated_rows_outlive_their_readers_on_another_stream(device, furthe
 def test_no_sync_accumulation_without_room_for_both_rows(device, monkeypatch, room, further):
     """No device memory for the float32 rows beside the held 2-byte ones: they replace them
     where they fit alone; where they do not, the call fails and loses nothing."""
-    from hybrid_training_amd import flat_param
-
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", 0)
     monkeypatch.setattr(flat_param, "_WIDEN_PIECE", 100)
     group = 2
     handles = _mp_handles(group, device, "float32")

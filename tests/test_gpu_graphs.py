@@ -31,7 +31,7 @@ from hybrid_training_amd import (
     StepGraph,
     UnsupportedFeatureError,
 )
-from hybrid_training_amd import _native
+from hybrid_training_amd import _native, flat_param
 from hybrid_training_amd.optim import PENDING_UNSCALE_ATTR
 
 pytestmark = pytest.mark.gpu
@@ -500,9 +500,10 @@ def _reduce(tail: _Tail, batch: list[torch.Tensor], accumulate: bool) -> list[to
     return out
 
 
-def test_recorded_micro_batches_replay_any_number_of_times():
+def test_recorded_micro_batches_replay_any_number_of_times(monkeypatch):
     """The first 2-byte micro-batch, a further one and the reduction recorded apart: the
     further one replayed twice adds twice, and the next cycle starts over."""
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", 0)
     config = OptimizerConfig(learning_rate=1e-3)
     eager, graphed = (_Tail(2, config, mp=_BF16_POLICY) for _ in range(2))
     batches = _micro_batches([eager], 8)
@@ -523,9 +524,10 @@ def test_recorded_micro_batches_replay_any_number_of_times():
 
 @pytest.mark.parametrize("bare", [False, True])
 @pytest.mark.parametrize("narrow_then_wide", [False, True])
-def test_micro_batches_recorded_after_an_eager_one(bare, narrow_then_wide):
+def test_micro_batches_recorded_after_an_eager_one(monkeypatch, bare, narrow_then_wide):
     """A 2-byte micro-batch accumulated eagerly, then a recorded one replayed twice and an
     eager reduction: the sums of all four, whatever the recording allocates before it."""
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", 0)
     config = OptimizerConfig(learning_rate=1e-3)
     eager, graphed = (_Tail(2, config, mp=_BF16_POLICY) for _ in range(2))
     batches = _micro_batches([eager], 4)
@@ -555,9 +557,10 @@ def test_micro_batches_recorded_after_an_eager_one(bare, narrow_then_wide):
         assert torch.equal(expect, got)
 
 
-def test_a_bare_capture_takes_a_first_micro_batch():
+def test_a_bare_capture_takes_a_first_micro_batch(monkeypatch):
     """Nothing a replay of an accumulation needs changes between replays, so a bare
     ``torch.cuda.graph`` may record it."""
+    monkeypatch.setattr(flat_param, "_HELD_MIN_ELEMENTS", 0)
     eager, graphed = (_Tail(2, OptimizerConfig(learning_rate=1e-3), mp=_BF16_POLICY) for _ in range(2))
     batches = _micro_batches([eager], 2)
     graph = torch.cuda.CUDAGraph()
