@@ -160,8 +160,8 @@ __device__ __forceinline__ void store_upto(void* base, int64_t e, int64_t n, con
     }
 }
 
-// K consecutive doubles from element e (K even, e a multiple of 2, base 16-byte aligned):
-// K / 2 non-temporal 16-byte loads.
+// K consecutive doubles from element e (K even): K / 2 non-temporal 16-byte loads from any
+// element boundary.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef f64x2 f64x2_any __attribute__((aligned(8)));
 template <int K>
@@ -184,7 +184,7 @@ __device__ __forceinline__ void store_f64(void* base, int64_t e, const double (&
 }
 // Four consecutive SB-byte elements (float64, float32, or bf16 / fp16 when SH) from
 // element e, widened exactly to double (Tensor.to(float64)), with 16-byte loads (8-byte
-// for 2-byte elements); base + e * SB must be aligned to 4 * SB bytes (16 for doubles).
+// for 2-byte elements) from any element boundary.
 template <int SB, bool SH>
 __device__ __forceinline__ void load4_as_f64(const void* base, int64_t e, double (&x)[4]) {
     if constexpr (SB == 8) {
@@ -754,7 +754,11 @@ __device__ __forceinline__ float quick_div(float x, float d, float r) {
     q = __builtin_fmaf(__builtin_fmaf(-q, d, x), r, q);
     return __builtin_amdgcn_div_fixupf(q, d, x);
 }
-// 1 / d where quick_div serves d, else 0.
+// 1 / d where quick_div serves d, else 0.  The groups with an instantiation of their own use it.
+// The run-time group loop divides: its 2-byte reductions are bound by the division too (16.8 M
+// elements, 12 bf16 ranks 88 us at 5.3 TB/s, 15 ranks 109 at 5.3, 16 ranks, which multiply, 97 at
+// 6.2; fp32 gradients 6.06, 5.84 and 5.97 TB/s), as are those of a fixed reduce dtype into another
+// master dtype (5 bf16 ranks into bf16 masters over fp32 sums 47 us, 8 ranks 54).
 float quick_reciprocal(float divisor) {
     const bool served = divisor >= 1.0f && divisor <= float(HBT_MAX_LOCAL_RANKS) && divisor == std::floor(divisor);
     return served ? 1.0f / divisor : 0.0f;
@@ -793,8 +797,8 @@ constexpr int kShareAccIssue = 1;
 constexpr int kShareHeldIssue = 2;
 // Consecutive tiles that one XCD reduces where a rank's slice does not start on a cache
 // line (xcd_order): each 512 B of bf16 then touches 5 lines, the fifth shared with the next
-// tile.  With one tile and with 8, 16 and 32, and pairs for held rows: 5 bf16 ranks of
-// 24.9 M elements held and reduced 188, 169, 168 and 166 us.  Slices on lines keep the
+// tile.  With one tile and with 8, 16 and 32: 5 bf16 ranks of 24.9 M elements reduced in 70.5,
+// 65.5, 63.4 and 62.4 us, held and reduced in 178, 170, 169 and 166.  Slices on lines keep the
 // dispatch order, which streams them faster (a Llama-3-8B layer of 8 ranks 88.6 us, 92 us
 // in runs of 4 or 16).
 constexpr int kShareRun = 32;
@@ -911,10 +915,11 @@ __device__ __forceinline__ double share_tile(const ShareRanks& ranks, const Shar
     double acc = 0.0;
     if (base < valid_numel && valid_numel >= kShareTile) {
         // The tile the real elements end in reads and sums the whole tile that ends there and
-        // keeps what lies past the tile before it.  Stepped element by element it took a memory round trip per
-        // rank for every 64 elements, at the very end of the launch: 8 ranks into a shard of
-        // 885,984 bf16 elements (3460 tiles and 224 elements) in 11.0 us so and in 5.3 us
-        // so.
+        // keeps what lies past the tile before it.  Stepped element by element it took a memory
+        // round trip per rank for every 64 elements, at the very end of the launch: 8
+        // bf16 ranks into a shard of 885,984 fp32 elements (3460 tiles and 224 elements) took
+        // 8.4 us of kernel so and take 4.3, with every rank's loads issued together
+        // (kShareBurstTiles).
         const bool whole = base + kShareTile <= valid_numel;
         const int counted = whole ? 0 : static_cast<int>(base + kShareTile - valid_numel);
         const int64_t e = (whole ? base : valid_numel - kShareTile) + int64_t(lane) * 4;
@@ -1862,7 +1867,12 @@ float host_round_to(float x, int32_t dtype) {
 // fit its 256 MB, and below 32 MB the L2 serves the next pass either way.  Kept and not
 // kept, whole tails: norm, clip and AdamW of 54 M fp32 elements (a 2-layer GPT-2 under DDP)
 // 418 and 433 us, of 30 M 226 and 239; norm and AdamW without a clip in place of 30 M 151
-// and 159; past 256 MB keeping slows the norm by 6% and saves nothing.
+// and 159; past 256 MB keeping slows the norm by 6% and saves nothing.  Each launch goes by its
+// own bytes, also where a list of more than 16 gradients takes several.  One answer for the
+// whole list, kept where all of it lies in that range, was slower: the norm and a deferred
+// AdamW step of 28 fp32 gradients of 360 MB 457 us by launch and 477 by list, of 40 bf16 ones
+// of 400 MB 507 and 525; norm, clip and AdamW of 40 bf16 gradients of 120 MB 415 and 429, of 32
+// fp32 ones of 440 MB 842 and 860, of 28 of 217 MB 411 and 413.
 bool keep_for_next_pass(const int64_t* numels, int32_t count, int32_t dtype) {
     int64_t bytes = 0;
     for (int32_t i = 0; i < count; ++i) bytes += numels[i] * dtype_size(dtype);

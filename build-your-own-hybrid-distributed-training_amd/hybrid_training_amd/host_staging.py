@@ -111,9 +111,8 @@ class HostStream:
 
         ``staged[k]`` is the device copy of ``operands[k].host[start : start + n]``.  It
         begins ``lead`` elements into its staging buffer, whose base is 256-byte aligned,
-        so a kernel that takes a vector path only on 16-byte aligned addresses sees the
-        same alignment as on the host tensor when ``lead`` is that tensor's element
-        offset from a 16-byte boundary.  ``resident = (device_flat, host_flat)``: after
+        so a kernel's vectors lie as they would over the host tensor when ``lead`` is that
+        tensor's element offset from a 16-byte boundary; no result depends on it.  ``resident = (device_flat, host_flat)``: after
         each launch, ``device_flat[start : start + n]`` is also written back to
         ``host_flat`` (a device tensor whose host copy follows it).
         """

@@ -355,8 +355,8 @@ def gradient_norm_pass(
 
     A gradient in host memory (a parameter shard kept on the host) is uploaded through
     the device's :class:`~hybrid_training_amd.host_staging.HostStream` and summed there
-    chunk by chunk; its partials are the ones the same values would give in HBM at the
-    same 16-byte alignment, so the result does not depend on where the gradient lives.
+    chunk by chunk; its partials are the ones the same values would give in HBM, so the
+    result does not depend on where the gradient lives.
     """
     lib = _native.library()
     batches: dict[tuple[torch.dtype, float], list[tuple[torch.Tensor, int, int, float]]] = {}
@@ -517,9 +517,10 @@ def norm_chunk_elems(dtype: torch.dtype) -> int:
 def _stream_sqnorm(lib, grad, offset, length, weight, dtype, unscale, partials, slot, device) -> None:
     """The partials of a host gradient's segment, from slot ``slot``, summed on ``device``.
 
-    Each staged chunk holds whole norm chunks of the segment and starts at the
-    segment's own offset from a 16-byte boundary, so every partial is summed over the
-    same elements in the same order as a launch over the segment in HBM would sum it.
+    Each staged chunk holds whole norm chunks of the segment, so every partial is summed over
+    the same elements in the same order as a launch over the segment in HBM would sum it; it
+    starts at the segment's own offset from a 16-byte boundary, so its vectors lie as they
+    would there.
     """
     flat = grad.detach().reshape(-1)
     size = flat.element_size()
@@ -593,7 +594,7 @@ def unscale_with_partials(grads: Sequence[torch.Tensor], dtype: torch.dtype, uns
     (``hbt_scale_inplace_sqnorm``): each gradient leaves with a :class:`NormPartials`
     record of its whole length, so the overflow check and a following clip read none
     of them again.  A gradient in host memory streams through ``device``, its staged
-    chunks placed at its own 16-byte alignment as the norm pass places them, and is
+    chunks placed at its own 16-byte offset as the norm pass places them, and is
     final on the host when this returns.  Float64 gradients are scaled in double
     (``hbt_scale_inplace_f64``) without partials; the overflow check sums them after."""
     if dtype == torch.float64:
