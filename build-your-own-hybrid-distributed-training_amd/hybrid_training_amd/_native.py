@@ -716,6 +716,10 @@ def bump_versions(tensors: Iterable[torch.Tensor]) -> None:
         increment_version(written)
 
 
+#: Packers of a short plan's words by its rows, as :func:`struct.pack` would find them each time.
+_PACKERS: dict[int, Any] = {}
+
+
 class CopyPlan:
     """Interval table for one ``hbt_copy_intervals`` launch.
 
@@ -728,8 +732,12 @@ class CopyPlan:
 
     def __init__(self, device: torch.device) -> None:
         self.device = torch.device(device)
-        self._rows: list[tuple[int, int, int]] = []
-        self._flat: bytes | None = None  # the rows as the launch takes them, kept for a repeated run
+        # The rows (source address, destination address, n) one after another, only appended to,
+        # and as the launch takes them, formed once for a repeated run: the words packed, or the
+        # tuple of rows a longer plan's table is kept under.
+        self._words: list[int] = []
+        self._packed: bytes | tuple[tuple[int, int, int], ...] = ()
+        self._packed_count = 0
         # The tensors the rows address, held for the plan's lifetime.  A row records
         # only addresses: a temporary the caller made for it (a dense or device copy)
         # and dropped before run() would hand its memory to the next allocation on the
@@ -741,7 +749,7 @@ class CopyPlan:
         self._dests: dict[int, torch.Tensor] = {}
 
     def __len__(self) -> int:
-        return len(self._rows)
+        return len(self._words) // 3
 
     @classmethod
     def from_rows(cls, device: torch.device, rows: list[tuple[int, int, int]]) -> "CopyPlan":
@@ -753,7 +761,7 @@ class CopyPlan:
         version counters of the tensors written (:func:`bump_versions`).
         """
         plan = cls(device)
-        plan._rows = [row for row in rows if row[2] > 0]
+        plan._words = list(chain.from_iterable([row for row in rows if row[2] > 0]))
         return plan
 
     def add(self, src: torch.Tensor, src_offset: int, dst: torch.Tensor, dst_offset: int, n: int) -> None:
@@ -773,13 +781,8 @@ class CopyPlan:
             return
         self._keep.append(src)
         self._dests[id(dst)] = dst
-        self._rows.append(
-            (
-                src.data_ptr() + src_offset * src.element_size(),
-                dst.data_ptr() + dst_offset * dst.element_size(),
-                n,
-            )
-        )
+        self._words += (src.data_ptr() + src_offset * src.element_size(),
+                        dst.data_ptr() + dst_offset * dst.element_size(), n)
 
     def add_zero(self, dst: torch.Tensor, dst_offset: int, n: int) -> None:
         """Queue ``dst[dst_offset : dst_offset + n] = 0``."""
@@ -791,7 +794,19 @@ class CopyPlan:
         if n == 0:
             return
         self._dests[id(dst)] = dst
-        self._rows.append((0, dst.data_ptr() + dst_offset * dst.element_size(), n))
+        self._words += (0, dst.data_ptr() + dst_offset * dst.element_size(), n)
+
+    def _pack(self, count: int) -> bytes | tuple[tuple[int, int, int], ...]:
+        words = self._words
+        if count <= COPY_MAX_ROWS:
+            pack = _PACKERS.get(count)
+            if pack is None:
+                pack = _PACKERS[count] = struct.Struct(f"{3 * count}q").pack
+            self._packed = pack(*words)
+        else:
+            self._packed = tuple(zip(words[::3], words[1::3], words[2::3]))
+        self._packed_count = count
+        return self._packed
 
     def run(
         self,
@@ -802,20 +817,18 @@ class CopyPlan:
         divisor: float = 1.0,
     ) -> None:
         """Launch the copy on the current stream of the plan's device."""
-        if not self._rows:
+        count = len(self._words) // 3
+        if count == 0:
             return
         src_code = dtype_code(src_dtype)
         dst_code = dtype_code(dst_dtype)
         lib = library()
-        if len(self._rows) <= COPY_MAX_ROWS:
+        rows = self._packed if count == self._packed_count else self._pack(count)
+        if count <= COPY_MAX_ROWS:
             # The table rides in the launch: nothing to build on the device or to keep.
             graph_recording()  # a capture that a replay could not repeat correctly is refused
-            count = len(self._rows)
-            flat = self._flat
-            if flat is None or len(flat) != 24 * count:  # rows are only ever appended
-                flat = self._flat = struct.pack(f"{3 * count}q", *chain.from_iterable(self._rows))
             with device_guard(self.device):
-                status = lib.hbt_copy_rows(flat, count, src_code, dst_code, op, float(divisor),
+                status = lib.hbt_copy_rows(rows, count, src_code, dst_code, op, float(divisor),
                                            stream_of(self.device))
             check(status, "native.hbt_copy_rows")
             bump_versions(self._dests.values())
@@ -825,11 +838,11 @@ class CopyPlan:
             # An 8-byte element moves as two dwords.
             src_code = dst_code = DTYPE_F32
             scale = 2
-        table, first, aligned = _prepared_plan(self.device, tuple(self._rows), src_code, dst_code, scale)
+        table, first, aligned = _prepared_plan(self.device, rows, src_code, dst_code, scale)
         with device_guard(self.device):
             status = lib.hbt_copy_intervals(
                 table.data_ptr(),
-                len(self._rows),
+                count,
                 first,
                 src_code,
                 dst_code,
