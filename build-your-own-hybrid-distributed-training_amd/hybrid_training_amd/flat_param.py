@@ -75,7 +75,7 @@ _SHARED_TILE_SUMS = 8192
 #: (one accumulated micro-batch and two, held and as float32 rows, 8 bf16 ranks: of 8 M
 #: elements 34 and 32 us, 50 and 43; of 16 M 34 and 40, 55 and 65; of 64 M 87 and 133, 189 and
 #: 228; 2 ranks: 31 and 30, 45 and 38; 33 and 42, 59 and 67; 104 and 146, 204 and 242).
-_HELD_MIN_ELEMENTS = 12 << 20
+_HELD_MIN_ELEMENTS = 10 << 20
 
 #: Elements of a held micro-batch uploaded at a time when it was moved to host memory.
 _WIDEN_PIECE = 1 << 19
@@ -524,7 +524,8 @@ class FlatParamHandle:
                   for s in self._all_shards(peer_shards, "fsdp.full_tensors")]
         dtype, length = shards[0].dtype, self._shard_numel
         for shard in shards:
-            _native.require_device_tensor(shard, "fsdp.full_tensors")
+            if not shard.is_cuda:
+                _native.require_device_tensor(shard, "fsdp.full_tensors")
         out = {e.name: torch.empty(e.shape, dtype=dtype, device=self._device) for e in self._entries}
         size = dtype.itemsize
         bases = [shard.data_ptr() for shard in shards]
