@@ -74,7 +74,8 @@ _SHARED_TILE_SUMS = 8192
 #: dtype: below, an accumulation is bound by the host, and holding costs it another allocation
 #: (one accumulated micro-batch and two, held and as float32 rows, 8 bf16 ranks: of 8 M
 #: elements 34 and 32 us, 50 and 43; of 16 M 34 and 40, 55 and 65; of 64 M 87 and 133, 189 and
-#: 228; 2 ranks: 31 and 30, 45 and 38; 33 and 42, 59 and 67; 104 and 146, 204 and 242).
+#: 228; 2 ranks: 31 and 30, 45 and 38; 33 and 42, 59 and 67; 104 and 146, 204 and 242).  2 ranks
+#: cross near 10 M elements, 8 near 12 M.
 _HELD_MIN_ELEMENTS = 10 << 20
 
 #: Elements of a held micro-batch uploaded at a time when it was moved to host memory.
